@@ -249,9 +249,10 @@ int aq_ctx_create(int device, size_t hbm_budget, aq_ctx** out) {
             size_t free_b = 0, total_b = 0;
             AQ_HIP(hipMemGetInfo(&free_b, &total_b));
             ctx->budget = hbm_budget ? hbm_budget : static_cast<size_t>(0.9 * double(free_b));
-            ctx->d_partials = static_cast<double*>(dmalloc(ctx, sizeof(double) * (8 * 1024 + 64)));
+            ctx->d_partials = static_cast<double*>(dmalloc(ctx, sizeof(double) * kRedSlots * kRedPartials));
             AQ_CHECK(ctx->d_partials, AQ_ERR_OOM, "device allocation of reduction slots failed");
-            AQ_HIP(hipHostMalloc(&ctx->h_result, sizeof(double) * 64, hipHostMallocDefault));
+            AQ_HIP(hipHostMalloc(&ctx->h_result, sizeof(double) * kRedSlots, hipHostMallocDefault));
+            AQ_HIP(hipHostGetDevicePointer(reinterpret_cast<void**>(&ctx->d_result), ctx->h_result, 0));
         } catch (...) {
             if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
             delete ctx;

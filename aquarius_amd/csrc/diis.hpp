@@ -61,8 +61,20 @@ class DIIS {
     bool used_eps_retry = false;
 
     void extrapolate(const std::vector<Tensor*>& x, const std::vector<Tensor*>& dx) {
+        if (nextrap_ > 1) extrapolate(x, dx, [] {});
+    }
+
+    // `synced` is called once, after the first synchronisation of the stream
+    // (results of reductions queued before this call are then on the host).
+    template <class F>
+    void extrapolate(const std::vector<Tensor*>& x, const std::vector<Tensor*>& dx, F&& synced) {
         const int n = nextrap_, n1 = n + 1;
-        if (n <= 1) return;
+        if (n <= 1) {
+            AQ_HIP(hipStreamSynchronize(ctx_->stream));
+            resolve_timing(ctx_);
+            synced();
+            return;
+        }
         // slot k holds iteration n-k (diis.hpp:82-85)
         std::rotate(old_x_.begin(), old_x_.end() - 1, old_x_.end());
         std::rotate(old_dx_.begin(), old_dx_.end() - 1, old_dx_.end());
@@ -73,28 +85,44 @@ class DIIS {
             e_.swap(r);
             std::rotate(c_.begin(), c_.end() - 1, c_.end());
         }
-        store(old_x_[0], x);    // :92-105
-        store(old_dx_[0], dx);  // :107-120
+        // the newest slots (:92-120): the residuals are stored by the launch
+        // that forms their products, x by the extrapolation (or `keep`)
+        reserve(old_x_[0], x);
+        reserve(old_dx_[0], dx);
 
         // e[i][0] = <dx, old_dx[i]> for every stored slot (:122-135)
         int nreal = 1;
         while (nreal < n && !old_dx_[nreal].empty()) ++nreal;
         std::vector<double> p(nreal, 0.0);
-        // up to kDotSlots history slots per launch (the context's reduction
-        // slots); each inner product is reduced on its own, so the grouping
-        // does not change any value
-        constexpr int kDotSlots = 8;
-        for (int j = 0; j < ndx_; ++j) {
-            for (int first = 0; first < nreal; first += kDotSlots) {
-                const int kk = std::min(kDotSlots, nreal - first);
-                std::vector<const double*> ys;
-                for (int i = 0; i < kk; ++i) ys.push_back(dptr(old_dx_[first + i][j]));
-                launch_multi_dot(ctx_, dptr(*dx[j]), ys.data(), kk, tsize(*dx[j]), 0);
+        // up to kDiisDots history slots and kDiisSegs tensors per launch; each
+        // inner product is reduced on its own, so the grouping does not
+        // change any value
+        bool told = false;
+        for (int j0 = 0; j0 < ndx_; j0 += kDiisSegs) {
+            const int nj = std::min(kDiisSegs, ndx_ - j0);
+            for (int first = 0; first < nreal; first += kDiisDots) {
+                const int kk = std::min(kDiisDots, nreal - first);
+                DiisDot seg[kDiisSegs];
+                for (int j = 0; j < nj; ++j) {
+                    seg[j].x = dptr(*dx[j0 + j]);
+                    seg[j].copy = first == 0 ? dptr(old_dx_[0][j0 + j]) : nullptr;
+                    for (int i = 0; i < kk; ++i) seg[j].y[i] = dptr(old_dx_[first + i][j0 + j]);
+                    seg[j].n = tsize(*dx[j0 + j]);
+                }
+                launch_diis_dot(ctx_, nj, seg, kk, kFirstSlot);
                 AQ_HIP(hipStreamSynchronize(ctx_->stream));
-                for (int i = 0; i < kk; ++i) p[first + i] += ctx_->h_result[i];
+                if (!told) synced();
+                told = true;
+                for (int j = 0; j < nj; ++j)
+                    for (int i = 0; i < kk; ++i) p[first + i] += ctx_->h_result[kFirstSlot + j * kDiisDots + i];
             }
         }
+        if (!told) {
+            AQ_HIP(hipStreamSynchronize(ctx_->stream));
+            synced();
+        }
         resolve_timing(ctx_);
+        for (auto& t : old_dx_[0]) bump_t(t);
         E(0, 0) = p[0];
         for (int i = 1; i < nreal; ++i) {
             E(i, 0) = p[i];
@@ -108,18 +136,22 @@ class DIIS {
         E(nreal, nreal) = 0.0;
         c_[nreal] = -1.0;
 
-        if (nreal == 1) return;   // :151
+        if (nreal == 1) {         // :151
+            keep(x);
+            return;
+        }
 
         if (--start_ > 1) {       // :153-164
-            if (damping_ > 0.0)
+            keep(x);
+            if (damping_ > 0.0) {
+                const double cf[2] = {damping_ - 1.0, damping_};
                 for (int i = 0; i < nx_; ++i) {
                     double* a = dptr(old_x_[0][i]);
-                    const double* b = dptr(old_x_[1][i]);
-                    const double* xs[2] = {a, b};
-                    const double cf[2] = {damping_ - 1.0, damping_};
-                    launch_lincomb(ctx_, a, xs, cf, 2, tsize(old_x_[0][i]));
+                    const DiisComb seg{a, nullptr, {a, dptr(old_x_[1][i])}, tsize(old_x_[0][i])};
+                    launch_diis_combine(ctx_, 1, &seg, cf, 2);
                     bump_t(old_x_[0][i]);
                 }
+            }
             return;
         }
 
@@ -142,22 +174,23 @@ class DIIS {
             info = solve_small(m, A, b);
             used_eps_retry = true;
         }
+        if (info != 0) keep(x);
         AQ_CHECK(info == 0, AQ_ERR_NUMERIC, "DIIS: Info in hesv: " + std::to_string(info));
         for (int i = 0; i < m; ++i) c_[i] = b[i];
 
-        // x = sum_i c_i old_x[i], dx = sum_i c_i old_dx[i] (:205-226)
-        for (int j = 0; j < ndx_; ++j) {
-            std::vector<const double*> xs;
-            for (int i = 0; i < nreal; ++i) xs.push_back(dptr(old_dx_[i][j]));
-            launch_lincomb(ctx_, dptr(*dx[j]), xs.data(), c_.data(), nreal, tsize(*dx[j]));
-            bump_t(*dx[j]);
-        }
-        for (int j = 0; j < nx_; ++j) {
-            std::vector<const double*> xs;
-            for (int i = 0; i < nreal; ++i) xs.push_back(dptr(old_x_[i][j]));
-            launch_lincomb(ctx_, dptr(*x[j]), xs.data(), c_.data(), nreal, tsize(*x[j]));
-            bump_t(*x[j]);
-        }
+        // x = sum_i c_i old_x[i], dx = sum_i c_i old_dx[i] (:205-226), the
+        // newest term read from x (then stored into its slot) and dx itself
+        std::vector<DiisComb> seg;
+        const bool apart = distinct(x, dx);
+        if (!apart) keep(x);      // a tensor listed twice is overwritten only from stored copies, in order
+        for (int j = 0; j < ndx_; ++j) seg.push_back(terms(dx[j], apart, nullptr, old_dx_, j, nreal));
+        for (int j = 0; j < nx_; ++j) seg.push_back(terms(x[j], apart, dptr(old_x_[0][j]), old_x_, j, nreal));
+        const size_t per = apart ? kDiisSegs : 1;
+        for (size_t q = 0; q < seg.size(); q += per)
+            launch_diis_combine(ctx_, int(std::min(per, seg.size() - q)), &seg[q], c_.data(), nreal);
+        for (int j = 0; j < ndx_; ++j) bump_t(*dx[j]);
+        for (int j = 0; j < nx_; ++j) bump_t(*x[j]);
+        for (auto& t : old_x_[0]) bump_t(t);
     }
 
     const std::vector<double>& coefficients() const { return c_; }
@@ -165,16 +198,35 @@ class DIIS {
   private:
     double& E(int i, int j) { return e_[i * (nextrap_ + 1) + j]; }
 
-    void store(std::vector<Tensor>& slot, const std::vector<Tensor*>& src) {
-        if (slot.empty()) {
-            for (auto* t : src) slot.emplace_back(*t);   // deep copy
-        } else {
-            for (size_t i = 0; i < src.size(); ++i) {
-                AQ_HIP(hipMemcpyAsync(dptr(slot[i]), dptr(*src[i]), size_t(tsize(*src[i])) * 8,
-                                      hipMemcpyDeviceToDevice, ctx_->stream));
-                bump_t(slot[i]);
-            }
+    // first reduction slot of the inner products; a caller's results that are
+    // read by `synced` sit below it
+    static constexpr int kFirstSlot = kRedSlots - kDiisSegs * kDiisDots;
+
+    void reserve(std::vector<Tensor>& slot, const std::vector<Tensor*>& src) {
+        if (!slot.empty()) return;
+        for (auto* t : src) slot.emplace_back(ctx_, t->lengths(), false);
+    }
+    // x into its newest history slot
+    void keep(const std::vector<Tensor*>& x) {
+        for (size_t i = 0; i < x.size(); ++i) {
+            AQ_HIP(hipMemcpyAsync(dptr(old_x_[0][i]), dptr(*x[i]), size_t(tsize(*x[i])) * 8,
+                                  hipMemcpyDeviceToDevice, ctx_->stream));
+            bump_t(old_x_[0][i]);
         }
+    }
+    static bool distinct(const std::vector<Tensor*>& x, const std::vector<Tensor*>& dx) {
+        std::vector<const double*> p;
+        for (auto* t : x) p.push_back(dptr(*t));
+        for (auto* t : dx) p.push_back(dptr(*t));
+        std::sort(p.begin(), p.end());
+        return std::adjacent_find(p.begin(), p.end()) == p.end();
+    }
+    // the combination for tensor j; live: its newest term is `t` as it stands,
+    // and goes to `copy`
+    static DiisComb terms(Tensor* t, bool live, double* copy, std::vector<std::vector<Tensor>>& old, int j, int nreal) {
+        DiisComb s{dptr(*t), live ? copy : nullptr, {live ? dptr(*t) : dptr(old[0][j])}, tsize(*t)};
+        for (int i = 1; i < nreal; ++i) s.x.push_back(dptr(old[i][j]));
+        return s;
     }
 
     aq_ctx* ctx_;

@@ -319,7 +319,7 @@ void launch_weight(aq_ctx* ctx, double* x, int ndim, const int64_t* len, const d
 // Deterministic: a fixed number of blocks (a function of n only) each write
 // one partial; one block combines the partials in a fixed tree order.
 
-constexpr int RB = 1024;   // max partial blocks per slot
+constexpr int RB = kRedPartials;   // max partial blocks per slot
 
 enum RedOp { RED_SUM = 0, RED_MAX = 1 };
 
@@ -357,21 +357,37 @@ __global__ __launch_bounds__(TPB) void k_reduce_partial(const double* __restrict
     if (threadIdx.x == 0) partial[blockIdx.x] = r;
 }
 
-__global__ __launch_bounds__(TPB) void k_reduce_final(const double* partial, int np, int op, double* out) {
+// One block per reduction: combine slot's partials and write the result into
+// pinned host memory (visible to the host at the next synchronisation), so a
+// set of reductions costs one launch and no copies.  Latency-bound: at o=5,
+// v=19 the former launch-plus-copy per slot (2.4 + 2.3 us each, 10 slots per
+// iteration at DIIS order 8) was 9 ms of a 70 ms profile.
+struct FinalArgs {
+    int slot[kRedSlots], np[kRedSlots], op[kRedSlots];
+};
+
+__global__ __launch_bounds__(TPB) void k_reduce_final(const double* __restrict__ partials, FinalArgs f, double* out) {
+    const int k = blockIdx.x;
+    const double* p = partials + int64_t(f.slot[k]) * RB;
     double acc = 0.0;
-    for (int i = threadIdx.x; i < np; i += TPB) acc = red(acc, partial[i], op);
-    const double r = block_reduce(acc, op);
-    if (threadIdx.x == 0) *out = r;
+    for (int i = threadIdx.x; i < f.np[k]; i += TPB) acc = red(acc, p[i], f.op[k]);
+    const double r = block_reduce(acc, f.op[k]);
+    if (threadIdx.x == 0) out[f.slot[k]] = r;
 }
 
 static double* partial_slot(aq_ctx* ctx, int slot) { return ctx->d_partials + int64_t(slot) * RB; }
-static double* result_slot(aq_ctx* ctx, int slot) { return ctx->d_partials + int64_t(8) * RB + slot; }
 
-static void finish(aq_ctx* ctx, int slot, unsigned np, int op) {
-    hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(TPB), 0, ctx->stream, partial_slot(ctx, slot), int(np), op,
-                       result_slot(ctx, slot));
+static void finish(aq_ctx* ctx, const FinalArgs& f, int n) {
+    hipLaunchKernelGGL(k_reduce_final, dim3(unsigned(n)), dim3(TPB), 0, ctx->stream, ctx->d_partials, f,
+                       ctx->d_result);
     AQ_HIP(hipGetLastError());
-    AQ_HIP(hipMemcpyAsync(ctx->h_result + slot, result_slot(ctx, slot), 8, hipMemcpyDeviceToHost, ctx->stream));
+}
+static void finish(aq_ctx* ctx, int slot, unsigned np, int op) {
+    FinalArgs f{};
+    f.slot[0] = slot;
+    f.np[0] = int(np);
+    f.op[0] = op;
+    finish(ctx, f, 1);
 }
 
 void launch_dot(aq_ctx* ctx, const double* a, const double* b, int64_t n, int slot) {
@@ -582,8 +598,6 @@ void launch_ccsd_update(aq_ctx* ctx, const UpdateArgs& u, int slot_e1, int slot_
                            partial_slot(ctx, slot_c1));
         AQ_HIP(hipGetLastError());
     }
-    finish(ctx, slot_e1, g1, RED_SUM);
-    finish(ctx, slot_c1, g1, RED_MAX);
     {
         // algorithmic bytes: read Z2, T2, VABIJSA; write Z2, T2, Tau
         TimedLaunch tl(ctx, "ccsd_update_t2", 0.0, 8.0 * 6 * n2);
@@ -591,8 +605,9 @@ void launch_ccsd_update(aq_ctx* ctx, const UpdateArgs& u, int slot_e1, int slot_
                            partial_slot(ctx, slot_c2));
         AQ_HIP(hipGetLastError());
     }
-    finish(ctx, slot_e2, g2, RED_SUM);
-    finish(ctx, slot_c2, g2, RED_MAX);
+    const FinalArgs f{{slot_e1, slot_c1, slot_e2, slot_c2}, {int(g1), int(g1), int(g2), int(g2)},
+                      {RED_SUM, RED_MAX, RED_SUM, RED_MAX}};
+    finish(ctx, f, 4);
 }
 
 // ------------------------------------------------------- packed ladder
@@ -870,7 +885,7 @@ void launch_ladder_unpack(aq_ctx* ctx, const double* Sp, const double* Sm, int v
 }
 
 double pair_asymmetry(aq_ctx* ctx, const double* X, int n1, int n2, int slot) {
-    AQ_CHECK(slot >= 0 && slot < 8, AQ_ERR_INVALID, "reduction slot out of range");
+    AQ_CHECK(slot >= 0 && slot < kRedSlots, AQ_ERR_INVALID, "reduction slot out of range");
     const int64_t n = int64_t(n1) * n1 * n2 * n2;
     if (n == 0) return 0.0;
     const unsigned g = red_blocks(n);
@@ -942,73 +957,134 @@ void launch_eri_expand(aq_ctx* ctx, const double* compact, const int* shell_of, 
 
 constexpr int MAXK = 16;
 
-struct PtrList {
-    const double* p[MAXK];
+// Inner products of residuals with their history.  A launch covers up to
+// kDiisSegs tensors (blocks [first[s], first[s+1]) belong to tensor s): each
+// block reads its part of x once, forms the nk products and, in the launch
+// that holds the newest slot (copy != null), also stores x into that slot and
+// takes x * x for it.  HBM-bound: 8 (nk + 1) bytes per element.
+struct DotSeg {
+    const double* x;
+    double* copy;
+    const double* y[kDiisDots];
+    int64_t n;
+};
+struct DotArgs {
+    DotSeg s[kDiisSegs];
+    int first[kDiisSegs + 1];
+    int nseg, nk;
 };
 
-// partial[slot_k][block] = sum x*y_k for k < nk (x read once)
-__global__ __launch_bounds__(TPB) void k_multi_dot(const double* __restrict__ x, PtrList ys, int nk, int64_t n,
-                                                    double* partials) {
-    double acc[MAXK];
+__global__ __launch_bounds__(TPB) void k_diis_dot(DotArgs g, double* partials) {
+    int q = 0;
+    while (q + 1 < g.nseg && int(blockIdx.x) >= g.first[q + 1]) ++q;
+    const DotSeg& s = g.s[q];
+    const int blk = int(blockIdx.x) - g.first[q];
+    const int64_t stride = int64_t(g.first[q + 1] - g.first[q]) * TPB;
+    double acc[kDiisDots];
 #pragma unroll
-    for (int k = 0; k < MAXK; ++k) acc[k] = 0.0;
-    for (int64_t i = int64_t(blockIdx.x) * TPB + threadIdx.x; i < n; i += int64_t(gridDim.x) * TPB) {
-        const double xv = x[i];
+    for (int k = 0; k < kDiisDots; ++k) acc[k] = 0.0;
+    for (int64_t i = int64_t(blk) * TPB + threadIdx.x; i < s.n; i += stride) {
+        const double xv = s.x[i];
+        if (s.copy) s.copy[i] = xv;
 #pragma unroll
-        for (int k = 0; k < MAXK; ++k)
-            if (k < nk) acc[k] += xv * ys.p[k][i];
+        for (int k = 0; k < kDiisDots; ++k)
+            if (k < g.nk) acc[k] += xv * (k == 0 && s.copy ? xv : s.y[k][i]);
     }
-    for (int k = 0; k < nk; ++k) {
+    double* part = partials + int64_t(q) * kDiisDots * RB;
+    for (int k = 0; k < g.nk; ++k) {
         const double r = block_reduce(acc[k], RED_SUM);
-        if (threadIdx.x == 0) partials[int64_t(k) * RB + blockIdx.x] = r;
+        if (threadIdx.x == 0) part[int64_t(k) * RB + blk] = r;
     }
 }
 
-void launch_multi_dot(aq_ctx* ctx, const double* x, const double* const* ys, int k, int64_t n, int first_slot) {
-    AQ_CHECK(k >= 1 && k <= MAXK && first_slot + k <= 8, AQ_ERR_INVALID, "multi-dot arity");
-    PtrList pl{};
-    for (int i = 0; i < k; ++i) pl.p[i] = ys[i];
-    const unsigned g = red_blocks(n);
+void launch_diis_dot(aq_ctx* ctx, int nseg, const DiisDot* seg, int nk, int first_slot) {
+    AQ_CHECK(nseg >= 1 && nseg <= kDiisSegs && nk >= 1 && nk <= kDiisDots &&
+                 first_slot + nseg * kDiisDots <= kRedSlots,
+             AQ_ERR_INVALID, "DIIS dot arity");
+    DotArgs g{};
+    g.nseg = nseg;
+    g.nk = nk;
+    FinalArgs f{};
+    double n = 0.0;
+    for (int q = 0; q < nseg; ++q) {
+        g.s[q].x = seg[q].x;
+        g.s[q].copy = seg[q].copy;
+        for (int k = 0; k < nk; ++k) g.s[q].y[k] = seg[q].y[k];
+        g.s[q].n = seg[q].n;
+        n += double(seg[q].n);
+        const int blocks = int(red_blocks(seg[q].n));
+        g.first[q + 1] = g.first[q] + blocks;
+        for (int k = 0; k < nk; ++k) {
+            f.slot[q * nk + k] = first_slot + q * kDiisDots + k;
+            f.np[q * nk + k] = blocks;
+            f.op[q * nk + k] = RED_SUM;
+        }
+    }
     {
-        TimedLaunch tl(ctx, "diis_dot", 2.0 * n * k, 8.0 * n * (k + 1));
-        hipLaunchKernelGGL(k_multi_dot, dim3(g), dim3(TPB), 0, ctx->stream, x, pl, k, n, partial_slot(ctx, first_slot));
+        TimedLaunch tl(ctx, "diis_dot", 2.0 * n * nk, 8.0 * n * (nk + 1));
+        hipLaunchKernelGGL(k_diis_dot, dim3(unsigned(g.first[nseg])), dim3(TPB), 0, ctx->stream, g,
+                           partial_slot(ctx, first_slot));
         AQ_HIP(hipGetLastError());
     }
-    for (int i = 0; i < k; ++i) finish(ctx, first_slot + i, g, RED_SUM);
+    finish(ctx, f, nseg * nk);
 }
 
-// out = sum_k c_k * xs_k, accumulated in the reference's order
-// (out = x0*c0; out += x_k*c_k, diis.hpp:205-226).  More than MAXK terms run
-// as several launches; each later launch continues from `out` (cont = 1), so
-// every element is summed left to right exactly as in one pass.
-struct CoefList {
+// out = sum_k c_k * x_k for several tensors in one launch, accumulated in the
+// reference's order (out = x0*c0; out += x_k*c_k, diis.hpp:205-226).  The
+// newest term x_0 may be `out` itself; where copy != null its value is stored
+// there (the history slot) before it is overwritten, so the slot costs no pass
+// of its own.  More than MAXK terms run as several launches; each later launch
+// continues from `out` (cont = 1), so every element is summed left to right
+// exactly as in one pass.  HBM-bound: 8 (nk + 1 or 2) bytes per element.
+struct CombSeg {
+    double* out;
+    double* copy;
+    const double* x[MAXK];
+    int64_t n;
+};
+struct CombArgs {
+    CombSeg s[kDiisSegs];
+    int64_t first[kDiisSegs + 1];
     double c[MAXK];
+    int nseg, nk, cont;
 };
 
-__global__ __launch_bounds__(TPB) void k_lincomb(double* out, PtrList xs, CoefList c, int nk, int64_t n, int cont) {
-    for (int64_t i = int64_t(blockIdx.x) * TPB + threadIdx.x; i < n; i += int64_t(gridDim.x) * TPB) {
-        double s = cont ? out[i] + xs.p[0][i] * c.c[0] : xs.p[0][i] * c.c[0];
-        for (int k = 1; k < nk; ++k) s = s + xs.p[k][i] * c.c[k];
-        out[i] = s;
+__global__ __launch_bounds__(TPB) void k_diis_combine(CombArgs g) {
+    int q = 0;
+    while (q + 1 < g.nseg && int64_t(blockIdx.x) >= g.first[q + 1]) ++q;
+    const CombSeg& s = g.s[q];
+    const int64_t stride = (g.first[q + 1] - g.first[q]) * TPB;
+    for (int64_t i = (int64_t(blockIdx.x) - g.first[q]) * TPB + threadIdx.x; i < s.n; i += stride) {
+        const double x0 = s.x[0][i];
+        if (s.copy) s.copy[i] = x0;
+        double v = g.cont ? s.out[i] + x0 * g.c[0] : x0 * g.c[0];
+        for (int k = 1; k < g.nk; ++k) v = v + s.x[k][i] * g.c[k];
+        s.out[i] = v;
     }
 }
 
-void launch_lincomb(aq_ctx* ctx, double* out, const double* const* xs, const double* c, int k, int64_t n) {
-    AQ_CHECK(k >= 1, AQ_ERR_INVALID, "lincomb arity");
+void launch_diis_combine(aq_ctx* ctx, int nseg, const DiisComb* seg, const double* c, int k) {
+    AQ_CHECK(k >= 1 && nseg >= 1 && nseg <= kDiisSegs, AQ_ERR_INVALID, "DIIS combination arity");
     for (int first = 0; first < k; first += MAXK) {
         const int kk = std::min(MAXK, k - first);
-        PtrList pl{};
-        CoefList cl{};
-        for (int i = 0; i < kk; ++i) {
-            pl.p[i] = xs[first + i];
-            cl.c[i] = c[first + i];
+        CombArgs g{};
+        g.nseg = nseg;
+        g.nk = kk;
+        g.cont = int(first > 0);
+        double n = 0.0;
+        for (int i = 0; i < kk; ++i) g.c[i] = c[first + i];
+        for (int q = 0; q < nseg; ++q) {
+            g.s[q].out = seg[q].out;
+            g.s[q].copy = first == 0 ? seg[q].copy : nullptr;
+            for (int i = 0; i < kk; ++i) g.s[q].x[i] = seg[q].x[size_t(first + i)];
+            g.s[q].n = seg[q].n;
+            n += double(seg[q].n);
+            g.first[q + 1] = g.first[q] + int64_t(grid_for(seg[q].n, TPB * 4));
         }
         TimedLaunch tl(ctx, "diis_lincomb", 2.0 * n * kk, 8.0 * n * (kk + 1 + (first > 0)));
-        hipLaunchKernelGGL(k_lincomb, dim3(grid_for(n, TPB * 4)), dim3(TPB), 0, ctx->stream, out, pl, cl, kk, n,
-                           int(first > 0));
+        hipLaunchKernelGGL(k_diis_combine, dim3(unsigned(g.first[nseg])), dim3(TPB), 0, ctx->stream, g);
         AQ_HIP(hipGetLastError());
     }
-    AQ_HIP(hipGetLastError());
 }
 
 }  // namespace aqamd

@@ -76,6 +76,9 @@ struct PendingTiming {
 
 // ------------------------------------------------------------ context
 
+constexpr int kRedSlots = 40;       // concurrent reductions of a context
+constexpr int kRedPartials = 1024;  // partials per reduction
+
 struct CacheEntry {
     void* ptr = nullptr;
     size_t bytes = 0;
@@ -138,8 +141,9 @@ struct aq_ctx {
     size_t cache_bytes = 0;
 
     // reductions
-    double* d_partials = nullptr;   // device: 8 slots x 1024 partials, then 64 result slots
-    double* h_result = nullptr;     // pinned host result slots (64)
+    double* d_partials = nullptr;   // device: kRedSlots slots x kRedPartials partials
+    double* h_result = nullptr;     // pinned host result slots (kRedSlots)
+    double* d_result = nullptr;     // the same slots as the device addresses them
 
     // HIP-graph capture: mem_gen counts frees of device memory (a captured
     // graph holds raw pointers and is valid only while nothing it uses was
@@ -286,11 +290,24 @@ void launch_eri_expand(aq_ctx* ctx, const double* compact, const int* shell_of, 
                        const int64_t* pair_size, const int64_t* prefix, const int64_t* rowstart, int64_t n,
                        int64_t total, double* out);
 
-// DIIS helpers (elementwise.hip)
-void launch_multi_dot(aq_ctx* ctx, const double* x, const double* const* ys, int k, int64_t n,
-                      int first_slot);
-void launch_lincomb(aq_ctx* ctx, double* out, const double* const* xs, const double* c, int k,
-                    int64_t n);
+// DIIS helpers (elementwise.hip), each over up to kDiisSegs tensors per launch
+constexpr int kDiisSegs = 4;   // tensors per launch
+constexpr int kDiisDots = 8;   // history slots per dot launch
+struct DiisDot {
+    const double* x;                  // the residual
+    double* copy;                     // its newest history slot, filled by the launch, or null
+    const double* y[kDiisDots];       // stored residuals (y[0] is not read when copy is set)
+    int64_t n;
+};
+// results of tensor q, slot k in h_result[first_slot + q*kDiisDots + k]; caller syncs
+void launch_diis_dot(aq_ctx* ctx, int nseg, const DiisDot* seg, int nk, int first_slot);
+struct DiisComb {
+    double* out;
+    double* copy;                     // receives x[0] (may be null)
+    std::vector<const double*> x;     // x[0] may be out
+    int64_t n;
+};
+void launch_diis_combine(aq_ctx* ctx, int nseg, const DiisComb* seg, const double* c, int k);
 
 // ---- GEMM (gemm.hip)
 struct GemmDesc {

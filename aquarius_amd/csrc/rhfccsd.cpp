@@ -402,11 +402,12 @@ struct aq_rhfccsd {
             UpdateArgs u{o, v, dptr(Z1), dptr(Z2), dptr(T1), dptr(T2), dptr(Tau), dptr(VABIJSA), dptr(fAI),
                          dptr(d_dA), dptr(d_dI)};
             launch_ccsd_update(ctx, u, 0, 1, 2, 3);                // :313-323
-            AQ_HIP(hipStreamSynchronize(ctx->stream));
-            resolve_timing(ctx);
             for (const Tensor* t : {&Z1, &Z2, &T1, &T2, &Tau}) bump_t(*t);
-            energy = 2 * ctx->h_result[0] + ctx->h_result[1];
-            conv = std::max(ctx->h_result[2], ctx->h_result[3]);
+            // one synchronisation serves the update's results and the DIIS products
+            diis->extrapolate({&T1, &T2}, {&Z1, &Z2}, [&] {        // :325-326
+                energy = 2 * ctx->h_result[0] + ctx->h_result[1];
+                conv = std::max(ctx->h_result[2], ctx->h_result[3]);
+            });
         } else {
             Z1.weight({&dA, &dI});                                 // :313
             Z2.weight({&dA, &dA, &dI, &dI});                       // :314
@@ -416,8 +417,8 @@ struct aq_rhfccsd {
             Tau["abij"] += T1["ai"] * T1["bj"];                    // :320
             energy = 2 * scalar(fAI["ai"] * T1["ai"]) + scalar(VABIJSA["abij"] * Tau["abij"]);   // :322
             conv = std::max(Z1.norm(0), Z2.norm(0));               // :323
+            diis->extrapolate({&T1, &T2}, {&Z1, &Z2});             // :325-326
         }
-        diis->extrapolate({&T1, &T2}, {&Z1, &Z2});                 // :325-326
         ++iter;
     }
 
