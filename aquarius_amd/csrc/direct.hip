@@ -1,0 +1,481 @@
+// FP64 contractions read straight from the operands' labelled layouts.
+//
+//   C(m,n,b) = alpha * sum_k A(m,k,b) B(k,n,b) + beta * C(m,n,b)
+//
+// m, n and k are groups of labels with arbitrary strides in A, B and C, so no
+// operand is permuted into a matrix first and no result is permuted
+// afterwards.  FP64 MFMA on gfx950 is slow against its operands: a 16x16x4
+// instruction takes 64 cycles for two 512-byte fragments, so fragments are
+// loaded from global memory (L1/L2) into registers directly, without LDS
+// staging and without a barrier in the k loop; every wave runs on its own.
+//
+// A block of 256 threads = WM x WN x WK waves owns a (16 FM WM) x (16 FN WN)
+// output tile; each wave has FM x FN 16x16 MFMA blocks, and WK waves share the
+// k range (added in LDS, in wave order, at the end).  Work goes in chunks of
+// 16 k: lane group q = lane/16 takes k = 4q..4q+3, so an operand whose k is
+// contiguous is read with two 16-byte loads per row and chunk, and one whose
+// rows are contiguous with 128-byte runs; the k offsets of both operands come
+// from an LDS table built once per block, the row offsets from registers.
+// Several chunks are in flight per wave.
+//
+// When the output has too few tiles, the k range is also split over blocks and
+// a second launch adds the partial tiles in split order.  (Having the last
+// block of a tile add them in the same launch was measured 5 to 15 times
+// slower: each block's device-scope fence writes back its XCD's whole L2; 485
+// blocks, M = N = 344: 9 us without a split, 117 us with two.)
+#include "direct.hpp"
+
+#include <algorithm>
+#include <cstdio>
+#include <cmath>
+
+namespace aqamd {
+
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+typedef double f64x2u __attribute__((ext_vector_type(2), aligned(8)));   // 16-byte load, 8-byte aligned
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kKT = 1024;   // k offsets held at a time
+
+// offset of index x (below 2^31) through a digit group; the divisions by the
+// digit lengths are multiplications (set_divider)
+__device__ __forceinline__ uint32_t digit_offset(const DirDigits& d, const uint32_t* st, uint32_t x) {
+    uint32_t off = 0;
+#pragma unroll
+    for (int k = 0; k + 1 < kDirDigits; ++k) {
+        if (k + 1 >= d.nd) break;
+        const uint32_t q = __umulhi(x, d.mul[k]) >> d.shift[k];
+        off += (x - q * d.len[k]) * st[k];
+        x = q;
+    }
+    return d.nd > 0 ? off + x * st[d.nd - 1] : 0u;
+}
+
+template <int FM, int FN, int WM, int WN, int WK, int ST, bool VA, bool VB>
+__device__ __forceinline__ void direct_tile(const DirectArgs& g, uint32_t bid) {
+    static_assert(WM * WN * WK == 4, "4 waves");
+    constexpr int TM = 16 * FM * WM, TN = 16 * FN * WN;
+    constexpr int RED = WK > 1 ? WK * TM * TN * 8 : 16;
+    constexpr int TAB = 2 * kKT * 4;
+    __shared__ __attribute__((aligned(16))) char lds[RED > TAB ? RED : TAB];
+    uint32_t* ta = reinterpret_cast<uint32_t*>(lds);
+    uint32_t* tb = ta + kKT;
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wk = wave % WK, wm = (wave / WK) % WM, wn = wave / (WK * WM);
+    const int l16 = lane & 15, q = lane >> 4;
+
+    // block -> (batch, tile, split), split fastest; tiles m fastest
+    const uint32_t split = bid % g.nsplit;
+    const uint32_t bt = bid / g.nsplit;
+    const uint32_t tiles = g.tilesM * g.tilesN;
+    const uint32_t b = bt / tiles, tile = bt % tiles;
+    const uint32_t m0 = (tile % g.tilesM) * TM, n0 = (tile / g.tilesM) * TN;
+    const uint32_t kbeg = split * g.kchunk, kend = min(g.K, kbeg + g.kchunk);
+
+    const char* Ab = reinterpret_cast<const char*>(g.A + uint64_t(b) * g.bsA);
+    const char* Bb = reinterpret_cast<const char*>(g.B + uint64_t(b) * g.bsB);
+
+    // byte offsets of this lane's operand rows; rows past the edge read the
+    // last one (they only feed outputs that are not stored)
+    uint32_t ra[FM], rb[FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+        ra[i] = digit_offset(g.m, g.m.s0, min(m0 + (wm * FM + i) * 16 + l16, g.M - 1)) * 8u;
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+        rb[j] = digit_offset(g.n, g.n.s0, min(n0 + (wn * FN + j) * 16 + l16, g.N - 1)) * 8u;
+
+    f64x4 acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[i][j] = f64x4{0, 0, 0, 0};
+
+    // The k loop issues its loads without conditions, ST - 1 chunks ahead (past
+    // the end it reads the last full chunk again): behind a branch the compiler
+    // would have to wait for every outstanding load at the join.  The partial
+    // last chunk is loaded first, by the wave whose turn it is, and used last.
+    double va[ST][4][FM], vb[ST][4][FN], ua[4][FM], ub[4][FN];
+    for (uint32_t kb = kbeg; kb < kend; kb += kKT) {
+        const uint32_t klen = min(uint32_t(kKT), kend - kb);
+        const uint32_t nfull = klen / 16;
+        if (kb != kbeg) __syncthreads();   // every wave is done with the previous table
+        for (uint32_t k = tid; k < (klen + 15) / 16 * 16; k += 256) {
+            const uint32_t kk = kb + min(k, klen - 1);   // past the end: the last k, zeroed after the load
+            ta[k] = digit_offset(g.k, g.k.s0, kk) * 8u;
+            tb[k] = digit_offset(g.k, g.k.s1, kk) * 8u;
+        }
+        __syncthreads();
+
+        auto offsets = [&](const uint32_t* t, uint32_t c) { return *reinterpret_cast<const u32x4*>(t + c * 16 + 4 * q); };
+        auto each = [&](double* x, const char* base, uint32_t row, const u32x4 o, int step) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s) x[s * step] = *reinterpret_cast<const double*>(base + (row + o[s]));
+        };
+        auto run = [&](double* x, const char* base, uint32_t row, const u32x4 o, int step) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const f64x2u y = *reinterpret_cast<const f64x2u*>(base + (row + o[0] + 16u * h));
+                x[2 * h * step] = y[0];
+                x[(2 * h + 1) * step] = y[1];
+            }
+        };
+        auto load = [&](double (&xa)[4][FM], double (&xb)[4][FN], uint32_t c) {
+            const u32x4 oa = offsets(ta, c), ob = offsets(tb, c);
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+                if constexpr (VA) run(&xa[0][i], Ab, ra[i], oa, FM);
+                else each(&xa[0][i], Ab, ra[i], oa, FM);
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+                if constexpr (VB) run(&xb[0][j], Bb, rb[j], ob, FN);
+                else each(&xb[0][j], Bb, rb[j], ob, FN);
+        };
+        auto mma = [&](const double (&xa)[4][FM], const double (&xb)[4][FN]) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int i = 0; i < FM; ++i)
+#pragma unroll
+                    for (int j = 0; j < FN; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(xb[s][j], xa[s][i], acc[i][j], 0, 0, 0);
+        };
+
+        const bool tail = klen % 16 != 0 && nfull % WK == uint32_t(wk);
+        if (tail) {
+            const u32x4 oa = offsets(ta, nfull), ob = offsets(tb, nfull);
+#pragma unroll
+            for (int i = 0; i < FM; ++i) each(&ua[0][i], Ab, ra[i], oa, FM);
+#pragma unroll
+            for (int j = 0; j < FN; ++j) each(&ub[0][j], Bb, rb[j], ob, FN);
+        }
+        if (nfull > uint32_t(wk)) {
+            const uint32_t nw = (nfull - wk + WK - 1) / WK;   // this wave's full chunks
+            auto chunk = [&](uint32_t i) { return min(wk + i * WK, nfull - 1); };
+#pragma unroll
+            for (int s = 0; s < ST - 1; ++s) load(va[s], vb[s], chunk(s));
+            uint32_t i = 0;
+            for (; i + ST <= nw; i += ST) {
+#pragma unroll
+                for (int s = 0; s < ST; ++s) {
+                    load(va[(s + ST - 1) % ST], vb[(s + ST - 1) % ST], chunk(i + s + ST - 1));
+                    __builtin_amdgcn_sched_barrier(0);
+                    mma(va[s], vb[s]);
+                }
+            }
+#pragma unroll
+            for (int s = 0; s < ST - 1; ++s)
+                if (i + s < nw) mma(va[s], vb[s]);
+        }
+        if (tail) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const bool in = nfull * 16 + 4 * q + s < klen;
+#pragma unroll
+                for (int i = 0; i < FM; ++i) ua[s][i] = in ? ua[s][i] : 0.0;
+#pragma unroll
+                for (int j = 0; j < FN; ++j) ub[s][j] = in ? ub[s][j] : 0.0;
+            }
+            mma(ua, ub);
+        }
+    }
+
+    // lane holds tile element (m = l16 of block i, n = q + 4r of block j)
+    double* Cb = g.C + uint64_t(b) * g.bsC;
+    if (WK == 1 && g.nsplit == 1) {
+        uint32_t cn[FN][4];
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                cn[j][r] = digit_offset(g.n, g.n.s1, min(n0 + (wn * FN + j) * 16 + q + 4 * r, g.N - 1));
+#pragma unroll
+        for (int i = 0; i < FM; ++i) {
+            const uint32_t m = m0 + (wm * FM + i) * 16 + l16;
+            const uint32_t cm = digit_offset(g.m, g.m.s1, min(m, g.M - 1));
+            // every C value of the row is read before any is written (one round trip)
+            double cv[FN][4];
+            if (g.beta != 0.0) {
+#pragma unroll
+                for (int j = 0; j < FN; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) cv[j][r] = Cb[cm + cn[j][r]];
+            }
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const uint32_t n = n0 + (wn * FN + j) * 16 + q + 4 * r;
+                    if (m < g.M && n < g.N) {
+                        double v = g.alpha * acc[i][j][r];
+                        if (g.beta != 0.0) v += g.beta * cv[j][r];
+                        Cb[cm + cn[j][r]] = v;
+                    }
+                }
+        }
+        return;
+    }
+
+    constexpr int TE = TM * TN, NE = TE / 256;   // tile elements, and per thread
+    static_assert(TE % 256 == 0, "whole tile per thread count");
+    double v[NE];
+    if (WK > 1) {
+        double* red = reinterpret_cast<double*>(lds);
+        __syncthreads();   // the k tables are no longer read
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    red[wk * TE + ((wn * FN + j) * 16 + q + 4 * r) * TM + (wm * FM + i) * 16 + l16] = acc[i][j][r];
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < NE; ++r) {
+            double s = red[tid + 256 * r];
+#pragma unroll
+            for (int w = 1; w < WK; ++w) s += red[w * TE + tid + 256 * r];
+            v[r] = s;
+        }
+    }
+    if (g.nsplit > 1) {
+        double* P = g.P + uint64_t(bt) * g.nsplit * TE;
+        double* mine = P + uint64_t(split) * TE;
+        if (WK > 1) {
+#pragma unroll
+            for (int r = 0; r < NE; ++r) mine[tid + 256 * r] = v[r];
+        } else {
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int j = 0; j < FN; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        mine[((wn * FN + j) * 16 + q + 4 * r) * TM + (wm * FM + i) * 16 + l16] = acc[i][j][r];
+        }
+        return;
+    }
+#pragma unroll
+    for (int r = 0; r < NE; ++r) {
+        const uint32_t e = tid + 256 * r;
+        const uint32_t m = m0 + e % TM, n = n0 + e / TM;
+        if (m < g.M && n < g.N) {
+            double* c = Cb + digit_offset(g.m, g.m.s1, m) + digit_offset(g.n, g.n.s1, n);
+            const double x = g.alpha * v[r];
+            *c = g.beta != 0.0 ? g.beta * *c + x : x;
+        }
+    }
+}
+
+// C from the partial tiles of a split launch: one thread per tile element, the
+// splits added in order, eight loads in flight.
+__global__ __launch_bounds__(256) void k_direct_reduce(DirectArgs g, uint32_t tm, uint32_t te) {
+    const uint32_t per = te / 256;                      // blocks of 256 elements per tile
+    const uint32_t bt = blockIdx.x / per, e = (blockIdx.x % per) * 256 + threadIdx.x;
+    const uint32_t tiles = g.tilesM * g.tilesN;
+    const uint32_t b = bt / tiles, tile = bt % tiles;
+    const uint32_t m = (tile % g.tilesM) * tm + e % tm, n = (tile / g.tilesM) * (te / tm) + e / tm;
+    if (m >= g.M || n >= g.N) return;
+    const double* P = g.P + uint64_t(bt) * g.nsplit * te + e;
+    double v = 0.0;
+    uint32_t s = 0;
+    for (; s + 8 <= g.nsplit; s += 8) {
+        double x[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) x[u] = P[uint64_t(s + u) * te];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v += x[u];
+    }
+    for (; s < g.nsplit; ++s) v += P[uint64_t(s) * te];
+    double* c = g.C + uint64_t(b) * g.bsC + digit_offset(g.m, g.m.s1, m) + digit_offset(g.n, g.n.s1, n);
+    const double x = g.alpha * v;
+    *c = g.beta != 0.0 ? g.beta * *c + x : x;
+}
+
+// block id -> work id: the dispatcher deals ids to the 8 XCDs round-robin; give
+// each XCD a contiguous run, whose tiles share operand rows in its L2
+__device__ __forceinline__ uint32_t xcd_order(uint32_t bid, uint32_t nb) {
+    const uint32_t full = nb / 8 * 8;
+    return bid >= full ? bid : (bid % 8) * (nb / 8) + bid / 8;
+}
+
+template <int FM, int FN, int WM, int WN, int WK, int ST, bool VA, bool VB>
+__global__ __launch_bounds__(256) void k_direct(DirectArgs g) {
+    direct_tile<FM, FN, WM, WN, WK, ST, VA, VB>(g, xcd_order(blockIdx.x, gridDim.x));
+}
+
+// The tiles of up to kDirGroup problems of different contexts in one launch;
+// each tile is computed exactly as in a launch of its problem alone.
+struct DirectGroup {
+    DirectArgs p[kDirGroup];
+    uint32_t first[kDirGroup + 1];
+    int n;
+};
+
+template <int FM, int FN, int WM, int WN, int WK, int ST, bool VA, bool VB>
+__global__ __launch_bounds__(256) void k_direct_grouped(DirectGroup G) {
+    int p = 0;
+    while (p + 1 < G.n && blockIdx.x >= G.first[p + 1]) ++p;
+    direct_tile<FM, FN, WM, WN, WK, ST, VA, VB>(G.p[p], blockIdx.x - G.first[p]);
+}
+
+struct DirCfg {
+    int fm, fn, wm, wn, wk, stages;
+    int tm() const { return 16 * fm * wm; }
+    int tn() const { return 16 * fn * wn; }
+};
+constexpr DirCfg kDirCfg[] = {
+    {1, 1, 1, 1, 4, 4},   // 16 x 16: tiny outputs
+    {2, 2, 1, 1, 4, 3},   // 32 x 32, waves share k
+    {1, 1, 2, 2, 1, 4},   // 32 x 32, short k
+    {2, 2, 2, 2, 1, 3},   // 64 x 64
+    {4, 1, 1, 1, 4, 3},   // 64 x 16
+    {1, 4, 1, 1, 4, 3},   // 16 x 64
+    {4, 1, 4, 1, 1, 2},   // 256 x 16, short k
+    {1, 4, 1, 4, 1, 2},   // 16 x 256, short k
+};
+constexpr int kNDirCfg = int(sizeof(kDirCfg) / sizeof(kDirCfg[0]));
+
+template <int FM, int FN, int WM, int WN, int WK, int ST, class F>
+static void with_layout(int va, int vb, F&& f) {
+    if (va && vb) f(std::integral_constant<int, 3>{});
+    else if (va) f(std::integral_constant<int, 1>{});
+    else if (vb) f(std::integral_constant<int, 2>{});
+    else f(std::integral_constant<int, 0>{});
+}
+
+template <int FM, int FN, int WM, int WN, int WK, int ST>
+static void run_direct(int lay, dim3 grid, hipStream_t s, const DirectArgs* one, const DirectGroup* many) {
+    with_layout<FM, FN, WM, WN, WK, ST>(lay & 1, lay & 2, [&](auto L) {
+        constexpr int l = decltype(L)::value;
+        if (one)
+            hipLaunchKernelGGL((k_direct<FM, FN, WM, WN, WK, ST, (l & 1) != 0, (l & 2) != 0>), grid, dim3(256), 0, s, *one);
+        else
+            hipLaunchKernelGGL((k_direct_grouped<FM, FN, WM, WN, WK, ST, (l & 1) != 0, (l & 2) != 0>), grid, dim3(256), 0,
+                               s, *many);
+    });
+    AQ_HIP(hipGetLastError());
+}
+
+// config = shape index * 4 + layout bits
+static void dispatch_direct(int config, dim3 grid, hipStream_t s, const DirectArgs* one, const DirectGroup* many) {
+    const int lay = config & 3;
+    switch (config >> 2) {
+        case 0: run_direct<1, 1, 1, 1, 4, 4>(lay, grid, s, one, many); break;
+        case 1: run_direct<2, 2, 1, 1, 4, 3>(lay, grid, s, one, many); break;
+        case 2: run_direct<1, 1, 2, 2, 1, 4>(lay, grid, s, one, many); break;
+        case 3: run_direct<2, 2, 2, 2, 1, 3>(lay, grid, s, one, many); break;
+        case 4: run_direct<4, 1, 1, 1, 4, 3>(lay, grid, s, one, many); break;
+        case 5: run_direct<1, 4, 1, 1, 4, 3>(lay, grid, s, one, many); break;
+        case 6: run_direct<4, 1, 4, 1, 1, 2>(lay, grid, s, one, many); break;
+        default: run_direct<1, 4, 1, 4, 1, 2>(lay, grid, s, one, many); break;
+    }
+}
+
+void launch_direct_group(int config, const DirectArgs* const* p, int n, hipStream_t s) {
+    AQ_CHECK(n >= 1 && n <= kDirGroup, AQ_ERR_INVALID, "direct group size");
+    DirectGroup G{};
+    G.n = n;
+    for (int i = 0; i < n; ++i) {
+        G.p[i] = *p[i];
+        G.first[i + 1] = G.first[i] + p[i]->tilesM * p[i]->tilesN * p[i]->batch * p[i]->nsplit;
+    }
+    dispatch_direct(config, dim3(G.first[n]), s, nullptr, &G);
+}
+
+// Division of x < 2^31 by len >= 2 as (x * mul) >> (32 + shift): with
+// s = ceil(log2 len), mul = ceil(2^(31+s) / len) fits 32 bits and is exact
+// for those x (Granlund and Montgomery, PLDI 1994).
+void set_dividers(DirDigits& d) {
+    for (int k = 0; k < d.nd; ++k) {
+        uint32_t s = 1;
+        while ((uint64_t(1) << s) < d.len[k]) ++s;
+        d.mul[k] = uint32_t(((uint64_t(1) << (31 + s)) + d.len[k] - 1) / d.len[k]);
+        d.shift[k] = s - 1;
+    }
+}
+
+// k contiguous over every aligned group of four
+static bool k_runs(const DirDigits& k, const uint32_t* st) {
+    return k.nd >= 1 && st[0] == 1 && (k.nd == 1 || k.len[0] % 4 == 0);
+}
+
+// Tile shape and split of one problem: the least modelled time over the
+// shapes and power-of-two splits.  Model (clock cycles; the constants are a
+// least-regret fit to 39 contractions of the CCSD iteration at five sizes, o =
+// 5 to 20, v = 19 to 140, timed in every shape and split; its choices are
+// within 2% of the best choice on average): a chunk of 16 k costs a wave its
+// MFMAs (64 each) or the L1 accesses of its fragments, and a single wave at
+// least the load latency over the chunks in flight; blocks queue on 256 CUs;
+// operand tiles come in at a rate of the whole chip; a split pays a second
+// launch and the traffic of the partial tiles.
+struct Pick {
+    int cfg = -1;
+    uint32_t nsplit = 1;
+    double us = 1e300;
+};
+
+static Pick pick_shape(const DirectArgs& a) {
+    constexpr double kL1 = 286.0, kLatency = 1033.0, kStart = 2337.0, kBlock = 258.0, kChip = 5534.0;
+    constexpr double kLaunch = 1.5, kSplit = 2.6, kSplitBytes = 3509.0, kPerSplit = 0.06, kGHz = 2400.0;
+    Pick best;
+    const double chunks = std::ceil(a.K / 16.0);
+    for (int c = 0; c < kNDirCfg; ++c) {
+        const DirCfg& f = kDirCfg[c];
+        const double tiles = double((a.M + f.tm() - 1) / f.tm()) * double((a.N + f.tn() - 1) / f.tn()) * a.batch;
+        for (uint32_t s = 1; s <= 128; s *= 2) {
+            if (s > 1 && (chunks / s < f.wk || tiles * s > 16384)) break;
+            const double blocks = tiles * s;
+            const double per_wave = std::ceil(std::ceil(chunks / s) / f.wk);
+            const double busy = std::max(f.fm * f.fn * 256.0, (f.fm + f.fn) * kL1);
+            const double alone = per_wave * std::max(kLatency / (f.stages - 1), busy) + kStart;
+            const double queued = std::ceil(blocks / 256.0) * (per_wave * busy + kBlock);
+            const double fed = (f.tm() + f.tn()) * 128.0 * f.wk * per_wave * blocks / kChip;
+            double t = kLaunch + std::max({alone, queued, fed}) / kGHz;
+            if (s > 1) t += kSplit + tiles * f.tm() * f.tn() * 8.0 * (2 * s + 1) / kSplitBytes / kGHz + s * kPerSplit;
+            if (t < best.us) best = {c, s, t};
+        }
+    }
+    return best;
+}
+
+bool direct_contract(aq_ctx* ctx, DirectArgs a) {
+    const Pick p = pick_shape(a);
+    if (p.cfg < 0) return false;
+    const DirCfg& f = kDirCfg[p.cfg];
+    a.tilesM = (a.M + f.tm() - 1) / f.tm();
+    a.tilesN = (a.N + f.tn() - 1) / f.tn();
+    const uint32_t chunks = (a.K + 15) / 16;
+    a.kchunk = (chunks + p.nsplit - 1) / p.nsplit * 16;
+    a.nsplit = (a.K + a.kchunk - 1) / a.kchunk;
+    const uint64_t tiles = uint64_t(a.tilesM) * a.tilesN * a.batch;
+    if (tiles * a.nsplit >= (uint64_t(1) << 31)) return false;
+    Scratch part(ctx, a.nsplit > 1 ? size_t(tiles) * a.nsplit * f.tm() * f.tn() * 8 : 0);
+    for (DirDigits* d : {&a.m, &a.n, &a.k}) set_dividers(*d);
+    a.P = part.as<double>();
+    const int config = p.cfg * 4 + (k_runs(a.k, a.k.s0) ? 1 : 0) + (k_runs(a.k, a.k.s1) ? 2 : 0);
+    char name[64];
+    snprintf(name, sizeof(name), "direct_f64_%dx%d", f.tm(), f.tn());
+    const double mn = double(a.M) * a.N * a.batch;
+    // a server's slots merge same-kernel problems of different jobs; the thin
+    // ones launch alone, as thin GEMMs do
+    const bool grouped = ctx->batcher && !ctx->capture && a.M > 16 && a.N > 16 &&
+                         batcher_offer_direct(ctx, config, a, int64_t(tiles) * a.nsplit);
+    if (!grouped) {
+        TimedLaunch tl(ctx, name, 2.0 * mn * a.K,
+                       8.0 * ((double(a.M) + a.N) * a.K * a.batch + mn * (a.beta != 0.0 ? 2 : 1)));
+        dispatch_direct(config, dim3(unsigned(tiles * a.nsplit)), ctx->stream, &a, nullptr);
+    }
+    if (a.nsplit > 1) {
+        const uint32_t te = uint32_t(f.tm() * f.tn());
+        TimedLaunch tl(ctx, "direct_reduce", mn * a.nsplit, 8.0 * double(tiles) * te * (a.nsplit + 1));
+        hipLaunchKernelGGL(k_direct_reduce, dim3(unsigned(tiles * (te / 256))), dim3(256), 0, ctx->stream, a,
+                           uint32_t(f.tm()), te);
+        AQ_HIP(hipGetLastError());
+    }
+    return true;
+}
+
+}  // namespace aqamd

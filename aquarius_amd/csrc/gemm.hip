@@ -24,7 +24,7 @@
 // and consecutive tiles walk groups of 8 tile rows with m fastest, so one
 // XCD's co-resident blocks cover a square of tiles and share row panels of A
 // and column panels of B in that XCD's L2.
-#include "internal.hpp"
+#include "direct.hpp"
 
 #include <algorithm>
 #include <chrono>
@@ -988,6 +988,9 @@ static int tuned_variant(aq_ctx* ctx, const GemmDesc& d, int BM, int BN, const G
 
 namespace {
 
+// One kernel: a GEMM instantiation, or (fmt = kDirectKey, ta = its config) a
+// direct contraction's.
+constexpr int kDirectKey = -1;
 struct GroupKey {
     int fmt, ta, tb, bm, bn;
     bool operator==(const GroupKey& o) const {
@@ -1045,7 +1048,8 @@ struct GemmBatcher {
     };
     struct Item {
         GroupKey key;
-        GemmArgs a;
+        const GemmArgs* a;                // the submitter's, which waits until the launch
+        const DirectArgs* d;              // or a direct contraction's
         int64_t blocks;
         hipEvent_t ready;                 // the member's operands are written
         Launch* launch = nullptr;
@@ -1082,7 +1086,7 @@ static void launch_group(GemmBatcher* b, const GroupKey& key) {
         G.n = int(take.size());
         int64_t blocks = 0;
         for (int i = 0; i < G.n; ++i) {
-            G.p[i] = take[size_t(i)]->a;
+            if (take[size_t(i)]->a) G.p[i] = *take[size_t(i)]->a;
             G.first[i] = blocks;
             blocks += take[size_t(i)]->blocks;
             AQ_HIP(hipStreamWaitEvent(b->stream, take[size_t(i)]->ready, 0));
@@ -1095,7 +1099,13 @@ static void launch_group(GemmBatcher* b, const GroupKey& key) {
         } else {
             AQ_HIP(hipEventCreateWithFlags(&L->done, hipEventDisableTiming));
         }
-        launch_grouped(key, G, blocks, b->stream, b->cus);
+        if (key.fmt == kDirectKey) {
+            const DirectArgs* d[kMaxGroup];
+            for (int i = 0; i < G.n; ++i) d[i] = take[size_t(i)]->d;
+            launch_direct_group(key.ta, d, G.n, b->stream);
+        } else {
+            launch_grouped(key, G, blocks, b->stream, b->cus);
+        }
         AQ_HIP(hipGetLastError());
         AQ_HIP(hipEventRecord(L->done, b->stream));
     } catch (...) {
@@ -1120,11 +1130,11 @@ static void launch_group(GemmBatcher* b, const GroupKey& key) {
 // partner).  Returns true once it ran in a grouped launch (ctx->stream is
 // then ordered after it), false when it found no partner: the caller launches
 // it alone on its own stream, exactly as without grouping.
-static bool batcher_submit(aq_ctx* ctx, const GroupKey& key, const GemmArgs& a, int64_t blocks) {
+static bool batcher_submit(aq_ctx* ctx, const GroupKey& key, const GemmArgs* a, const DirectArgs* d, int64_t blocks) {
     GemmBatcher* b = ctx->batcher;
     if (!ctx->group_ready) AQ_HIP(hipEventCreateWithFlags(&ctx->group_ready, hipEventDisableTiming));
     AQ_HIP(hipEventRecord(ctx->group_ready, ctx->stream));
-    GemmBatcher::Item item{key, a, blocks, ctx->group_ready};
+    GemmBatcher::Item item{key, a, d, blocks, ctx->group_ready};
     std::unique_lock<std::mutex> lk(b->mu);
     b->pending.push_back(&item);
     struct Unlist {   // an item still pending when this frame unwinds is withdrawn (mu held)
@@ -1166,6 +1176,10 @@ static bool batcher_submit(aq_ctx* ctx, const GroupKey& key, const GemmArgs& a, 
     }
     AQ_HIP(e);
     return true;
+}
+
+bool batcher_offer_direct(aq_ctx* ctx, int config, const DirectArgs& a, int64_t blocks) {
+    return batcher_submit(ctx, GroupKey{kDirectKey, config, 0, 0, 0}, nullptr, &a, blocks);
 }
 
 GemmBatcher* batcher_create(int device, int window_us) {
@@ -1324,7 +1338,7 @@ void gemm(aq_ctx* ctx, const GemmDesc& d) {
             part.reset(new Scratch(ctx, size_t(nsplit) * d.batch * d.M * d.N * 8));
             a.P = part->as<double>();
         }
-        if (batcher_submit(ctx, GroupKey{int(d.fmt), d.transA ? 1 : 0, d.transB ? 1 : 0, BM, BN}, a,
+        if (batcher_submit(ctx, GroupKey{int(d.fmt), d.transA ? 1 : 0, d.transB ? 1 : 0, BM, BN}, &a, nullptr,
                            base_tiles * d.batch * nsplit)) {
             if (nsplit > 1)
                 launch_reduce_splitk(ctx, a.P, nsplit, d.M, d.N, d.batch, d.beta, d.C, d.ldc, d.strideC, d.cmap);

@@ -8,7 +8,7 @@
 // blocks are permuted/converted once per solve), one MFMA GEMM (batched,
 // split-K when M*N is small), and one strided pass into C when C's label
 // order interleaves the two free groups.
-#include "internal.hpp"
+#include "direct.hpp"
 
 #include <algorithm>
 #include <cstring>
@@ -345,6 +345,121 @@ static void bump(aq_tensor* t) { t->version += 1; }
 
 // ------------------------------------------------------------- contract
 
+// `labs` in the order of L's dimensions
+static std::string order_as(const std::string& labs, const Labeled& L) {
+    std::string r;
+    for (char c : L.lab)
+        if (labs.find(c) != std::string::npos) r.push_back(c);
+    return r;
+}
+
+// The label of unit stride and more than one element, or 0.
+static char unit_label(const Labeled& L) {
+    for (size_t k = 0; k < L.lab.size(); ++k)
+        if (L.stride[k] == 1 && L.len[k] > 1) return L.lab[k];
+    return 0;
+}
+
+// Labels `order` (first fastest) as digits with their strides in X and Y (an
+// absent label has stride 0); neighbours contiguous in both are merged.
+// False: more digits than a kernel takes.
+static bool digits_of(const std::string& order, const Labeled& X, const Labeled& Y, DirDigits& d) {
+    d = DirDigits{};
+    for (char c : order) {
+        const size_t x = X.lab.find(c), y = Y.lab.find(c);
+        const int64_t len = x != std::string::npos ? X.len[x] : Y.len[y];
+        if (len == 1) continue;
+        const uint32_t sx = x != std::string::npos ? uint32_t(X.stride[x]) : 0u;
+        const uint32_t sy = y != std::string::npos ? uint32_t(Y.stride[y]) : 0u;
+        if (d.nd > 0) {
+            const uint32_t l = d.len[d.nd - 1];
+            if (sx == d.s0[d.nd - 1] * l && sy == d.s1[d.nd - 1] * l) {
+                d.len[d.nd - 1] = l * uint32_t(len);
+                continue;
+            }
+        }
+        if (d.nd == kDirDigits) return false;
+        d.len[d.nd] = uint32_t(len);
+        d.s0[d.nd] = sx;
+        d.s1[d.nd] = sy;
+        d.nd += 1;
+    }
+    return true;
+}
+
+// Whether the direct kernels (direct.hip) serve a contraction better than the
+// GEMM kernels on permuted operands.  Measured per contraction of the CCSD
+// iteration, amplitude operands permuted anew and integrals cached on the GEMM
+// side (time GEMM side / direct, us):
+//  - up to 6e8 FLOP nearly everything gains: o=5, v=19 490/203, o=8, v=43
+//    699/274, o=11, v=60 860/440 over the 39 contractions.  Exceptions: rows
+//    contiguous in one operand but not in C (scattered stores), e.g. 39600 x
+//    11 x 60 11.0/14.7, from 2e5 outputs on; and a matrix-vector product along
+//    a large operand's contiguous index (12100 x 1 x 1540 31/48);
+//  - small outputs with a long inner extent (a split GEMM with a serial sum of
+//    partials): 110 x 110 x 21560 50/32, 140 x 20 x 392000 244/160;
+//  - a short side and a short inner extent against a long side: 140 x 56000 x
+//    140 111/81;
+//  - large products whose operands are both contiguous along the rows: 975^3
+//    63/44, 1540^3 190/165, 2800^3 838/783 (the GEMM side 12-23% permutes);
+//    with k contiguous in one of them the GEMM side is the faster (1540^3
+//    193/265).
+static bool direct_size(const DirectArgs& a, bool scattered, bool rows_x, bool rows_y, int64_t sizeX) {
+    const double out = double(a.M) * a.N * a.batch, flops = 2.0 * out * a.K;
+    if (scattered && out > 2e5) return false;
+    if (a.N == 1 && !rows_x && sizeX > 8000000) return false;
+    if (flops <= 6e8) return true;
+    if (out <= 2.5e4) return flops <= 2e10;
+    if (a.M <= 200 && a.K <= 200 && double(a.N) >= 50.0 * a.M) return flops <= 2e10;
+    return rows_x && rows_y && !scattered && a.M > 200 && a.N > 200 && a.K > 200 && flops <= 5e10;
+}
+
+// The contraction through the direct kernels, if they take it.  C must be
+// simple (unique labels, no broadcast, no alias).
+static bool run_direct(aq_ctx* ctx, double alpha, const Labeled& A, const Labeled& B, double beta, double* Cdata,
+                       const Labeled& C, bool c_simple, const std::string& Mlab, const std::string& Nlab,
+                       const std::string& Klab, const std::string& Blab) {
+    if (!c_simple) return false;
+    // byte offsets inside a tensor are 32-bit
+    constexpr int64_t kMost = int64_t(1) << 28;
+    if (A.size() >= kMost || B.size() >= kMost || C.size() >= kMost) return false;
+    const int64_t M = prod_len(Mlab, A), N = prod_len(Nlab, B), K = prod_len(Klab, A), NB = prod_len(Blab, A);
+    // the rows of the product are the group that holds C's unit-stride label,
+    // so that consecutive lanes store consecutive elements
+    const char uc = unit_label(C);
+    const bool swap = Nlab.find(uc) != std::string::npos || (Mlab.find(uc) == std::string::npos && N > M);
+    const Labeled &X = swap ? B : A, &Y = swap ? A : B;
+    const std::string &Rl = swap ? Nlab : Mlab, &Cl = swap ? Mlab : Nlab;
+    // an operand's unit-stride label goes first in its group (coalesced reads)
+    const char ux = unit_label(X), uy = unit_label(Y);
+    auto has = [](const std::string& labs, char c) { return c && labs.find(c) != std::string::npos; };
+    const bool rows_x = has(Rl, ux), rows_y = has(Cl, uy);
+    DirectArgs a{};
+    std::string bl;
+    for (char c : order_as(Blab, C))
+        if (C.len[C.lab.find(c)] != 1) bl.push_back(c);
+    if (bl.size() > 1) return false;
+    if (!digits_of(order_as(Rl, rows_x ? X : C), X, C, a.m) || !digits_of(order_as(Cl, rows_y ? Y : C), Y, C, a.n) ||
+        !digits_of(order_as(Klab, has(Klab, ux) ? X : Y), X, Y, a.k))
+        return false;
+    a.M = uint32_t(swap ? N : M);
+    a.N = uint32_t(swap ? M : N);
+    a.K = uint32_t(K);
+    a.batch = uint32_t(NB);
+    if (!direct_size(a, rows_x && has(Rl, uc) && ux != uc, rows_x, rows_y, X.size())) return false;
+    a.A = X.data;
+    a.B = Y.data;
+    a.C = Cdata;
+    a.alpha = alpha;
+    a.beta = beta;
+    if (!bl.empty()) {
+        a.bsA = uint32_t(X.stride[X.lab.find(bl[0])]);
+        a.bsB = uint32_t(Y.stride[Y.lab.find(bl[0])]);
+        a.bsC = uint32_t(C.stride[C.lab.find(bl[0])]);
+    }
+    return direct_contract(ctx, a);
+}
+
 static void contract_impl(aq_ctx* ctx, double alpha, const aq_tensor* tA, const char* ia, const aq_tensor* tB,
                           const char* ib, double beta, aq_tensor* tC, const char* ic) {
     Labeled A0 = label(tA, ia, "A"), B0 = label(tB, ib, "B"), C0 = label(tC, ic, "C");
@@ -388,6 +503,11 @@ static void contract_impl(aq_ctx* ctx, double alpha, const aq_tensor* tA, const 
             launch_strided_sum(ctx, p, 0.0, tC->data, beta, tC->data);
             bump(tC);
         }
+        return;
+    }
+
+    if (fmt == FMT_F64 && run_direct(ctx, alpha, A, B, beta, tC->data, C0, c_simple, Mlab, Nlab, Klab, Blab_c)) {
+        bump(tC);
         return;
     }
 
