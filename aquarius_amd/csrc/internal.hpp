@@ -281,8 +281,9 @@ void launch_ladder_unpack(aq_ctx* ctx, const double* Sp, const double* Sm, int v
 // Tau, TauSA, T2SA from T1 and T2 in one pass (rhfccsd.cxx:231-238)
 void launch_tau_sa(aq_ctx* ctx, const double* T1, const double* T2, int v, int o, double* Tau, double* TauSA,
                    double* T2SA);
-// max |X(p,q,r,s) - X(q,p,s,r)| of X[n1,n1,n2,n2] (synchronising)
-double pair_asymmetry(aq_ctx* ctx, const double* X, int n1, int n2, int slot);
+// max |X(p,q,r,s) - X(q,p,s,r)| and max |X| of X[n1,n1,n2,n2] into result
+// slots `slot` and `slot` + 1; caller syncs
+void launch_pair_asymmetry(aq_ctx* ctx, const double* X, int n1, int n2, int slot);
 
 // AO integrals (elementwise.hip): (pq|rs) [n,n,n,n] from the compact
 // canonical shell-quartet storage (fe::CompactEri), all pointers on the device

@@ -133,9 +133,11 @@ struct aq_rhfccsd {
     void derive_packed() {
         packed = false;
         if (cfg.packed_ladder && o >= 2 && v >= 2) {
-            const double dV = pair_asymmetry(ctx, dptr(VABCD), v, v, 0);
-            const double dI = pair_asymmetry(ctx, dptr(VABIJ), v, o, 0);
-            const double nV = VABCD.norm(0), nI = VABIJ.norm(0);
+            launch_pair_asymmetry(ctx, dptr(VABCD), v, v, 0);
+            launch_pair_asymmetry(ctx, dptr(VABIJ), v, o, 2);
+            AQ_HIP(hipStreamSynchronize(ctx->stream));
+            const double* h = ctx->h_result;
+            const double dV = h[0], nV = h[1], dI = h[2], nI = h[3];
             packed = dV <= 1e-13 * (1.0 + nV) && dI <= 1e-13 * (1.0 + nI);
         }
         if (!packed) {
@@ -149,7 +151,8 @@ struct aq_rhfccsd {
         }
         const int64_t P = int64_t(v) * (v + 1) / 2, Q = int64_t(v) * (v - 1) / 2;
         const int64_t Op = int64_t(o) * (o + 1) / 2, Om = int64_t(o) * (o - 1) / 2;
-        auto mk = [&](std::initializer_list<int64_t> l) { return Tensor(ctx, std::vector<int64_t>(l), true); };
+        // every element is written before it is read: no clearing pass
+        auto mk = [&](std::initializer_list<int64_t> l) { return Tensor(ctx, std::vector<int64_t>(l), false); };
         if (!Vp.handle()) {
             Vp = mk({P, P});
             Vm = mk({Q, Q});
@@ -166,7 +169,10 @@ struct aq_rhfccsd {
     // rhfccsd.cxx:45-98
     void setup() {
         const int64_t vo[2] = {v, o}, vvoo[4] = {v, v, o, o}, voov[4] = {v, o, o, v};
-        auto mk = [&](std::initializer_list<int64_t> l) { return Tensor(ctx, std::vector<int64_t>(l), true); };
+        // the tensors a caller can read before they are formed are cleared
+        auto mk = [&](std::initializer_list<int64_t> l, bool clear = true) {
+            return Tensor(ctx, std::vector<int64_t>(l), clear);
+        };
         (void)vo;
         (void)vvoo;
         (void)voov;
@@ -175,10 +181,10 @@ struct aq_rhfccsd {
         Z1 = mk({v, o});
         Z2 = mk({v, v, o, o});
         Tau = mk({v, v, o, o});
-        T2SA = mk({v, v, o, o});
-        TauSA = mk({v, v, o, o});
-        VABIJSA = mk({v, v, o, o});
-        VAIJBSA = mk({v, o, o, v});
+        T2SA = mk({v, v, o, o}, false);
+        TauSA = mk({v, v, o, o}, false);
+        VABIJSA = mk({v, v, o, o}, false);
+        VAIJBSA = mk({v, o, o, v}, false);
         FAE = mk({v, v});
         FMI = mk({o, o});
         FME = mk({o, v});
