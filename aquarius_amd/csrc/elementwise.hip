@@ -219,6 +219,119 @@ void launch_strided_convert(aq_ctx* ctx, const StridedPlan& p, const double* src
     }
 }
 
+// ------------------------------------------- X[d] = beta X[d] + alpha X[pi d]
+//
+// A sum whose source is the destination under a permutation of dimensions that
+// is its own inverse (Z["abij"] += Z["baji"], W["mnij"] += W["nmji"]): the
+// elements d and pi d are read together and written together, so no snapshot
+// of the source is needed.  HBM-bound, one read and one write per element: a
+// copy plus a transposing sum read three times and wrote twice (o = 31, v =
+// 189, 275 MB: 104 + 182 us, in place 132 us).
+struct PairPlan {
+    int nd;
+    int64_t len[MAXDIM], st[MAXDIM];
+    int part[MAXDIM];           // pi: dimension k of d is dimension part[k] of pi d
+};
+
+__device__ __forceinline__ void pair_offsets(const PairPlan& p, int skip0, int skip1, int64_t x, int64_t& off,
+                                             int64_t& poff) {
+    off = 0;
+    poff = 0;
+    for (int k = 0; k < p.nd; ++k) {
+        if (k == skip0 || k == skip1) continue;
+        const int64_t q = x / p.len[k], c = x - q * p.len[k];
+        x = q;
+        off += c * p.st[k];
+        poff += c * p.st[p.part[k]];
+    }
+}
+
+// Dimension d0 (unit stride) changes places with d1: a block holds the 32 x 32
+// tile (i0, i1) of one slab of the other dimensions and its mirror, tile (i1,
+// i0) of the partner slab, in LDS; the block of the pair with the lower slab
+// offset (then tile) does both.
+constexpr int PT = 32;
+__global__ __launch_bounds__(TPB) void k_pair_transpose(PairPlan p, int d0, int d1, int64_t nt, int64_t total,
+                                                        double alpha, double beta, double* __restrict__ X) {
+    __shared__ double ta[PT][PT + 1], tb[PT][PT + 1];
+    const int tx = threadIdx.x % PT, ty = threadIdx.x / PT;
+    constexpr int R = TPB / PT, N = PT / R;
+    const int64_t L = p.len[d0], S = p.st[d1];
+    for (int64_t w = blockIdx.x; w < total; w += gridDim.x) {
+        const int64_t t0 = w % nt, t1 = w / nt % nt;
+        int64_t off, poff;
+        pair_offsets(p, d0, d1, w / (nt * nt), off, poff);
+        if (poff < off || (poff == off && t1 < t0)) continue;      // the partner's block does it
+        const bool self = poff == off && t0 == t1;
+        double a[N], b[N];
+        __syncthreads();   // the previous pair's tiles have been read
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            const int64_t i0 = t0 * PT + tx, i1 = t1 * PT + ty + R * k;   // X(i0, i1)
+            const int64_t j0 = t1 * PT + tx, j1 = t0 * PT + ty + R * k;   // its mirror's tile
+            a[k] = i0 < L && i1 < L ? X[off + i0 + i1 * S] : 0.0;
+            b[k] = j0 < L && j1 < L ? X[poff + j0 + j1 * S] : 0.0;
+            ta[ty + R * k][tx] = a[k];
+            tb[ty + R * k][tx] = b[k];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            const int64_t i0 = t0 * PT + tx, i1 = t1 * PT + ty + R * k;
+            const int64_t j0 = t1 * PT + tx, j1 = t0 * PT + ty + R * k;
+            const double pa = alpha * tb[tx][ty + R * k], pb = alpha * ta[tx][ty + R * k];
+            if (i0 < L && i1 < L) X[off + i0 + i1 * S] = beta == 0.0 ? pa : beta * a[k] + pa;
+            if (!self && j0 < L && j1 < L) X[poff + j0 + j1 * S] = beta == 0.0 ? pb : beta * b[k] + pb;
+        }
+    }
+}
+
+// Dimension d0 (unit stride) stays in place: whole rows change places.
+__global__ __launch_bounds__(TPB) void k_pair_rows(PairPlan p, int d0, int64_t rows, double alpha, double beta,
+                                                   double* __restrict__ X) {
+    const int64_t L = p.len[d0], n = rows * L;
+    for (int64_t x = int64_t(blockIdx.x) * TPB + threadIdx.x; x < n; x += int64_t(gridDim.x) * TPB) {
+        const int64_t row = x / L, i = x - row * L;
+        int64_t off, poff;
+        pair_offsets(p, d0, d0, row, off, poff);
+        if (poff < off) continue;
+        const double a = X[off + i], b = X[poff + i];
+        const double pa = alpha * b, pb = alpha * a;
+        X[off + i] = beta == 0.0 ? pa : beta * a + pa;
+        if (poff != off) X[poff + i] = beta == 0.0 ? pb : beta * b + pb;
+    }
+}
+
+bool launch_sum_pairs(aq_ctx* ctx, const StridedPlan& sp, double alpha, double beta, double* X) {
+    if (sp.nr != 0 || sp.nd == 0 || sp.nout == 0) return false;
+    PairPlan p{};
+    p.nd = sp.nd;
+    int d0 = -1;
+    for (int k = 0; k < sp.nd; ++k) {
+        p.len[k] = sp.len[k];
+        p.st[k] = sp.sdst[k];
+        p.part[k] = -1;
+        for (int m = 0; m < sp.nd; ++m)
+            if (sp.sdst[m] == sp.ssrc[k] && sp.ssrc[m] == sp.sdst[k] && sp.len[m] == sp.len[k]) p.part[k] = m;
+        if (p.part[k] < 0) return false;      // not its own inverse, or a broadcast
+        if (sp.sdst[k] == 1) d0 = k;
+    }
+    if (d0 < 0) return false;
+    const int d1 = p.part[d0];
+    TimedLaunch tl(ctx, "sum_pairs", 0.0, 16.0 * sp.nout);
+    if (d1 != d0) {
+        const int64_t nt = (p.len[d0] + PT - 1) / PT;
+        const int64_t total = nt * nt * (sp.nout / (p.len[d0] * p.len[d1]));
+        hipLaunchKernelGGL(k_pair_transpose, dim3(grid_for(total, 1)), dim3(TPB), 0, ctx->stream, p, d0, d1, nt, total,
+                           alpha, beta, X);
+    } else {
+        hipLaunchKernelGGL(k_pair_rows, dim3(grid_for(sp.nout, TPB * 4)), dim3(TPB), 0, ctx->stream, p, d0,
+                           sp.nout / p.len[d0], alpha, beta, X);
+    }
+    AQ_HIP(hipGetLastError());
+    return true;
+}
+
 // -------------------------------------------------------------------- fill
 
 __global__ __launch_bounds__(TPB) void k_fill(double* x, int64_t n, double alpha, double beta) {

@@ -224,6 +224,9 @@ void launch_fill(aq_ctx* ctx, double* x, int64_t n, double alpha, double beta);
 void launch_zero_bytes(aq_ctx* ctx, void* p, size_t bytes);   // bytes % 4 == 0; a kernel, not a memset
 void launch_strided_sum(aq_ctx* ctx, const StridedPlan& p, double alpha, const double* src,
                         double beta, double* dst);
+// X[d] = beta X[d] + alpha X[pi d] in place, for a plan whose source is the
+// destination under a permutation pi that is its own inverse; false: not taken
+bool launch_sum_pairs(aq_ctx* ctx, const StridedPlan& p, double alpha, double beta, double* X);
 void launch_strided_convert(aq_ctx* ctx, const StridedPlan& p, const double* src, void* dst, Fmt fmt,
                             int64_t plane_stride);
 void launch_div(aq_ctx* ctx, const double* A, const double* B, double* C, int64_t n, double alpha, double beta);

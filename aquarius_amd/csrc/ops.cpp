@@ -694,6 +694,10 @@ static void sum_impl(aq_ctx* ctx, double alpha, const aq_tensor* tA, const char*
     bool identity = p.nr == 0;
     for (int k = 0; k < p.nd && identity; ++k) identity = p.ssrc[k] == p.sdst[k];
     if (overlaps(tA, tB) && !identity) {
+        if (!A.has_repeat && !B.has_repeat && alpha != 0.0 && launch_sum_pairs(ctx, p, alpha, beta, tB->data)) {
+            bump(tB);
+            return;
+        }
         // snapshot the source before writing the destination (aliased sum)
         Scratch snap(ctx, size_t(tA->size) * 8);
         AQ_HIP(hipMemcpyAsync(snap.p, tA->data, size_t(tA->size) * 8, hipMemcpyDeviceToDevice, ctx->stream));
