@@ -8,6 +8,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #pragma clang fp contract(off)
 
@@ -561,29 +562,64 @@ void launch_scatter_keys(aq_ctx* ctx, double* x, int64_t n, const int64_t* keys,
 }
 
 // -------------------------------------------------------------- split-K
-
-__global__ __launch_bounds__(TPB) void k_splitk(const double* __restrict__ P, int nsplit, int64_t m, int64_t n,
-                                                 int64_t batch, double beta, double* C, int64_t ldc, int64_t strideC,
-                                                 CMap map) {
-    const int64_t mn = m * n, tot = mn * batch;
-    for (int64_t i = int64_t(blockIdx.x) * TPB + threadIdx.x; i < tot; i += int64_t(gridDim.x) * TPB) {
+//
+// C = beta C + sum over the splits, in order.  FP64 partials hold alpha times
+// the accumulators; the FP32-accumulated formats keep the accumulators
+// themselves (float, exact) and are scaled here, which gives the same sums
+// from half the bytes.  Eight loads are in flight per thread: with one, a
+// small output of many splits (192 x 192 of 220) waited for memory 220 times.
+template <typename T, typename I>
+__global__ __launch_bounds__(TPB) void k_splitk(const T* __restrict__ P, int nsplit, int64_t m, int64_t n,
+                                                 int64_t batch, double alpha, double beta, double* C, int64_t ldc,
+                                                 int64_t strideC, CMap map) {
+    const I mn = I(m * n), tot = I(m * n * batch), stride = I(gridDim.x) * I(TPB);
+    auto term = [&](T x) { return sizeof(T) == 8 ? double(x) : alpha * double(x); };
+    for (I i = I(blockIdx.x) * I(TPB) + I(threadIdx.x); i < tot; i += stride) {
+        const T* p = P + i;
         double s = 0.0;
-        for (int k = 0; k < nsplit; ++k) s += P[int64_t(k) * tot + i];
-        const int64_t b = i / mn, r = i % mn;
-        const int64_t col = r / m, row = r % m;
+        int k = 0;
+        for (; k + 8 <= nsplit; k += 8) {
+            T x[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) x[u] = p[int64_t(k + u) * int64_t(tot)];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) s += term(x[u]);
+        }
+        if (k + 4 <= nsplit) {
+            T x[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) x[u] = p[int64_t(k + u) * int64_t(tot)];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) s += term(x[u]);
+            k += 4;
+        }
+        for (; k < nsplit; ++k) s += term(p[int64_t(k) * int64_t(tot)]);
+        const I b = i / mn, r = i - b * mn;
+        const I col = r / I(m), row = r - col * I(m);
         const int64_t off = map.mapped ? cmap_digits(map.nm, map.ml, map.ms, row) + cmap_digits(map.nn, map.nl, map.ns, col)
-                                       : row + col * ldc;
-        double* c = C + b * strideC + off;
+                                       : int64_t(row) + int64_t(col) * ldc;
+        double* c = C + int64_t(b) * strideC + off;
         *c = beta == 0.0 ? s : beta * *c + s;
     }
 }
 
-void launch_reduce_splitk(aq_ctx* ctx, const double* P, int nsplit, int64_t m, int64_t n, int64_t batch, double beta,
-                          double* C, int64_t ldc, int64_t strideC, const CMap& map) {
+void launch_reduce_splitk(aq_ctx* ctx, const void* P, bool f32, int nsplit, int64_t m, int64_t n, int64_t batch,
+                          double alpha, double beta, double* C, int64_t ldc, int64_t strideC, const CMap& map) {
     const int64_t tot = m * n * batch;
-    TimedLaunch tl(ctx, "splitk_reduce", double(tot) * nsplit, 8.0 * tot * (nsplit + 1));
-    hipLaunchKernelGGL(k_splitk, dim3(grid_for(tot, TPB)), dim3(TPB), 0, ctx->stream, P, nsplit, m, n, batch, beta, C,
-                       ldc, strideC, map);
+    const double bytes = (f32 ? 4.0 : 8.0) * tot * nsplit + 8.0 * tot * (beta != 0.0 ? 2 : 1);
+    TimedLaunch tl(ctx, "splitk_reduce", double(tot) * nsplit, bytes);
+    const dim3 grid(grid_for(tot, TPB));
+    auto go = [&](auto* p, auto zero) {
+        typedef std::remove_const_t<std::remove_pointer_t<decltype(p)>> T;
+        hipLaunchKernelGGL((k_splitk<T, decltype(zero)>), grid, dim3(TPB), 0, ctx->stream, p, nsplit, m, n, batch, alpha,
+                           beta, C, ldc, strideC, map);
+    };
+    // 32-bit indices while index + stride cannot wrap
+    const bool small = tot < (int64_t(1) << 31);
+    if (f32 && small) go(static_cast<const float*>(P), uint32_t(0));
+    else if (f32) go(static_cast<const float*>(P), int64_t(0));
+    else if (small) go(static_cast<const double*>(P), uint32_t(0));
+    else go(static_cast<const double*>(P), int64_t(0));
     AQ_HIP(hipGetLastError());
 }
 

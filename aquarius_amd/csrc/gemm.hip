@@ -3,8 +3,9 @@
 //   C[m + n*ldc] = alpha * sum_k opA(m,k) * opB(k,n) + beta * C[m + n*ldc]
 //   opA(m,k) = transA ? A[k + m*lda] : A[m + k*lda]
 //   opB(k,n) = transB ? B[n + k*ldb] : B[k + n*ldb]
-// with a batch dimension (grid z) and optional split-K (partials in FP64,
-// reduced in a fixed order, so results do not depend on scheduling).
+// with a batch dimension (grid z) and optional split-K (partials of the
+// accumulators' precision, reduced in FP64 in a fixed order, so results do not
+// depend on scheduling).
 //
 // FP64 path: v_mfma_f64_16x16x4f64.  FP32 path: v_mfma_f32_16x16x4f32.
 // Both share one template: 256 threads = 4 waves, block tile BM x BN, BK = 16,
@@ -55,7 +56,7 @@ struct GemmArgs {
     double alpha, beta;
     double* C;
     int64_t ldc, strideC;
-    double* P;   // split-K partials [split][batch][M*N], or null
+    void* P;     // split-K partials [split][batch][M*N] (FP64: alpha * acc; else the float acc), or null
     int batch;
     int transA, transB;
     int off32;   // every per-thread tile offset of A and B fits 32 bits (FP64/FP32 interior fast path)
@@ -75,6 +76,22 @@ __device__ __forceinline__ void column_offsets(const GemmArgs& g, bool mapped, i
             const int64_t n = col(j, r);
             co[j][r] = mapped ? (n < g.N ? cmap_digits(g.cmap.nn, g.cmap.nl, g.cmap.ns, n) : 0) : n * ldc;
         }
+}
+
+// One lane's partial tile: FM x FN blocks, rows m, m + 16, ..., columns col(j, r).
+template <int FM, int FN, typename T, class Acc, class ColOf>
+__device__ __forceinline__ void store_partial(const GemmArgs& g, T* P, const Acc (&acc)[FM][FN], int64_t m, ColOf col) {
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+        if (m + i * 16 >= g.M) break;
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int64_t n = col(j, r);
+                if (n < g.N) P[m + i * 16 + n * g.M] = sizeof(T) == 8 ? T(g.alpha * double(acc[i][j][r])) : T(acc[i][j][r]);
+            }
+    }
 }
 
 // tile t -> (tile row, tile col).  G == 0: rows of tiles, n fastest.  G > 0:
@@ -405,16 +422,23 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs g, int64_t bx, int bz) 
     }
 
     // epilogue: lane holds C[m = mb + lane%16][n = nb + drow(lane, r)]
-    double* Cb = g.P ? g.P + (int64_t(split) * g.batch + b) * (g.M * g.N) : g.C + int64_t(b) * g.strideC;
-    const int64_t ldc = g.P ? g.M : g.ldc;
-    const bool mapped = !g.P && g.cmap.mapped;
+    if (g.P) {
+        // T is the accumulators' type: what the reduction adds
+        T* Pb = static_cast<T*>(g.P) + (int64_t(split) * g.batch + b) * (g.M * g.N);
+        store_partial<FM, FN>(g, Pb, acc, m0 + wm * WTM + lane % 16,
+                              [&](int j, int r) { return n0 + wn * WTN + j * 16 + Mfma<T>::drow(lane, r); });
+        return;
+    }
+    double* Cb = g.C + int64_t(b) * g.strideC;
+    const int64_t ldc = g.ldc;
+    const bool mapped = g.cmap.mapped;
     int64_t co[FN][4];
     column_offsets<FN>(g, mapped, ldc,
                        [&](int j, int r) { return n0 + wn * WTN + j * 16 + Mfma<T>::drow(lane, r); }, co);
     // per row of blocks, every C value is read before any is written: one
     // memory round trip per row instead of one per element (a load after a
     // store to C could alias it, so the compiler keeps that order)
-    const bool addc = !g.P && g.beta != 0.0;
+    const bool addc = g.beta != 0.0;
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
         const int64_t m = m0 + wm * WTM + i * 16 + lane % 16;
@@ -725,15 +749,21 @@ __device__ __forceinline__ void gemm_tile_bf16x3(const GemmArgs g, int64_t bx, i
         }
     }
 
-    double* Cb = g.P ? g.P + (int64_t(split) * g.batch + b) * (g.M * g.N) : g.C + int64_t(b) * g.strideC;
-    const int64_t ldc = g.P ? g.M : g.ldc;
-    const bool mapped = !g.P && g.cmap.mapped;
+    if (g.P) {
+        float* Pb = static_cast<float*>(g.P) + (int64_t(split) * g.batch + b) * (g.M * g.N);
+        store_partial<FM, FN>(g, Pb, acc, m0 + wm * WTM + lane % 16,
+                              [&](int j, int r) { return n0 + wn * WTN + j * 16 + 4 * (lane / 16) + r; });
+        return;
+    }
+    double* Cb = g.C + int64_t(b) * g.strideC;
+    const int64_t ldc = g.ldc;
+    const bool mapped = g.cmap.mapped;
     int64_t co[FN][4];
     column_offsets<FN>(g, mapped, ldc, [&](int j, int r) { return n0 + wn * WTN + j * 16 + 4 * (lane / 16) + r; },
                        co);
     // per row of blocks, every C value is read before any is written (one
     // memory round trip per row instead of one per element)
-    const bool addc = !g.P && g.beta != 0.0;
+    const bool addc = g.beta != 0.0;
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
         const int64_t m = m0 + wm * WTM + i * 16 + lane % 16;
@@ -843,10 +873,29 @@ static void run_cfg(aq_ctx* ctx, const GemmArgs& a, dim3 grid, int variant) {
 #undef AQ_LAUNCH
 }
 
-// Measured on MI355X (square 8192^3 / ladder / ring shapes): the register-lean
-// BK-16 variant with two waves per SIMD hides the global-load latency that a
-// single wave per SIMD exposes (FP64 35 -> 56 TF/s; FP32 unchanged at ~108).
-int default_gemm_variant(Fmt fmt) { return fmt == FMT_BF16X2 ? 0 : 2; }
+// The variant of the large tile without a tuner.
+//
+// FP64/FP32, measured on MI355X (square 8192^3 / ladder / ring shapes): the
+// register-lean BK-16 variant with two waves per SIMD hides the global-load
+// latency that a single wave per SIMD exposes (FP64 35 -> 56 TF/s; FP32
+// unchanged at ~108).
+//
+// BF16x3: 128 x 128 blocks, two per CU (rounds of 512), or 256 x 256 with
+// eight waves and direct loads, one per CU (rounds of 256).  A full round of
+// the large blocks takes 1.31 times a round of the small ones (2800^3, one
+// round of either: 210 and 160 us) for twice the tiles, so the choice is the
+// smaller rounds * time: 6080^3 split 4 ways 1459 -> 1153 us, 4959 x 841 x
+// 29241 868 -> 624, 18528 x 528 x 18528 1777 -> 1161, 19600 x 400 x 400 65 ->
+// 58; 6144 x 1024 x 36864 (96 large blocks) stays at 1590 against 2427.
+static int default_gemm_variant(const GemmDesc& d, int nsplit) {
+    if (d.fmt != FMT_BF16X2) return 2;
+    if (d.M < 256 || d.N < 256) return 0;
+    auto rounds = [&](int64_t b, int64_t resident) {
+        const int64_t blocks = ((d.M + b - 1) / b) * ((d.N + b - 1) / b) * d.batch * nsplit;
+        return double((blocks + resident - 1) / resident);
+    };
+    return 1.31 * rounds(256, 256) < rounds(128, 512) ? 3 : 0;
+}
 
 template <int BM, int BN, int WM, int WN, bool DIRECT = false>
 static void run_cfg_bf16(aq_ctx* ctx, const GemmArgs& a, dim3 grid) {
@@ -925,8 +974,10 @@ int half_octave(int64_t x) { return int(std::lround(2.0 * std::log2(double(std::
 
 }  // namespace
 
+static size_t partial_bytes(Fmt fmt) { return fmt == FMT_F64 ? 8 : 4; }
+
 static int tuned_variant(aq_ctx* ctx, const GemmDesc& d, int BM, int BN, const GemmArgs& a) {
-    const int defv = default_gemm_variant(d.fmt);
+    const int defv = default_gemm_variant(d, a.nsplit);
     if (!(BM == 128 && BN == 128)) return defv;             // only the large tile has variants
     TuneKey key{ctx->device, int(d.fmt), d.transA, d.transB, half_octave(d.M), half_octave(d.N), half_octave(d.K),
                 half_octave(d.batch)};
@@ -939,7 +990,7 @@ static int tuned_variant(aq_ctx* ctx, const GemmDesc& d, int BM, int BN, const G
     if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return defv;
     // trial output (and partials) so that C is untouched
     const size_t cbytes = size_t(a.M) * size_t(a.N) * size_t(a.batch) * 8;
-    const size_t pbytes = a.nsplit > 1 ? size_t(a.nsplit) * cbytes : 0;
+    const size_t pbytes = a.nsplit > 1 ? size_t(a.nsplit) * cbytes / 8 * partial_bytes(d.fmt) : 0;
     if (ctx_in_use(ctx) + cbytes + pbytes > ctx->budget) return defv;
     TuneEntry e;
     {
@@ -949,7 +1000,7 @@ static int tuned_variant(aq_ctx* ctx, const GemmDesc& d, int BM, int BN, const G
         t.ldc = a.M;
         t.strideC = a.M * a.N;
         t.beta = 0.0;
-        t.P = a.nsplit > 1 ? tp.as<double>() : nullptr;
+        t.P = a.nsplit > 1 ? tp.p : nullptr;
         t.cmap = CMap{};   // the trial writes its scratch output column-major
         hipEvent_t e0, e1;
         AQ_HIP(hipEventCreate(&e0));
@@ -1335,27 +1386,28 @@ void gemm(aq_ctx* ctx, const GemmDesc& d) {
     if (ctx->batcher && !ctx->capture && group_shape(d.fmt, BM, BN)) {
         std::unique_ptr<Scratch> part;
         if (nsplit > 1) {
-            part.reset(new Scratch(ctx, size_t(nsplit) * d.batch * d.M * d.N * 8));
-            a.P = part->as<double>();
+            part.reset(new Scratch(ctx, size_t(nsplit) * d.batch * d.M * d.N * partial_bytes(d.fmt)));
+            a.P = part->p;
         }
         if (batcher_submit(ctx, GroupKey{int(d.fmt), d.transA ? 1 : 0, d.transB ? 1 : 0, BM, BN}, &a, nullptr,
                            base_tiles * d.batch * nsplit)) {
             if (nsplit > 1)
-                launch_reduce_splitk(ctx, a.P, nsplit, d.M, d.N, d.batch, d.beta, d.C, d.ldc, d.strideC, d.cmap);
+                launch_reduce_splitk(ctx, a.P, d.fmt != FMT_F64, nsplit, d.M, d.N, d.batch, d.alpha, d.beta, d.C, d.ldc,
+                             d.strideC, d.cmap);
             return;
         }
         a.P = nullptr;   // alone: the launch below allocates its own partials
     }
 
     int variant = ctx->gemm_variant[d.fmt];
-    if (variant < 0) variant = ctx->autotune ? tuned_variant(ctx, d, BM, BN, a) : default_gemm_variant(d.fmt);
+    if (variant < 0) variant = ctx->autotune ? tuned_variant(ctx, d, BM, BN, a) : default_gemm_variant(d, nsplit);
     variant_shape(d.fmt, variant, d.M, d.N, BM, BN);
     const int64_t tiles = ((d.M + BM - 1) / BM) * ((d.N + BN - 1) / BN);
 
     std::unique_ptr<Scratch> part;
     if (nsplit > 1) {
-        part.reset(new Scratch(ctx, size_t(nsplit) * d.batch * d.M * d.N * 8));
-        a.P = part->as<double>();
+        part.reset(new Scratch(ctx, size_t(nsplit) * d.batch * d.M * d.N * partial_bytes(d.fmt)));
+        a.P = part->p;
     }
     dim3 grid(unsigned(tiles), 1, unsigned(d.batch * nsplit));
     const double flops = 2.0 * double(d.M) * double(d.N) * double(d.K) * double(d.batch);
@@ -1381,7 +1433,8 @@ void gemm(aq_ctx* ctx, const GemmDesc& d) {
         AQ_HIP(hipGetLastError());
     }
     if (nsplit > 1)
-        launch_reduce_splitk(ctx, a.P, nsplit, d.M, d.N, d.batch, d.beta, d.C, d.ldc, d.strideC, d.cmap);
+        launch_reduce_splitk(ctx, a.P, d.fmt != FMT_F64, nsplit, d.M, d.N, d.batch, d.alpha, d.beta, d.C, d.ldc,
+                             d.strideC, d.cmap);
 }
 
 int autotune_entries(aq_tune_entry* out, int cap) {

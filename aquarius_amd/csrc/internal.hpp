@@ -262,8 +262,9 @@ __device__ __forceinline__ int64_t cmap_digits(int nd, const int64_t* len, const
     }
     return nd > 0 ? off + int64_t(r) * st[nd - 1] : 0;
 }
-void launch_reduce_splitk(aq_ctx* ctx, const double* P, int nsplit, int64_t m, int64_t n,
-                          int64_t batch, double beta, double* C, int64_t ldc, int64_t strideC, const CMap& map);
+// P: partials, double (alpha applied) or, f32, the float accumulators
+void launch_reduce_splitk(aq_ctx* ctx, const void* P, bool f32, int nsplit, int64_t m, int64_t n, int64_t batch,
+                          double alpha, double beta, double* C, int64_t ldc, int64_t strideC, const CMap& map);
 
 // fused CCSD update (elementwise.hip)
 struct UpdateArgs {
