@@ -51,13 +51,18 @@ __device__ __forceinline__ uint32_t digit_offset(const DirDigits& d, const uint3
     return d.nd > 0 ? off + x * st[d.nd - 1] : 0u;
 }
 
-template <int FM, int FN, int WM, int WN, int WK, int ST, bool VA, bool VB>
-__device__ __forceinline__ void direct_tile(const DirectArgs& g, uint32_t bid) {
+// LDS of a tile: the k tables, then (WK > 1) the waves' accumulators.
+constexpr int direct_lds(int fm, int fn, int wm, int wn, int wk) {
+    const int red = wk > 1 ? wk * fm * fn * wm * wn * 256 * 8 : 0, tab = 2 * kKT * 4;
+    return red > tab ? red : tab;
+}
+
+// TILE: the tile goes to the partial buffer whatever the split (batched stages,
+// whose assembly adds the tiles of several products).
+template <int FM, int FN, int WM, int WN, int WK, int ST, bool VA, bool VB, bool TILE = false>
+__device__ __forceinline__ void direct_tile(const DirectArgs& g, uint32_t bid, char* lds) {
     static_assert(WM * WN * WK == 4, "4 waves");
     constexpr int TM = 16 * FM * WM, TN = 16 * FN * WN;
-    constexpr int RED = WK > 1 ? WK * TM * TN * 8 : 16;
-    constexpr int TAB = 2 * kKT * 4;
-    __shared__ __attribute__((aligned(16))) char lds[RED > TAB ? RED : TAB];
     uint32_t* ta = reinterpret_cast<uint32_t*>(lds);
     uint32_t* tb = ta + kKT;
 
@@ -184,7 +189,7 @@ __device__ __forceinline__ void direct_tile(const DirectArgs& g, uint32_t bid) {
 
     // lane holds tile element (m = l16 of block i, n = q + 4r of block j)
     double* Cb = g.C + uint64_t(b) * g.bsC;
-    if (WK == 1 && g.nsplit == 1) {
+    if (!TILE && WK == 1 && g.nsplit == 1) {
         uint32_t cn[FN][4];
 #pragma unroll
         for (int j = 0; j < FN; ++j)
@@ -240,7 +245,7 @@ __device__ __forceinline__ void direct_tile(const DirectArgs& g, uint32_t bid) {
             v[r] = s;
         }
     }
-    if (g.nsplit > 1) {
+    if (TILE || g.nsplit > 1) {
         double* P = g.P + uint64_t(bt) * g.nsplit * TE;
         double* mine = P + uint64_t(split) * TE;
         if (WK > 1) {
@@ -303,7 +308,8 @@ __device__ __forceinline__ uint32_t xcd_order(uint32_t bid, uint32_t nb) {
 
 template <int FM, int FN, int WM, int WN, int WK, int ST, bool VA, bool VB>
 __global__ __launch_bounds__(256) void k_direct(DirectArgs g) {
-    direct_tile<FM, FN, WM, WN, WK, ST, VA, VB>(g, xcd_order(blockIdx.x, gridDim.x));
+    __shared__ __attribute__((aligned(16))) char lds[direct_lds(FM, FN, WM, WN, WK)];
+    direct_tile<FM, FN, WM, WN, WK, ST, VA, VB>(g, xcd_order(blockIdx.x, gridDim.x), lds);
 }
 
 // The tiles of up to kDirGroup problems of different contexts in one launch;
@@ -316,9 +322,10 @@ struct DirectGroup {
 
 template <int FM, int FN, int WM, int WN, int WK, int ST, bool VA, bool VB>
 __global__ __launch_bounds__(256) void k_direct_grouped(DirectGroup G) {
+    __shared__ __attribute__((aligned(16))) char lds[direct_lds(FM, FN, WM, WN, WK)];
     int p = 0;
     while (p + 1 < G.n && blockIdx.x >= G.first[p + 1]) ++p;
-    direct_tile<FM, FN, WM, WN, WK, ST, VA, VB>(G.p[p], blockIdx.x - G.first[p]);
+    direct_tile<FM, FN, WM, WN, WK, ST, VA, VB>(G.p[p], blockIdx.x - G.first[p], lds);
 }
 
 struct DirCfg {
@@ -417,13 +424,16 @@ struct Pick {
     double us = 1e300;
 };
 
-static Pick pick_shape(const DirectArgs& a) {
+// stage: one of a level's problems (square tiles only; partial tiles are added by
+// the assembly, so a split costs no launch of its own).
+static Pick pick_shape(const DirectArgs& a, bool stage = false) {
     constexpr double kL1 = 286.0, kLatency = 1033.0, kStart = 2337.0, kBlock = 258.0, kChip = 5534.0;
     constexpr double kLaunch = 1.5, kSplit = 2.6, kSplitBytes = 3509.0, kPerSplit = 0.06, kGHz = 2400.0;
     Pick best;
     const double chunks = std::ceil(a.K / 16.0);
     for (int c = 0; c < kNDirCfg; ++c) {
         const DirCfg& f = kDirCfg[c];
+        if (stage && c != 0 && c != 1 && c != 3) continue;
         const double tiles = double((a.M + f.tm() - 1) / f.tm()) * double((a.N + f.tn() - 1) / f.tn()) * a.batch;
         for (uint32_t s = 1; s <= 128; s *= 2) {
             if (s > 1 && (chunks / s < f.wk || tiles * s > 16384)) break;
@@ -434,11 +444,144 @@ static Pick pick_shape(const DirectArgs& a) {
             const double queued = std::ceil(blocks / 256.0) * (per_wave * busy + kBlock);
             const double fed = (f.tm() + f.tn()) * 128.0 * f.wk * per_wave * blocks / kChip;
             double t = kLaunch + std::max({alone, queued, fed}) / kGHz;
-            if (s > 1) t += kSplit + tiles * f.tm() * f.tn() * 8.0 * (2 * s + 1) / kSplitBytes / kGHz + s * kPerSplit;
+            if (s > 1) t += (stage ? 0.3 : kSplit) + tiles * f.tm() * f.tn() * 8.0 * (2 * s + 1) / kSplitBytes / kGHz + s * kPerSplit;
             if (t < best.us) best = {c, s, t};
         }
     }
     return best;
+}
+
+// ------------------------------------------------------- batched stages
+//
+// One launch over the tiles of many independent contractions (of one job, or
+// of several jobs' stages merged): block -> (job, problem, tile).  The problem
+// descriptors are in device memory, built once per solver; every tile goes to
+// its problem's partial buffer and k_assemble forms the tensors from them.
+// Bound by latency at the sizes it serves (a block runs a few us, most of it
+// waiting for its first operands), so what counts is that all products of a
+// level run side by side and that a stage is 8 launches instead of 57.
+struct StageGroup {
+    const DirectArgs* prob[kDirGroup];
+    const uint32_t* first[kDirGroup];   // block offsets of each job's problems (np + 1)
+    uint32_t np[kDirGroup];
+    uint32_t start[kDirGroup + 1];
+    int n;
+};
+
+template <int FM, int FN, int WM, int WN, int WK, int ST>
+__device__ __forceinline__ void stage_tile(const DirectArgs& g, uint32_t bid, char* lds) {
+    switch (g.config & 3) {
+        case 0: direct_tile<FM, FN, WM, WN, WK, ST, false, false, true>(g, bid, lds); break;
+        case 1: direct_tile<FM, FN, WM, WN, WK, ST, true, false, true>(g, bid, lds); break;
+        case 2: direct_tile<FM, FN, WM, WN, WK, ST, false, true, true>(g, bid, lds); break;
+        default: direct_tile<FM, FN, WM, WN, WK, ST, true, true, true>(g, bid, lds); break;
+    }
+}
+
+__global__ __launch_bounds__(256) void k_stage(StageGroup G) {
+    __shared__ __attribute__((aligned(16))) char lds[direct_lds(2, 2, 1, 1, 4)];   // the largest of the shapes
+    int j = 0;
+    while (j + 1 < G.n && blockIdx.x >= G.start[j + 1]) ++j;
+    const uint32_t bid = blockIdx.x - G.start[j];
+    const uint32_t* first = G.first[j];
+    uint32_t p = 0;
+    while (p + 1 < G.np[j] && bid >= first[p + 1]) ++p;
+    const DirectArgs& g = G.prob[j][p];
+    switch (g.config >> 2) {
+        case 0: stage_tile<1, 1, 1, 1, 4, 4>(g, bid - first[p], lds); break;
+        case 1: stage_tile<2, 2, 1, 1, 4, 3>(g, bid - first[p], lds); break;
+        default: stage_tile<2, 2, 2, 2, 1, 3>(g, bid - first[p], lds); break;
+    }
+}
+
+void launch_stage(const StageLevel* const* l, int n, hipStream_t s) {
+    AQ_CHECK(n >= 1 && n <= kDirGroup, AQ_ERR_INVALID, "stage group size");
+    StageGroup G{};
+    G.n = n;
+    for (int i = 0; i < n; ++i) {
+        G.prob[i] = l[i]->prob;
+        G.first[i] = l[i]->first;
+        G.np[i] = l[i]->np;
+        G.start[i + 1] = G.start[i] + l[i]->blocks;
+    }
+    hipLaunchKernelGGL(k_stage, dim3(G.start[n]), dim3(256), 0, s, G);
+    AQ_HIP(hipGetLastError());
+}
+
+// Value of a term at digits d (of the output's dimensions): a strided tensor
+// element; a tile element of a product at its row and column index; or one of
+// the packed-pair products S+ / S- (symmetric / antisymmetric under exchange of
+// the pair (d0,d1), and of (d2,d3)).
+__device__ __forceinline__ double term_value(const AsmTerm& t, const uint32_t (&d)[4]) {
+    uint32_t m = d[0] * t.s0[0] + d[1] * t.s0[1] + d[2] * t.s0[2] + d[3] * t.s0[3];
+    if (t.kind == 0) return t.coef * t.p[m];
+    uint32_t n = d[0] * t.s1[0] + d[1] * t.s1[1] + d[2] * t.s1[2] + d[3] * t.s1[3];
+    double sign = t.coef;
+    if (t.kind >= 2) {
+        const uint32_t a = min(d[0], d[1]), b = max(d[0], d[1]), i = min(d[2], d[3]), j = max(d[2], d[3]);
+        if (t.kind == 2) {
+            m = a + b * (b + 1) / 2;
+            n = i + j * (j + 1) / 2;
+        } else {
+            if (a == b || i == j) return 0.0;
+            m = a + b * (b - 1) / 2;
+            n = i + j * (j - 1) / 2;
+            if ((d[0] < d[1]) != (d[2] < d[3])) sign = -sign;
+        }
+    }
+    const uint32_t tile = (m >> t.ltm) + t.tilesM * (n >> t.ltn);
+    const uint32_t e = ((n & ((1u << t.ltn) - 1)) << t.ltm) + (m & ((1u << t.ltm) - 1));
+    const double* p = t.p + ((uint64_t(tile) * t.nsplit) << (t.ltm + t.ltn)) + e;
+    double v = p[0];
+    for (uint32_t s = 1; s < t.nsplit; ++s) v += p[uint64_t(s) << (t.ltm + t.ltn)];
+    return sign * v;
+}
+
+// out[d] = sum of the terms at d, plus, where the output is symmetrised, the
+// same sum at (d1, d0, d3, d2).  One thread per element, first dimension
+// fastest; block -> output by prefix.
+__global__ __launch_bounds__(256) void k_assemble(const AsmOut* __restrict__ outs, const AsmTerm* __restrict__ terms,
+                                                  int nout) {
+    int o = 0;
+    while (o + 1 < nout && blockIdx.x >= outs[o + 1].first) ++o;
+    const AsmOut& q = outs[o];
+    const uint32_t x = (blockIdx.x - q.first) * 256 + threadIdx.x;
+    if (x >= q.n) return;
+    uint32_t d[4], r = x;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const uint32_t c = r / q.len[k];
+        d[k] = r - c * q.len[k];
+        r = c;
+    }
+    d[3] = r;
+    const uint32_t e[4] = {d[1], d[0], d[3], d[2]};
+    double v = 0.0, w = 0.0;
+    for (uint32_t k = 0; k < q.nterms; ++k) {
+        const AsmTerm& t = terms[q.term + k];
+        v += term_value(t, d);
+        if (q.sym) w += term_value(t, e);
+    }
+    q.out[x] = q.sym ? v + w : v;
+}
+
+void launch_assemble(hipStream_t s, const AsmOut* outs, const AsmTerm* terms, int nout, uint32_t blocks) {
+    hipLaunchKernelGGL(k_assemble, dim3(blocks), dim3(256), 0, s, outs, terms, nout);
+    AQ_HIP(hipGetLastError());
+}
+
+void plan_stage_problem(DirectArgs& a) {
+    const Pick p = pick_shape(a, true);
+    const DirCfg& f = kDirCfg[p.cfg];
+    a.tilesM = (a.M + f.tm() - 1) / f.tm();
+    a.tilesN = (a.N + f.tn() - 1) / f.tn();
+    a.kchunk = ((a.K + 15) / 16 + p.nsplit - 1) / p.nsplit * 16;
+    a.nsplit = (a.K + a.kchunk - 1) / a.kchunk;
+    for (DirDigits* d : {&a.m, &a.n, &a.k}) set_dividers(*d);
+    const uint32_t shape = p.cfg == 3 ? 2 : uint32_t(p.cfg);   // k_stage's shapes: 16, 32, 64
+    a.config = shape * 4 + (k_runs(a.k, a.k.s0) ? 1 : 0) + (k_runs(a.k, a.k.s1) ? 2 : 0);
+    a.tm = uint32_t(f.tm());
+    a.tn = uint32_t(f.tn());
 }
 
 bool direct_contract(aq_ctx* ctx, DirectArgs a) {

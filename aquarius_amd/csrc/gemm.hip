@@ -1041,7 +1041,8 @@ namespace {
 
 // One kernel: a GEMM instantiation, or (fmt = kDirectKey, ta = its config) a
 // direct contraction's.
-constexpr int kDirectKey = -1;
+// kStageKey, ta = level: a level of a batched stage.
+constexpr int kDirectKey = -1, kStageKey = -2;
 struct GroupKey {
     int fmt, ta, tb, bm, bn;
     bool operator==(const GroupKey& o) const {
@@ -1101,6 +1102,7 @@ struct GemmBatcher {
         GroupKey key;
         const GemmArgs* a;                // the submitter's, which waits until the launch
         const DirectArgs* d;              // or a direct contraction's
+        const StageLevel* l;              // or a stage level
         int64_t blocks;
         hipEvent_t ready;                 // the member's operands are written
         Launch* launch = nullptr;
@@ -1154,6 +1156,10 @@ static void launch_group(GemmBatcher* b, const GroupKey& key) {
             const DirectArgs* d[kMaxGroup];
             for (int i = 0; i < G.n; ++i) d[i] = take[size_t(i)]->d;
             launch_direct_group(key.ta, d, G.n, b->stream);
+        } else if (key.fmt == kStageKey) {
+            const StageLevel* l[kMaxGroup];
+            for (int i = 0; i < G.n; ++i) l[i] = take[size_t(i)]->l;
+            launch_stage(l, G.n, b->stream);
         } else {
             launch_grouped(key, G, blocks, b->stream, b->cus);
         }
@@ -1181,11 +1187,12 @@ static void launch_group(GemmBatcher* b, const GroupKey& key) {
 // partner).  Returns true once it ran in a grouped launch (ctx->stream is
 // then ordered after it), false when it found no partner: the caller launches
 // it alone on its own stream, exactly as without grouping.
-static bool batcher_submit(aq_ctx* ctx, const GroupKey& key, const GemmArgs* a, const DirectArgs* d, int64_t blocks) {
+static bool batcher_submit(aq_ctx* ctx, const GroupKey& key, const GemmArgs* a, const DirectArgs* d, const StageLevel* l,
+                           int64_t blocks) {
     GemmBatcher* b = ctx->batcher;
     if (!ctx->group_ready) AQ_HIP(hipEventCreateWithFlags(&ctx->group_ready, hipEventDisableTiming));
     AQ_HIP(hipEventRecord(ctx->group_ready, ctx->stream));
-    GemmBatcher::Item item{key, a, d, blocks, ctx->group_ready};
+    GemmBatcher::Item item{key, a, d, l, blocks, ctx->group_ready};
     std::unique_lock<std::mutex> lk(b->mu);
     b->pending.push_back(&item);
     struct Unlist {   // an item still pending when this frame unwinds is withdrawn (mu held)
@@ -1230,7 +1237,11 @@ static bool batcher_submit(aq_ctx* ctx, const GroupKey& key, const GemmArgs* a, 
 }
 
 bool batcher_offer_direct(aq_ctx* ctx, int config, const DirectArgs& a, int64_t blocks) {
-    return batcher_submit(ctx, GroupKey{kDirectKey, config, 0, 0, 0}, nullptr, &a, blocks);
+    return batcher_submit(ctx, GroupKey{kDirectKey, config, 0, 0, 0}, nullptr, &a, nullptr, blocks);
+}
+
+bool batcher_offer_stage(aq_ctx* ctx, int level, const StageLevel& l) {
+    return batcher_submit(ctx, GroupKey{kStageKey, level, 0, 0, 0}, nullptr, nullptr, &l, l.blocks);
 }
 
 GemmBatcher* batcher_create(int device, int window_us) {
@@ -1389,7 +1400,7 @@ void gemm(aq_ctx* ctx, const GemmDesc& d) {
             part.reset(new Scratch(ctx, size_t(nsplit) * d.batch * d.M * d.N * partial_bytes(d.fmt)));
             a.P = part->p;
         }
-        if (batcher_submit(ctx, GroupKey{int(d.fmt), d.transA ? 1 : 0, d.transB ? 1 : 0, BM, BN}, &a, nullptr,
+        if (batcher_submit(ctx, GroupKey{int(d.fmt), d.transA ? 1 : 0, d.transB ? 1 : 0, BM, BN}, &a, nullptr, nullptr,
                            base_tiles * d.batch * nsplit)) {
             if (nsplit > 1)
                 launch_reduce_splitk(ctx, a.P, d.fmt != FMT_F64, nsplit, d.M, d.N, d.batch, d.alpha, d.beta, d.C, d.ldc,

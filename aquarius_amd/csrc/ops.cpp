@@ -460,6 +460,48 @@ static bool run_direct(aq_ctx* ctx, double alpha, const Labeled& A, const Labele
     return direct_contract(ctx, a);
 }
 
+bool plan_product(const aq_tensor* tA, const char* ia, const aq_tensor* tB, const char* ib, const char* ic,
+                  DirectArgs& a, uint32_t* mulM, uint32_t* mulN) {
+    const Labeled A = label(tA, ia, "A"), B = label(tB, ib, "B");
+    const std::string cl(ic);
+    for (char c : A.lab + B.lab) label_len({&A, &B}, c);
+    const Labeled C = packed(nullptr, cl, lens_of(cl, {&A, &B}));
+    constexpr int64_t kMost = int64_t(1) << 28;
+    if (A.has_repeat || B.has_repeat || A.size() >= kMost || B.size() >= kMost || C.size() >= kMost) return false;
+    const std::string Ml = filter(A.lab, B.lab, false, cl, true), Nl = filter(B.lab, A.lab, false, cl, true);
+    const std::string Kl = filter(A.lab, B.lab, true, cl, false);
+    if (Ml.size() + Nl.size() != cl.size() || Ml.size() + Kl.size() != A.lab.size() || Nl.size() + Kl.size() != B.lab.size())
+        return false;
+    const bool swap = Nl.find(cl[0]) != std::string::npos;   // rows hold the first output label
+    const Labeled &X = swap ? B : A, &Y = swap ? A : B;
+    const std::string &Rl = swap ? Nl : Ml, &Cl = swap ? Ml : Nl;
+    const char ux = unit_label(X), uy = unit_label(Y);
+    auto has = [](const std::string& labs, char c) { return c && labs.find(c) != std::string::npos; };
+    const std::string ro = order_as(Rl, has(Rl, ux) ? X : C), co = order_as(Cl, has(Cl, uy) ? Y : C);
+    a = DirectArgs{};
+    if (!digits_of(ro, X, C, a.m) || !digits_of(co, Y, C, a.n) || !digits_of(order_as(Kl, has(Kl, ux) ? X : Y), X, Y, a.k))
+        return false;
+    auto multipliers = [&](const std::string& order, uint32_t* mul) {
+        for (size_t k = 0; k < cl.size(); ++k) mul[k] = 0;
+        uint32_t s = 1;
+        for (char c : order) {
+            const size_t k = cl.find(c);
+            mul[k] = s;
+            s *= uint32_t(C.len[k]);
+        }
+    };
+    multipliers(ro, mulM);
+    multipliers(co, mulN);
+    a.M = uint32_t(prod_len(Rl, X));
+    a.N = uint32_t(prod_len(Cl, Y));
+    a.K = uint32_t(prod_len(Kl, X));
+    a.batch = 1;
+    a.A = X.data;
+    a.B = Y.data;
+    a.alpha = 1.0;
+    return true;
+}
+
 static void contract_impl(aq_ctx* ctx, double alpha, const aq_tensor* tA, const char* ia, const aq_tensor* tB,
                           const char* ib, double beta, aq_tensor* tC, const char* ic) {
     Labeled A0 = label(tA, ia, "A"), B0 = label(tB, ib, "B"), C0 = label(tC, ic, "C");

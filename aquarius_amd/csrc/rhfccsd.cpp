@@ -27,6 +27,7 @@ using aqamd::tensor::Tensor;
 using aqamd::tensor::scalar;
 
 #include "diis.hpp"
+#include "stage.hpp"
 
 
 using namespace aqamd;
@@ -131,6 +132,7 @@ struct aq_rhfccsd {
     // The ladder can run on the (anti)symmetric packed forms when
     // <ab|ef> = <ba|fe> and <ab|ij> = <ba|ji> (so Tau(ef,ij) = Tau(fe,ji)).
     void derive_packed() {
+        program.reset();   // holds addresses of the packed operators
         packed = false;
         if (cfg.packed_ladder && o >= 2 && v >= 2) {
             launch_pair_asymmetry(ctx, dptr(VABCD), v, v, 0);
@@ -213,9 +215,159 @@ struct aq_rhfccsd {
         diis.reset(new DIIS(ctx, cfg.diis_order, cfg.diis_start, cfg.diis_damping, 2, 2));   // :98
     }
 
+    // The contraction stage of a small system as a program of batched launches:
+    // the same products as contractions(), those that depend on nothing but
+    // amplitudes and integrals side by side, then those that need the first
+    // intermediates, and so on; two products that several intermediates share
+    // ("efam,fi" and "nmei,an") are formed once.  A stage is 10 launches instead
+    // of 57.  Used while every product is FP64 arithmetic and the doubles have at
+    // most kBatchedDoubles elements, where launches and their latency dominate.
+    static constexpr double kBatchedDoubles = 1.2e6;
+    std::unique_ptr<StageProgram> program;
+    bool program_refused = false;
+
+    bool batched(int prec) {
+        if (double(o) * o * v * v > kBatchedDoubles || program_refused) return false;
+        if (!program) {
+            if (ctx->capture) return false;   // built on an eager iteration
+            build_program();
+            if (!program) return false;
+        }
+        return prec == AQ_PREC_FP64 || program->largest_flops() < cfg.min_reduced_flops;
+    }
+
+    void build_program() {
+        std::unique_ptr<StageProgram> p(new StageProgram(ctx));
+        StageProgram& P = *p;
+        enum { kFirst, kSecond, kThird };
+        // from amplitudes and integrals
+        const int fme = P.product(kFirst, VABIJSA, "efmn", T1, "fn", "me");
+        const int fmi1 = P.product(kFirst, VABIJSA, "efmn", T2, "efin", "mi");
+        const int fmi2 = P.product(kFirst, VAIJK, "finm", T1, "fn", "mi");
+        const int fmi3 = P.product(kFirst, VAIJK, "fimn", T1, "fn", "mi");
+        const int fae1 = P.product(kFirst, VABIJSA, "efmn", T2, "afmn", "ae");
+        const int fae2 = P.product(kFirst, VABCI, "efam", T1, "fm", "ae");
+        const int fae3 = P.product(kFirst, VABCI, "feam", T1, "fm", "ae");
+        const int w1 = P.product(kFirst, VABIJ, "efmn", Tau, "efij", "mnij");
+        const int w2 = P.product(kFirst, VAIJK, "ejmn", T1, "ei", "mnij");
+        const int wmnej = P.product(kFirst, VABIJ, "efmn", T1, "fj", "mnej");
+        const int wamij1 = P.product(kFirst, VABCI, "efam", Tau, "efij", "amij");
+        const int wamij2 = P.product(kFirst, VAIBJ, "amej", T1, "ei", "amij");
+        const int wamij3 = P.product(kFirst, VAIJB, "amie", T1, "ej", "amij");
+        const int wamie1 = P.product(kFirst, VABIJSA, "efmn", T2SA, "afin", "amie");
+        const int it1 = P.product(kFirst, VABCI, "feam", T1, "fi", "amie");
+        const int it2 = P.product(kFirst, VABCI, "efam", T1, "fi", "amie");
+        const int wamei1 = P.product(kFirst, VABIJ, "efnm", T2, "afni", "amei");
+        const int z11 = P.product(kFirst, fAB, "ae", T1, "ei", "ai");
+        const int z12 = P.product(kFirst, VAIJBSA, "amie", T1, "em", "ai");
+        const int z13 = P.product(kFirst, VABCI, "efam", TauSA, "efim", "ai");
+        const int z21 = P.product(kFirst, VABCI, "abej", T1, "ei", "abij");
+        const int sp = packed ? P.product(kFirst, Vp, "pq", Tp, "iq", "pi") : -1;
+        const int sm = packed ? P.product(kFirst, Vm, "pq", Tm, "iq", "pi") : -1;
+        const int lad = packed ? -1 : P.product(kFirst, VABCD, "abef", Tau, "efij", "abij");
+        P.output(kFirst, FME, "me");
+        P.add(1.0, fAI, "em");                    // :244
+        P.add(1.0, fme);                          // :245
+        P.output(kFirst, WMNIJ, "mnij", true);    // :262
+        P.add(0.5, VIJKL, "mnij");                // :259
+        P.add(0.5, w1);                           // :260
+        P.add(1.0, w2);                           // :261
+        P.output(kFirst, WMNEJ, "mnej");
+        P.add(1.0, VAIJK, "ejmn");                // :264
+        P.add(1.0, wmnej);                        // :265
+        P.output(kFirst, WAMIJ, "amij");
+        P.add(1.0, VAIJK, "amij");                // :267
+        P.add(1.0, wamij1);                       // :268
+        P.add(1.0, wamij2);                       // :269
+        P.add(1.0, wamij3);                       // :270
+        // with FME, WMNIJ, WMNEJ, WAMIJ
+        const int fmi4 = P.product(kSecond, FME, "me", T1, "ei", "mi");
+        const int fae4 = P.product(kSecond, FME, "me", T1, "am", "ae");
+        const int wt1 = P.product(kSecond, WMNEJ, "mnei", T1, "an", "amie");
+        const int wt2 = P.product(kSecond, WMNEJ, "nmei", T1, "an", "amie");
+        const int z14 = P.product(kSecond, FME, "me", T2SA, "aeim", "ai");
+        const int z15 = P.product(kSecond, WMNEJ, "mnei", T2SA, "eamn", "ai");
+        const int z22 = P.product(kSecond, WAMIJ, "amij", T1, "bm", "abij");
+        const int z25 = P.product(kSecond, WMNIJ, "mnij", Tau, "abmn", "abij");
+        P.output(kSecond, FMI, "mi");
+        P.add(1.0, fIJ, "mi");                    // :247
+        P.add(1.0, fmi1);                         // :248
+        P.add(1.0, fmi4);                         // :249
+        P.add(2.0, fmi2);                         // :250
+        P.add(-1.0, fmi3);                        // :251
+        P.output(kSecond, FAE, "ae");
+        P.add(1.0, fAB, "ae");                    // :253
+        P.add(-1.0, fae1);                        // :254
+        P.add(-1.0, fae4);                        // :255
+        P.add(2.0, fae2);                         // :256
+        P.add(-1.0, fae3);                        // :257
+        P.output(kSecond, WAMIE, "amie");
+        P.add(1.0, VAIJBSA, "amie");              // :272
+        P.add(0.5, wamie1);                       // :273
+        P.add(2.0, it1);                          // :274
+        P.add(-1.0, it2);                         // :275
+        P.add(-2.0, wt1);                         // :276
+        P.add(1.0, wt2);                          // :277
+        P.output(kSecond, WAMEI, "amei");
+        P.add(1.0, VAIBJ, "amei");                // :279
+        P.add(-0.5, wamei1);                      // :280
+        P.add(1.0, it2);                          // :281
+        P.add(-1.0, wt2);                         // :282
+        // with FMI, FAE, WAMIE, WAMEI
+        const int z16 = P.product(kThird, FMI, "mi", T1, "am", "ai");
+        const int z23 = P.product(kThird, FAE, "ae", T2, "ebij", "abij");
+        const int z24 = P.product(kThird, FMI, "mi", T2, "abmj", "abij");
+        const int z26 = P.product(kThird, WAMIE, "amie", T2SA, "ebmj", "abij");
+        const int z27 = P.product(kThird, WAMEI, "amei", T2, "ebjm", "abij");
+        const int z28 = P.product(kThird, WAMEI, "amej", T2, "ebim", "abij");
+        P.output(kThird, Z1, "ai");
+        P.add(1.0, fAI, "ai");                    // :290
+        P.add(1.0, z11);                          // :291
+        P.add(-1.0, z16);                         // :292
+        P.add(1.0, z12);                          // :293
+        P.add(1.0, z14);                          // :294
+        P.add(1.0, z13);                          // :295
+        P.add(-1.0, z15);                         // :296
+        P.output(kThird, Z2, "abij", true);       // :309
+        P.add(0.5, VABIJ, "abij");                // :298
+        P.add(1.0, z21);                          // :299
+        P.add(-1.0, z22);                         // :300
+        P.add(1.0, z23);                          // :301
+        P.add(-1.0, z24);                         // :302
+        if (packed) {                             // :303  0.5 (S+ + S-)
+            P.add_pairs(0.5, sp, false);
+            P.add_pairs(0.5, sm, true);
+        } else {
+            P.add(0.5, lad);
+        }
+        P.add(0.5, z25);                          // :304
+        P.add(0.5, z26);                          // :305
+        P.add(-0.5, z27);                         // :306
+        P.add(-1.0, z28);                         // :307
+        program_refused = !P.ok();
+        if (program_refused) return;
+        P.finish();
+        program = std::move(p);
+    }
+
+    void batched_contractions() {
+        launch_tau_sa(ctx, dptr(T1), dptr(T2), v, o, dptr(Tau), dptr(TauSA), dptr(T2SA));   // :231-238
+        for (const Tensor* t : {&Tau, &TauSA, &T2SA}) bump_t(*t);
+        if (packed) {
+            launch_ladder_pack_t(ctx, dptr(Tau), v, o, dptr(Tp), dptr(Tm));
+            bump_t(Tp);
+            bump_t(Tm);
+        }
+        program->run();
+    }
+
     // The contraction stage of one iteration (rhfccsd.cxx:231-309): every
     // operation is stream-ordered and none synchronises with the host.
-    void contractions() {
+    void contractions(int prec) {
+        if (batched(prec)) {
+            batched_contractions();
+            return;
+        }
         // :231-238 in one pass over T2, rounded as the six operator calls
         //   Tau["abij"] = T2["abij"];  Tau["abij"] += T1["ai"] * T1["bj"];
         //   TauSA["abij"] = 2 * Tau["abij"];  TauSA["abij"] -= Tau["abji"];
@@ -342,7 +494,7 @@ struct aq_rhfccsd {
         ctx->capture = &log;
         bool ok = true;
         try {
-            contractions();
+            contractions(prec);
         } catch (...) {
             ok = false;
         }
@@ -383,7 +535,7 @@ struct aq_rhfccsd {
         if (want && graph.warm_prec == prec && capture_stage(prec)) return;
         {
             StageMark mark(ctx->batcher);
-            contractions();
+            contractions(prec);
         }
         graph.warm_prec = prec;
     }

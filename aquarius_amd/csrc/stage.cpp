@@ -1,0 +1,164 @@
+// StageProgram: see stage.hpp; the kernels are in direct.hip.
+#include "stage.hpp"
+
+#include <algorithm>
+#include <cstring>
+#include <numeric>
+
+namespace aqamd {
+
+int StageProgram::product(int level, const tensor::Tensor& A, const char* ia, const tensor::Tensor& B, const char* ib,
+                          const char* ic) {
+    Product p;
+    p.level = level;
+    p.ic = ic;
+    ok_ = ok_ && p.ic.size() <= 4 && plan_product(A.handle(), ia, B.handle(), ib, ic, p.a, p.mulM, p.mulN);
+    largest_ = std::max(largest_, 2.0 * double(p.a.M) * double(p.a.N) * double(p.a.K));
+    products_.push_back(p);
+    return int(products_.size()) - 1;
+}
+
+void StageProgram::output(int level, const tensor::Tensor& out, const char* ic, bool sym) {
+    outputs_.push_back({level, &out, ic, sym, {}});
+}
+void StageProgram::add(double coef, const tensor::Tensor& X, const char* ix) {
+    outputs_.back().terms.push_back({coef, &X, ix, -1, 0});
+}
+void StageProgram::add(double coef, int product) { outputs_.back().terms.push_back({coef, nullptr, "", product, 1}); }
+void StageProgram::add_pairs(double coef, int product, bool antisymmetric) {
+    outputs_.back().terms.push_back({coef, nullptr, "", product, antisymmetric ? 3 : 2});
+}
+
+static uint32_t log2_of(uint32_t x) {
+    uint32_t l = 0;
+    while ((1u << l) < x) ++l;
+    return l;
+}
+
+void StageProgram::finish() {
+    AQ_CHECK(ok_, AQ_ERR_UNSUPPORTED, "contraction not of the batched stage's form");
+    int nlevels = 0;
+    for (const auto& p : products_) nlevels = std::max(nlevels, p.level + 1);
+    levels_.assign(size_t(nlevels), Level{});
+
+    // tiles of every product, one buffer; a level's long blocks come first
+    int64_t total = 0;
+    std::vector<int64_t> at;
+    for (auto& p : products_) {
+        plan_stage_problem(p.a);
+        at.push_back(total);
+        total += int64_t(p.a.tilesM) * p.a.tilesN * p.a.nsplit * p.a.tm * p.a.tn;
+    }
+    tiles_ = tensor::Tensor(ctx_, std::vector<int64_t>{std::max<int64_t>(total, 1)}, false);
+    for (size_t k = 0; k < products_.size(); ++k) products_[k].a.P = tiles_.handle()->data + at[k];
+
+    std::vector<char> host;
+    auto place = [&](const void* src, size_t bytes) {
+        const size_t off = (host.size() + 15) / 16 * 16;
+        host.resize(off + bytes);
+        std::memcpy(host.data() + off, src, bytes);
+        return off;
+    };
+    struct Offsets { size_t prob, first, outs, terms; };
+    std::vector<Offsets> offs(static_cast<size_t>(nlevels));
+    for (int l = 0; l < nlevels; ++l) {
+        Level& L = levels_[size_t(l)];
+        std::vector<const Product*> ps;
+        for (const auto& p : products_)
+            if (p.level == l) ps.push_back(&p);
+        std::stable_sort(ps.begin(), ps.end(), [](const Product* x, const Product* y) {
+            auto block = [](const DirectArgs& a) { return double(a.kchunk) * a.tm * a.tn; };
+            return block(x->a) > block(y->a);
+        });
+        std::vector<DirectArgs> args;
+        std::vector<uint32_t> first{0};
+        for (const auto* p : ps) {
+            args.push_back(p->a);
+            first.push_back(first.back() + p->a.tilesM * p->a.tilesN * p->a.nsplit);
+            L.flops += 2.0 * double(p->a.M) * p->a.N * p->a.K;
+            L.bytes += 8.0 * (double(p->a.M) + p->a.N) * p->a.K;
+        }
+        L.s.np = uint32_t(args.size());
+        L.s.blocks = first.back();
+        std::vector<AsmOut> outs;
+        std::vector<AsmTerm> terms;
+        for (const auto& o : outputs_) {
+            if (o.level != l) continue;
+            AsmOut q{};
+            const aq_tensor* t = o.t->handle();
+            q.out = t->data;
+            q.n = uint32_t(t->size);
+            for (int k = 0; k < 4; ++k) q.len[k] = k < t->ndim ? uint32_t(t->len[size_t(k)]) : 1u;
+            q.first = L.blocks;
+            q.term = uint32_t(terms.size());
+            q.nterms = uint32_t(o.terms.size());
+            q.sym = o.sym ? 1 : 0;
+            L.blocks += (q.n + 255) / 256;
+            outs.push_back(q);
+            written_.push_back(o.t);
+            for (const auto& tm : o.terms) {
+                AsmTerm d{};
+                d.coef = tm.coef;
+                d.kind = uint32_t(tm.kind);
+                if (tm.kind == 0) {
+                    const aq_tensor* x = tm.t->handle();
+                    d.p = x->data;
+                    uint32_t s = 1;
+                    for (size_t k = 0; k < tm.ix.size(); ++k) {
+                        d.s0[o.ic.find(tm.ix[k])] = s;
+                        s *= uint32_t(x->len[k]);
+                    }
+                } else {
+                    const Product& p = products_[size_t(tm.product)];
+                    d.p = p.a.P;
+                    d.ltm = log2_of(p.a.tm);
+                    d.ltn = log2_of(p.a.tn);
+                    d.tilesM = p.a.tilesM;
+                    d.nsplit = p.a.nsplit;
+                    if (tm.kind == 1)
+                        for (size_t k = 0; k < p.ic.size(); ++k) {
+                            d.s0[o.ic.find(p.ic[k])] = p.mulM[k];
+                            d.s1[o.ic.find(p.ic[k])] = p.mulN[k];
+                        }
+                }
+                terms.push_back(d);
+            }
+        }
+        L.nout = int(outs.size());
+        Offsets& f = offs[size_t(l)];
+        f.prob = place(args.data(), args.size() * sizeof(DirectArgs));
+        f.first = place(first.data(), first.size() * sizeof(uint32_t));
+        f.outs = place(outs.data(), outs.size() * sizeof(AsmOut));
+        f.terms = place(terms.data(), terms.size() * sizeof(AsmTerm));
+    }
+    desc_ = tensor::Tensor(ctx_, std::vector<int64_t>{int64_t(host.size() + 7) / 8}, false);
+    char* dev = reinterpret_cast<char*>(desc_.handle()->data);
+    AQ_HIP(hipMemcpyAsync(dev, host.data(), host.size(), hipMemcpyHostToDevice, ctx_->stream));
+    AQ_HIP(hipStreamSynchronize(ctx_->stream));
+    for (int l = 0; l < nlevels; ++l) {
+        Level& L = levels_[size_t(l)];
+        const Offsets& f = offs[size_t(l)];
+        L.s.prob = reinterpret_cast<const DirectArgs*>(dev + f.prob);
+        L.s.first = reinterpret_cast<const uint32_t*>(dev + f.first);
+        L.outs = reinterpret_cast<const AsmOut*>(dev + f.outs);
+        L.terms = reinterpret_cast<const AsmTerm*>(dev + f.terms);
+    }
+}
+
+void StageProgram::run() {
+    for (size_t l = 0; l < levels_.size(); ++l) {
+        const Level& L = levels_[l];
+        if (L.s.np && !(ctx_->batcher && !ctx_->capture && batcher_offer_stage(ctx_, int(l), L.s))) {
+            TimedLaunch tl(ctx_, "stage_contract", L.flops, L.bytes);
+            const StageLevel* one = &L.s;
+            launch_stage(&one, 1, ctx_->stream);
+        }
+        if (L.nout) {
+            TimedLaunch tl(ctx_, "stage_assemble", 0.0, 0.0);
+            launch_assemble(ctx_->stream, L.outs, L.terms, L.nout, L.blocks);
+        }
+    }
+    for (const auto* t : written_) t->handle()->version += 1;
+}
+
+}  // namespace aqamd
