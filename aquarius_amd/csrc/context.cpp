@@ -11,6 +11,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
 
 namespace aqamd {
 
@@ -20,21 +21,117 @@ void set_last_error(const std::string& msg) { g_last_error = msg; }
 
 size_t ctx_in_use(const aq_ctx* ctx) { return ctx->tensor_bytes + ctx->pool_bytes + ctx->cache_bytes; }
 
+// Blocks that a server's jobs have freed, kept for its next jobs.  The device
+// pool releases its free memory to the driver once that exceeds what is in use
+// (36 to 46 ms per release here, twice in a burst of eight small jobs), and
+// every job's end frees nearly all it had.  Safe across the slots' streams: a
+// block carries an event recorded behind its last use, and a request from
+// another stream waits for it.  Bounded: beyond `limit` the oldest blocks go
+// back; a failed allocation and the server's end give everything back.
+struct BlockCache {
+    struct Block {
+        void* p;
+        size_t bytes;
+        hipStream_t stream;
+        hipEvent_t freed;
+    };
+    std::mutex mu;
+    std::list<Block> kept;                           // oldest first
+    std::unordered_map<void*, size_t> given;         // blocks in use
+    std::vector<hipEvent_t> spare;
+    size_t bytes = 0, limit = 0;
+
+    void* take(size_t n, hipStream_t stream) {
+        std::lock_guard<std::mutex> lk(mu);
+        auto best = kept.end();
+        for (auto it = kept.begin(); it != kept.end(); ++it)   // at most an eighth wasted
+            if (it->bytes >= n && it->bytes - n <= n / 8 && (best == kept.end() || it->bytes < best->bytes)) best = it;
+        if (best == kept.end()) return nullptr;
+        if (best->stream != stream && hipStreamWaitEvent(stream, best->freed, 0) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        void* p = best->p;
+        given[p] = best->bytes;
+        bytes -= best->bytes;
+        spare.push_back(best->freed);
+        kept.erase(best);
+        return p;
+    }
+    void note(void* p, size_t n) {
+        std::lock_guard<std::mutex> lk(mu);
+        given[p] = n;
+    }
+    // false: not one of ours (the caller frees it)
+    bool give(void* p, hipStream_t stream) {
+        std::lock_guard<std::mutex> lk(mu);
+        auto it = given.find(p);
+        if (it == given.end()) return false;
+        Block b{p, it->second, stream, nullptr};
+        given.erase(it);
+        if (b.bytes > limit) return false;
+        if (!spare.empty()) {
+            b.freed = spare.back();
+            spare.pop_back();
+        } else if (hipEventCreateWithFlags(&b.freed, hipEventDisableTiming) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        if (hipEventRecord(b.freed, stream) != hipSuccess) {
+            (void)hipGetLastError();
+            spare.push_back(b.freed);
+            return false;
+        }
+        kept.push_back(b);
+        bytes += b.bytes;
+        while (bytes > limit) release_oldest(stream);
+        return true;
+    }
+    void release_oldest(hipStream_t stream) {        // mu held
+        const Block b = kept.front();
+        kept.pop_front();
+        bytes -= b.bytes;
+        // a wait that cannot be queued is made on the host
+        if (b.stream != stream && hipStreamWaitEvent(stream, b.freed, 0) != hipSuccess) (void)hipEventSynchronize(b.freed);
+        (void)hipFreeAsync(b.p, stream);
+        spare.push_back(b.freed);
+    }
+    void flush(hipStream_t stream) {
+        std::lock_guard<std::mutex> lk(mu);
+        while (!kept.empty()) release_oldest(stream);
+    }
+    ~BlockCache() {
+        flush(nullptr);
+        (void)hipStreamSynchronize(nullptr);
+        for (auto e : spare) (void)hipEventDestroy(e);
+    }
+};
+
+BlockCache* block_cache_create(size_t limit) {
+    auto* c = new BlockCache();
+    c->limit = limit;
+    return c;
+}
+void block_cache_destroy(BlockCache* c) { delete c; }
+
 // Stream-ordered device memory: allocations and frees are ordered on the
 // context's stream, so one context releasing memory never synchronises the
 // device under other contexts (concurrent serving).
 void* dmalloc(aq_ctx* ctx, size_t bytes) {
+    if (ctx->blocks)
+        if (void* p = ctx->blocks->take(bytes, ctx->stream)) return p;
     void* p = nullptr;
     if (hipMallocAsync(&p, bytes, ctx->stream) != hipSuccess) {
         (void)hipGetLastError();
         return nullptr;
     }
+    if (ctx->blocks) ctx->blocks->note(p, bytes);
     return p;
 }
 
 void dfree(aq_ctx* ctx, void* p) {
     if (p) {
-        (void)hipFreeAsync(p, ctx->stream);
+        if (!ctx->blocks || !ctx->blocks->give(p, ctx->stream)) (void)hipFreeAsync(p, ctx->stream);
         ctx->mem_gen += 1;
     }
 }
@@ -44,11 +141,11 @@ void dfree(aq_ctx* ctx, void* p) {
 // driver.  The pool keeps freed blocks between synchronisations (release
 // threshold at its maximum), which is what makes repeated allocation cheap
 // within a job; across jobs of different sizes those cached blocks can be
-// the wrong shapes for the next request, so they are trimmed when a job
-// ends and before an allocation is retried.
-static void trim_device_pool(aq_ctx* ctx) {
+// the wrong shapes for the next request, so they are trimmed before an
+// allocation is retried.
+void trim_device_pool(int device) {
     hipMemPool_t pool;
-    if (hipDeviceGetDefaultMemPool(&pool, ctx->device) == hipSuccess) (void)hipMemPoolTrimTo(pool, 0);
+    if (hipDeviceGetDefaultMemPool(&pool, device) == hipSuccess) (void)hipMemPoolTrimTo(pool, 0);
     (void)hipGetLastError();
 }
 
@@ -109,13 +206,15 @@ static void* raw_alloc(aq_ctx* ctx, size_t bytes) {
         // giving up any cached operand copy.
         const auto t0 = std::chrono::steady_clock::now();
         pool_release_all(ctx);
+        if (ctx->blocks) ctx->blocks->flush(ctx->stream);
         AQ_HIP(hipStreamSynchronize(ctx->stream));
-        trim_device_pool(ctx);
+        trim_device_pool(ctx->device);
         p = dmalloc(ctx, bytes);
         if (!p) {
             evict_cache(ctx, ctx->budget);   // drop every cached copy
+            if (ctx->blocks) ctx->blocks->flush(ctx->stream);
             AQ_HIP(hipStreamSynchronize(ctx->stream));
-            trim_device_pool(ctx);
+            trim_device_pool(ctx->device);
             p = dmalloc(ctx, bytes);
         }
         if (alloc_trace())
@@ -165,6 +264,16 @@ void tensor_free(aq_ctx* ctx, double* p, size_t bytes) {
 }
 
 void note_cache_alloc(aq_ctx* ctx) { note_peak(ctx); }
+
+// cached operand copies and pooled scratch back to the device pool
+void drop_caches(aq_ctx* ctx) {
+    pool_release_all(ctx);
+    for (auto& kv : ctx->cache) dfree(ctx, kv.second.ptr);
+    ctx->cache.clear();
+    ctx->cache_lru.clear();
+    ctx->cache_bytes = 0;
+}
+
 
 // ---------------------------------------------------------------- timing
 
@@ -350,13 +459,10 @@ int aq_ctx_trim(aq_ctx* ctx) {
     return guarded([&] {
         AQ_CHECK(ctx, AQ_ERR_INVALID, "null context");
         AQ_HIP(hipStreamSynchronize(ctx->stream));
-        pool_release_all(ctx);
-        for (auto& kv : ctx->cache) dfree(ctx, kv.second.ptr);
-        ctx->cache.clear();
-        ctx->cache_lru.clear();
-        ctx->cache_bytes = 0;
+        drop_caches(ctx);
+        if (ctx->blocks) return;   // a server's slot: for its next jobs
         AQ_HIP(hipStreamSynchronize(ctx->stream));
-        trim_device_pool(ctx);
+        trim_device_pool(ctx->device);
     });
 }
 

@@ -118,6 +118,7 @@ struct aq_tensor {
 
 namespace aqamd {
 struct GemmBatcher;
+struct BlockCache;
 }
 
 struct aq_ctx {
@@ -139,6 +140,9 @@ struct aq_ctx {
     std::unordered_map<std::string, aqamd::CacheEntry> cache;
     std::list<std::string> cache_lru;   // front = most recent
     size_t cache_bytes = 0;
+
+    // freed blocks shared with a server's other slots (null: the device pool's)
+    aqamd::BlockCache* blocks = nullptr;
 
     // reductions
     double* d_partials = nullptr;   // device: kRedSlots slots x kRedPartials partials
@@ -178,6 +182,12 @@ double* tensor_alloc(aq_ctx* ctx, size_t bytes);     // persistent (counted agai
 void tensor_free(aq_ctx* ctx, double* p, size_t bytes);
 size_t ctx_in_use(const aq_ctx* ctx);
 void evict_cache(aq_ctx* ctx, size_t need);
+void drop_caches(aq_ctx* ctx);                       // operand copies and pooled scratch back to the allocator
+void trim_device_pool(int device);                   // the device pool's unused memory back to the driver
+// a server's freed blocks, kept for its next jobs (at most `limit` bytes); its
+// contexts are destroyed before it
+BlockCache* block_cache_create(size_t limit);
+void block_cache_destroy(BlockCache* c);
 void invalidate_cache(aq_ctx* ctx);                  // every cached copy must be rebuilt before use
 void noalloc_scratch_init(int device);               // noalloc.cpp: resolve the fixed device array once per device
 

@@ -59,6 +59,7 @@ struct aq_server {
     std::vector<aq_ctx*> ctxs;
     GemmBatcher* batcher = nullptr;   // cross-job GEMM grouping (null: off)
     std::vector<std::thread> workers;
+    BlockCache* blocks = nullptr;     // memory kept between jobs
     std::mutex mu;
     std::condition_variable cv_work, cv_done;
     std::deque<int64_t> queue;
@@ -101,7 +102,9 @@ struct aq_server {
             if (mo) aq_tensor_destroy(mo);
             for (auto* t : ints)
                 if (t) aq_tensor_destroy(t);
-            aq_ctx_trim(ctx);
+            // the job's memory goes to the server's block cache, for the next job
+            (void)hipStreamSynchronize(ctx->stream);
+            drop_caches(ctx);
         };
         try {
             if (!job.inputs.empty()) {
@@ -253,10 +256,13 @@ int aq_server_create(int device, size_t hbm_budget, int slots, double max_bypass
             }
             size_t free_b = 0, total_b = 0;
             AQ_HIP(hipMemGetInfo(&free_b, &total_b));
+            s->blocks = block_cache_create(total_b / 8);
+            for (auto* c : s->ctxs) c->blocks = s->blocks;
             s->budget = hbm_budget ? std::min(hbm_budget, size_t(0.95 * double(free_b))) : size_t(0.9 * double(free_b));
             for (int i = 0; i < slots; ++i) s->workers.emplace_back([s, i] { s->worker(i); });
         } catch (...) {
             for (auto* c : s->ctxs) aq_ctx_destroy(c);
+            block_cache_destroy(s->blocks);
             delete s;
             throw;
         }
@@ -412,6 +418,8 @@ int aq_server_destroy(aq_server* s) {
         for (auto& t : s->workers) t.join();
         for (auto* c : s->ctxs) aq_ctx_destroy(c);
         batcher_destroy(s->batcher);
+        block_cache_destroy(s->blocks);   // what was kept between jobs goes back
+        trim_device_pool(s->device);
         delete s;
     });
 }
