@@ -27,6 +27,7 @@
 
 #include <algorithm>
 #include <cstdio>
+#include <vector>
 #include <cmath>
 
 namespace aqamd {
@@ -51,6 +52,13 @@ __device__ __forceinline__ uint32_t digit_offset(const DirDigits& d, const uint3
     return d.nd > 0 ? off + x * st[d.nd - 1] : 0u;
 }
 
+// block id -> work id: the dispatcher deals ids to the 8 XCDs round-robin; give
+// each XCD a contiguous run, whose tiles share operand rows in its L2
+__device__ __forceinline__ uint32_t xcd_order(uint32_t bid, uint32_t nb) {
+    const uint32_t full = nb / 8 * 8;
+    return bid >= full ? bid : (bid % 8) * (nb / 8) + bid / 8;
+}
+
 // LDS of a tile: the k tables, then (WK > 1) the waves' accumulators.
 constexpr int direct_lds(int fm, int fn, int wm, int wn, int wk) {
     const int red = wk > 1 ? wk * fm * fn * wm * wn * 256 * 8 : 0, tab = 2 * kKT * 4;
@@ -71,10 +79,13 @@ __device__ __forceinline__ void direct_tile(const DirectArgs& g, uint32_t bid, c
     const int wk = wave % WK, wm = (wave / WK) % WM, wn = wave / (WK * WM);
     const int l16 = lane & 15, q = lane >> 4;
 
-    // block -> (batch, tile, split), split fastest; tiles m fastest
-    const uint32_t split = bid % g.nsplit;
-    const uint32_t bt = bid / g.nsplit;
+    // work id -> (split, batch, tile), tiles fastest (m, then n): the run of ids
+    // that one XCD gets (xcd_order) then covers few splits of many tiles, so its
+    // L2 fetches a k range of the operands once for all of them (110 x
+    // 110 x 21560, 16 tiles of 16 splits: 32 us with the splits fastest, 24 so)
     const uint32_t tiles = g.tilesM * g.tilesN;
+    const uint32_t split = bid / (tiles * g.batch);
+    const uint32_t bt = bid % (tiles * g.batch);
     const uint32_t b = bt / tiles, tile = bt % tiles;
     const uint32_t m0 = (tile % g.tilesM) * TM, n0 = (tile / g.tilesM) * TN;
     const uint32_t kbeg = split * g.kchunk, kend = min(g.K, kbeg + g.kchunk);
@@ -299,13 +310,6 @@ __global__ __launch_bounds__(256) void k_direct_reduce(DirectArgs g, uint32_t tm
     *c = g.beta != 0.0 ? g.beta * *c + x : x;
 }
 
-// block id -> work id: the dispatcher deals ids to the 8 XCDs round-robin; give
-// each XCD a contiguous run, whose tiles share operand rows in its L2
-__device__ __forceinline__ uint32_t xcd_order(uint32_t bid, uint32_t nb) {
-    const uint32_t full = nb / 8 * 8;
-    return bid >= full ? bid : (bid % 8) * (nb / 8) + bid / 8;
-}
-
 template <int FM, int FN, int WM, int WN, int WK, int ST, bool VA, bool VB>
 __global__ __launch_bounds__(256) void k_direct(DirectArgs g) {
     __shared__ __attribute__((aligned(16))) char lds[direct_lds(FM, FN, WM, WN, WK)];
@@ -325,7 +329,7 @@ __global__ __launch_bounds__(256) void k_direct_grouped(DirectGroup G) {
     __shared__ __attribute__((aligned(16))) char lds[direct_lds(FM, FN, WM, WN, WK)];
     int p = 0;
     while (p + 1 < G.n && blockIdx.x >= G.first[p + 1]) ++p;
-    direct_tile<FM, FN, WM, WN, WK, ST, VA, VB>(G.p[p], blockIdx.x - G.first[p], lds);
+    direct_tile<FM, FN, WM, WN, WK, ST, VA, VB>(G.p[p], xcd_order(blockIdx.x - G.first[p], G.first[p + 1] - G.first[p]), lds);
 }
 
 struct DirCfg {
@@ -418,22 +422,20 @@ static bool k_runs(const DirDigits& k, const uint32_t* st) {
 // least the load latency over the chunks in flight; blocks queue on 256 CUs;
 // operand tiles come in at a rate of the whole chip; a split pays a second
 // launch and the traffic of the partial tiles.
+constexpr double kL1 = 286.0, kLatency = 1033.0, kStart = 2337.0, kBlock = 258.0, kChip = 5534.0;
+constexpr double kLaunch = 1.5, kSplit = 2.6, kSplitBytes = 3509.0, kPerSplit = 0.06, kGHz = 2400.0;
+
 struct Pick {
     int cfg = -1;
     uint32_t nsplit = 1;
     double us = 1e300;
 };
 
-// stage: one of a level's problems (square tiles only; partial tiles are added by
-// the assembly, so a split costs no launch of its own).
-static Pick pick_shape(const DirectArgs& a, bool stage = false) {
-    constexpr double kL1 = 286.0, kLatency = 1033.0, kStart = 2337.0, kBlock = 258.0, kChip = 5534.0;
-    constexpr double kLaunch = 1.5, kSplit = 2.6, kSplitBytes = 3509.0, kPerSplit = 0.06, kGHz = 2400.0;
+static Pick pick_shape(const DirectArgs& a) {
     Pick best;
     const double chunks = std::ceil(a.K / 16.0);
     for (int c = 0; c < kNDirCfg; ++c) {
         const DirCfg& f = kDirCfg[c];
-        if (stage && c != 0 && c != 1 && c != 3) continue;
         const double tiles = double((a.M + f.tm() - 1) / f.tm()) * double((a.N + f.tn() - 1) / f.tn()) * a.batch;
         for (uint32_t s = 1; s <= 128; s *= 2) {
             if (s > 1 && (chunks / s < f.wk || tiles * s > 16384)) break;
@@ -444,7 +446,7 @@ static Pick pick_shape(const DirectArgs& a, bool stage = false) {
             const double queued = std::ceil(blocks / 256.0) * (per_wave * busy + kBlock);
             const double fed = (f.tm() + f.tn()) * 128.0 * f.wk * per_wave * blocks / kChip;
             double t = kLaunch + std::max({alone, queued, fed}) / kGHz;
-            if (s > 1) t += (stage ? 0.3 : kSplit) + tiles * f.tm() * f.tn() * 8.0 * (2 * s + 1) / kSplitBytes / kGHz + s * kPerSplit;
+            if (s > 1) t += kSplit + tiles * f.tm() * f.tn() * 8.0 * (2 * s + 1) / kSplitBytes / kGHz + s * kPerSplit;
             if (t < best.us) best = {c, s, t};
         }
     }
@@ -478,19 +480,24 @@ __device__ __forceinline__ void stage_tile(const DirectArgs& g, uint32_t bid, ch
     }
 }
 
-__global__ __launch_bounds__(256) void k_stage(StageGroup G) {
+// Fewer chunks in flight than the single kernels, for three waves per SIMD: the
+// blocks of a level are short and mostly wait (o = 8, v = 43: 37 us a launch
+// with 4/3/3 chunks and two waves, 29 us with 3/2/2 and three).
+__global__ __launch_bounds__(256, 3) void k_stage(StageGroup G) {
     __shared__ __attribute__((aligned(16))) char lds[direct_lds(2, 2, 1, 1, 4)];   // the largest of the shapes
     int j = 0;
     while (j + 1 < G.n && blockIdx.x >= G.start[j + 1]) ++j;
     const uint32_t bid = blockIdx.x - G.start[j];
     const uint32_t* first = G.first[j];
-    uint32_t p = 0;
-    while (p + 1 < G.np[j] && bid >= first[p + 1]) ++p;
+    // np <= 64: one load and a ballot instead of a chain of loads
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t p = __popcll(__ballot(lane + 1 < G.np[j] && bid >= first[min(lane + 1, G.np[j])]));
     const DirectArgs& g = G.prob[j][p];
+    const uint32_t id = xcd_order(bid - first[p], first[p + 1] - first[p]);
     switch (g.config >> 2) {
-        case 0: stage_tile<1, 1, 1, 1, 4, 4>(g, bid - first[p], lds); break;
-        case 1: stage_tile<2, 2, 1, 1, 4, 3>(g, bid - first[p], lds); break;
-        default: stage_tile<2, 2, 2, 2, 1, 3>(g, bid - first[p], lds); break;
+        case 0: stage_tile<1, 1, 1, 1, 4, 3>(g, id, lds); break;
+        case 1: stage_tile<2, 2, 1, 1, 4, 2>(g, id, lds); break;
+        default: stage_tile<2, 2, 2, 2, 1, 2>(g, id, lds); break;
     }
 }
 
@@ -533,36 +540,67 @@ __device__ __forceinline__ double term_value(const AsmTerm& t, const uint32_t (&
     const uint32_t e = ((n & ((1u << t.ltn) - 1)) << t.ltm) + (m & ((1u << t.ltm) - 1));
     const double* p = t.p + ((uint64_t(tile) * t.nsplit) << (t.ltm + t.ltn)) + e;
     double v = p[0];
-    for (uint32_t s = 1; s < t.nsplit; ++s) v += p[uint64_t(s) << (t.ltm + t.ltn)];
+    uint32_t s = 1;
+    for (; s + 8 <= t.nsplit; s += 8) {   // 8 loads in flight
+        double x[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) x[u] = p[uint64_t(s + u) << (t.ltm + t.ltn)];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v += x[u];
+    }
+    for (; s < t.nsplit; ++s) v += p[uint64_t(s) << (t.ltm + t.ltn)];
     return sign * v;
 }
 
-// out[d] = sum of the terms at d, plus, where the output is symmetrised, the
-// same sum at (d1, d0, d3, d2).  One thread per element, first dimension
-// fastest; block -> output by prefix.
+__device__ __forceinline__ double terms_at(const AsmTerm* terms, uint32_t n, const uint32_t (&d)[4]) {
+    double v = 0.0;
+    for (uint32_t k = 0; k < n; ++k) v += term_value(terms[k], d);
+    return v;
+}
+
+// out[d] = sum of the terms at d; block -> output by prefix, one thread per
+// element, first dimension fastest.  A symmetrised output [n1,n1,n2,n2] adds
+// the sum at (d1,d0,d3,d2): a block takes the 16 x 16 tile (t0,t1) of slab
+// (r,s), r <= s, and its mirror, the tile (t1,t0) of slab (s,r), forms each
+// element's sum once, along its first index, and exchanges them through LDS.
+// (o = 13, v = 75: the doubles, 11 products and a tensor, 128 -> 37 us.)
 __global__ __launch_bounds__(256) void k_assemble(const AsmOut* __restrict__ outs, const AsmTerm* __restrict__ terms,
                                                   int nout) {
-    int o = 0;
-    while (o + 1 < nout && blockIdx.x >= outs[o + 1].first) ++o;
+    __shared__ double ta[16][17], tb[16][17];
+    const int lane = threadIdx.x & 63;   // nout <= 64
+    const int o = __popcll(__ballot(lane + 1 < nout && blockIdx.x >= outs[min(lane + 1, nout - 1)].first));
     const AsmOut& q = outs[o];
-    const uint32_t x = (blockIdx.x - q.first) * 256 + threadIdx.x;
-    if (x >= q.n) return;
-    uint32_t d[4], r = x;
+    const AsmTerm* t = terms + q.term;
+    const uint32_t w = blockIdx.x - q.first;
+    if (!q.sym) {
+        const uint32_t x = w * 256 + threadIdx.x;
+        if (x >= q.n) return;
+        uint32_t d[4], r = x;
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        const uint32_t c = r / q.len[k];
-        d[k] = r - c * q.len[k];
-        r = c;
+        for (int k = 0; k < 3; ++k) {
+            const uint32_t c = r / q.len[k];
+            d[k] = r - c * q.len[k];
+            r = c;
+        }
+        d[3] = r;
+        q.out[x] = terms_at(t, q.nterms, d);
+        return;
     }
-    d[3] = r;
-    const uint32_t e[4] = {d[1], d[0], d[3], d[2]};
-    double v = 0.0, w = 0.0;
-    for (uint32_t k = 0; k < q.nterms; ++k) {
-        const AsmTerm& t = terms[q.term + k];
-        v += term_value(t, d);
-        if (q.sym) w += term_value(t, e);
-    }
-    q.out[x] = q.sym ? v + w : v;
+    const uint32_t n1 = q.len[0], n2 = q.len[2], nt = (n1 + 15) / 16;
+    const uint32_t t0 = w % nt, t1 = w / nt % nt;
+    uint32_t pair = w / (nt * nt), s = 0;
+    while (pair > s) pair -= ++s;          // pair = (r, s), r <= s
+    const uint32_t r = pair;
+    if (r == s && t1 < t0) return;         // the mirrored tile's block
+    const uint32_t tx = threadIdx.x % 16, ty = threadIdx.x / 16;
+    const uint32_t d[4] = {t0 * 16 + tx, t1 * 16 + ty, r, s}, e[4] = {t1 * 16 + tx, t0 * 16 + ty, s, r};
+    const bool in_d = d[0] < n1 && d[1] < n1, in_e = e[0] < n1 && e[1] < n1;
+    const double x = in_d ? terms_at(t, q.nterms, d) : 0.0, y = in_e ? terms_at(t, q.nterms, e) : 0.0;
+    ta[ty][tx] = x;
+    tb[ty][tx] = y;
+    __syncthreads();
+    if (in_d) q.out[d[0] + n1 * (d[1] + uint64_t(n1) * (r + n2 * s))] = x + tb[tx][ty];
+    if (in_e) q.out[e[0] + n1 * (e[1] + uint64_t(n1) * (s + n2 * r))] = y + ta[tx][ty];
 }
 
 void launch_assemble(hipStream_t s, const AsmOut* outs, const AsmTerm* terms, int nout, uint32_t blocks) {
@@ -570,18 +608,72 @@ void launch_assemble(hipStream_t s, const AsmOut* outs, const AsmTerm* terms, in
     AQ_HIP(hipGetLastError());
 }
 
-void plan_stage_problem(DirectArgs& a) {
-    const Pick p = pick_shape(a, true);
-    const DirCfg& f = kDirCfg[p.cfg];
-    a.tilesM = (a.M + f.tm() - 1) / f.tm();
-    a.tilesN = (a.N + f.tn() - 1) / f.tn();
-    a.kchunk = ((a.K + 15) / 16 + p.nsplit - 1) / p.nsplit * 16;
-    a.nsplit = (a.K + a.kchunk - 1) / a.kchunk;
-    for (DirDigits* d : {&a.m, &a.n, &a.k}) set_dividers(*d);
-    const uint32_t shape = p.cfg == 3 ? 2 : uint32_t(p.cfg);   // k_stage's shapes: 16, 32, 64
-    a.config = shape * 4 + (k_runs(a.k, a.k.s0) ? 1 : 0) + (k_runs(a.k, a.k.s1) ? 2 : 0);
-    a.tm = uint32_t(f.tm());
-    a.tn = uint32_t(f.tn());
+// Tiles and splits for the problems of one level, which share the chip: with a
+// bound T on what any block may take alone, each problem takes its cheapest
+// option in CU time within T, and the level takes the larger of T and the sum
+// of those; the T that gives the shortest level is kept.
+void plan_stage_level(DirectArgs* const* a, int n) {
+    struct Option {
+        int cfg;
+        uint32_t nsplit;
+        double alone, share;
+    };
+    constexpr double kStageBlock = 1000.0;   // CU cycles of a block's start and end
+    std::vector<std::vector<Option>> opts(static_cast<size_t>(n));
+    double lo = 1e300, hi = 0.0;
+    for (int i = 0; i < n; ++i) {
+        for (int c : {0, 1, 3}) {
+            const DirCfg& f = kDirCfg[c];
+            const double chunks = std::ceil(a[i]->K / 16.0);
+            const double tiles = double((a[i]->M + f.tm() - 1) / f.tm()) * double((a[i]->N + f.tn() - 1) / f.tn());
+            for (uint32_t s = 1; s <= 128; s *= 2) {
+                if (s > 1 && (chunks / s < f.wk || tiles * s > 16384)) break;
+                const double per_wave = std::ceil(std::ceil(chunks / s) / f.wk);
+                const double busy = std::max(f.fm * f.fn * 256.0, (f.fm + f.fn) * kL1);
+                const double cu = per_wave * busy + kStageBlock;
+                const double fed = (f.tm() + f.tn()) * 128.0 * f.wk * per_wave / kChip * 256.0;
+                const double sums = s > 1 ? f.tm() * f.tn() * 16.0 / kSplitBytes * 256.0 : 0.0;
+                const double alone = per_wave * std::max(kLatency, busy) + kStart + 60.0 * s;
+                opts[size_t(i)].push_back({c, s, alone, tiles * s * (std::max(cu, fed) + sums) / 256.0});
+                lo = std::min(lo, alone);
+                hi = std::max(hi, alone);
+            }
+        }
+    }
+    auto choose = [&](const std::vector<Option>& o, double T) {
+        const Option* best = nullptr;
+        for (const auto& x : o)   // within T the smallest share; otherwise the shortest
+            if (!best || (x.alone <= T ? best->alone > T || x.share < best->share : best->alone > T && x.alone < best->alone))
+                best = &x;
+        return best;
+    };
+    double bestT = hi, best_time = 1e300;
+    for (double T = lo; T <= hi * 1.15; T *= 1.15) {
+        double sum = 0.0, longest = 0.0;
+        for (const auto& o : opts) {
+            const Option* x = choose(o, T);
+            sum += x->share;
+            longest = std::max(longest, x->alone);
+        }
+        if (std::max(sum, longest) < best_time) {
+            best_time = std::max(sum, longest);
+            bestT = T;
+        }
+    }
+    for (int i = 0; i < n; ++i) {
+        const Option* x = choose(opts[size_t(i)], bestT);
+        const DirCfg& f = kDirCfg[x->cfg];
+        DirectArgs& p = *a[i];
+        p.tilesM = (p.M + f.tm() - 1) / f.tm();
+        p.tilesN = (p.N + f.tn() - 1) / f.tn();
+        p.kchunk = ((p.K + 15) / 16 + x->nsplit - 1) / x->nsplit * 16;
+        p.nsplit = (p.K + p.kchunk - 1) / p.kchunk;
+        for (DirDigits* d : {&p.m, &p.n, &p.k}) set_dividers(*d);
+        const uint32_t shape = x->cfg == 3 ? 2 : uint32_t(x->cfg);   // k_stage's shapes: 16, 32, 64
+        p.config = shape * 4 + (k_runs(p.k, p.k.s0) ? 1 : 0) + (k_runs(p.k, p.k.s1) ? 2 : 0);
+        p.tm = uint32_t(f.tm());
+        p.tn = uint32_t(f.tn());
+    }
 }
 
 bool direct_contract(aq_ctx* ctx, DirectArgs a) {

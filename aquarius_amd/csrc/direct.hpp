@@ -58,7 +58,7 @@ struct AsmOut {
     double* out;
     uint32_t len[4], n, first, term, nterms, sym;
 };
-void plan_stage_problem(DirectArgs& a);   // tile, split and layout of a problem (a.P is the caller's)
+void plan_stage_level(DirectArgs* const* a, int n);   // tiles, splits and layouts of a level's problems (P is the caller's)
 void launch_stage(const StageLevel* const* l, int n, hipStream_t s);
 void launch_assemble(hipStream_t s, const AsmOut* outs, const AsmTerm* terms, int nout, uint32_t blocks);
 // sum_k A[ia] B[ib] with output labels ic as a problem (sizes, digits, operands);

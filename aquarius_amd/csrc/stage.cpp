@@ -19,6 +19,10 @@ int StageProgram::product(int level, const tensor::Tensor& A, const char* ia, co
 }
 
 void StageProgram::output(int level, const tensor::Tensor& out, const char* ic, bool sym) {
+    if (sym) {
+        const auto l = out.lengths();
+        ok_ = ok_ && l.size() == 4 && l[0] == l[1] && l[2] == l[3];
+    }
     outputs_.push_back({level, &out, ic, sym, {}});
 }
 void StageProgram::add(double coef, const tensor::Tensor& X, const char* ix) {
@@ -44,8 +48,13 @@ void StageProgram::finish() {
     // tiles of every product, one buffer; a level's long blocks come first
     int64_t total = 0;
     std::vector<int64_t> at;
+    for (int l = 0; l < nlevels; ++l) {
+        std::vector<DirectArgs*> a;
+        for (auto& p : products_)
+            if (p.level == l) a.push_back(&p.a);
+        plan_stage_level(a.data(), int(a.size()));
+    }
     for (auto& p : products_) {
-        plan_stage_problem(p.a);
         at.push_back(total);
         total += int64_t(p.a.tilesM) * p.a.tilesN * p.a.nsplit * p.a.tm * p.a.tn;
     }
@@ -93,7 +102,8 @@ void StageProgram::finish() {
             q.term = uint32_t(terms.size());
             q.nterms = uint32_t(o.terms.size());
             q.sym = o.sym ? 1 : 0;
-            L.blocks += (q.n + 255) / 256;
+            const uint32_t nt = (q.len[0] + 15) / 16;
+            L.blocks += o.sym ? nt * nt * (q.len[2] * (q.len[2] + 1) / 2) : (q.n + 255) / 256;
             outs.push_back(q);
             written_.push_back(o.t);
             for (const auto& tm : o.terms) {
@@ -124,6 +134,7 @@ void StageProgram::finish() {
                 terms.push_back(d);
             }
         }
+        AQ_CHECK(args.size() <= 64 && outs.size() <= 64, AQ_ERR_INVALID, "stage level size");
         L.nout = int(outs.size());
         Offsets& f = offs[size_t(l)];
         f.prob = place(args.data(), args.size() * sizeof(DirectArgs));
