@@ -4,10 +4,12 @@
 //
 // m, n and k are groups of labels with arbitrary strides in A, B and C, so no
 // operand is permuted into a matrix first and no result is permuted
-// afterwards.  FP64 MFMA on gfx950 is slow against its operands: a 16x16x4
-// instruction takes 64 cycles for two 512-byte fragments, so fragments are
-// loaded from global memory (L1/L2) into registers directly, without LDS
-// staging and without a barrier in the k loop; every wave runs on its own.
+// afterwards.  Two kinds of tile:
+//  - from registers: FP64 MFMA on gfx950 is slow against its operands, a 16x16x4
+//    instruction takes 64 cycles for two 512-byte fragments, so fragments are
+//    loaded from global memory (L1/L2) into registers directly, without LDS
+//    staging and without a barrier in the k loop; every wave runs on its own;
+//  - staged through LDS, 64 x 64 and 128 x 128, for many long tiles (below).
 //
 // A block of 256 threads = WM x WN x WK waves owns a (16 FM WM) x (16 FN WN)
 // output tile; each wave has FM x FN 16x16 MFMA blocks, and WK waves share the
@@ -43,13 +45,16 @@ constexpr int kKT = 1024;   // k offsets held at a time
 __device__ __forceinline__ uint32_t digit_offset(const DirDigits& d, const uint32_t* st, uint32_t x) {
     uint32_t off = 0;
 #pragma unroll
-    for (int k = 0; k + 1 < kDirDigits; ++k) {
-        if (k + 1 >= d.nd) break;
-        const uint32_t q = __umulhi(x, d.mul[k]) >> d.shift[k];
-        off += (x - q * d.len[k]) * st[k];
-        x = q;
+    for (int k = 0; k < kDirDigits; ++k) {   // static indices only: the group stays in scalar registers
+        if (k + 1 < kDirDigits && k + 1 < d.nd) {
+            const uint32_t q = __umulhi(x, d.mul[k]) >> d.shift[k];
+            off += (x - q * d.len[k]) * st[k];
+            x = q;
+        } else if (k + 1 == d.nd) {
+            off += x * st[k];
+        }
     }
-    return d.nd > 0 ? off + x * st[d.nd - 1] : 0u;
+    return off;
 }
 
 // block id -> work id: the dispatcher deals ids to the 8 XCDs round-robin; give
@@ -63,6 +68,104 @@ __device__ __forceinline__ uint32_t xcd_order(uint32_t bid, uint32_t nb) {
 constexpr int direct_lds(int fm, int fn, int wm, int wn, int wk) {
     const int red = wk > 1 ? wk * fm * fn * wm * wn * 256 * 8 : 0, tab = 2 * kKT * 4;
     return red > tab ? red : tab;
+}
+
+// The epilogue: the tile into C, or (a split, a batched stage) into its place in
+// the partial buffer.
+template <int FM, int FN, int WM, int WN, int WK, bool TILE>
+__device__ __forceinline__ void store_tile(const DirectArgs& g, const f64x4 (&acc)[FM][FN], uint32_t split, uint32_t bt,
+                                           uint32_t m0, uint32_t n0, char* lds) {
+    constexpr int TM = 16 * FM * WM, TN = 16 * FN * WN;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wk = wave % WK, wm = (wave / WK) % WM, wn = wave / (WK * WM);
+    const int l16 = lane & 15, q = lane >> 4;
+    const uint32_t b = bt / (g.tilesM * g.tilesN);
+    // lane holds tile element (m = l16 of block i, n = q + 4r of block j)
+    double* Cb = g.C + uint64_t(b) * g.bsC;
+    if (!TILE && WK == 1 && g.nsplit == 1) {
+        uint32_t cn[FN][4];
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                cn[j][r] = digit_offset(g.n, g.n.s1, min(n0 + (wn * FN + j) * 16 + q + 4 * r, g.N - 1));
+#pragma unroll
+        for (int i = 0; i < FM; ++i) {
+            const uint32_t m = m0 + (wm * FM + i) * 16 + l16;
+            const uint32_t cm = digit_offset(g.m, g.m.s1, min(m, g.M - 1));
+            // every C value of the row is read before any is written (one round trip)
+            double cv[FN][4];
+            if (g.beta != 0.0) {
+#pragma unroll
+                for (int j = 0; j < FN; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) cv[j][r] = Cb[cm + cn[j][r]];
+            }
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const uint32_t n = n0 + (wn * FN + j) * 16 + q + 4 * r;
+                    if (m < g.M && n < g.N) {
+                        double v = g.alpha * acc[i][j][r];
+                        if (g.beta != 0.0) v += g.beta * cv[j][r];
+                        Cb[cm + cn[j][r]] = v;
+                    }
+                }
+        }
+        return;
+    }
+
+    constexpr int TE = TM * TN, NE = TE / 256;   // tile elements, and per thread
+    static_assert(TE % 256 == 0, "whole tile per thread count");
+    double v[NE];
+    if (WK > 1) {
+        double* red = reinterpret_cast<double*>(lds);
+        __syncthreads();   // the k tables are no longer read
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    red[wk * TE + ((wn * FN + j) * 16 + q + 4 * r) * TM + (wm * FM + i) * 16 + l16] = acc[i][j][r];
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < NE; ++r) {
+            double s = red[tid + 256 * r];
+#pragma unroll
+            for (int w = 1; w < WK; ++w) s += red[w * TE + tid + 256 * r];
+            v[r] = s;
+        }
+    }
+    if (TILE || g.nsplit > 1) {
+        double* P = g.P + uint64_t(bt) * g.nsplit * TE;
+        double* mine = P + uint64_t(split) * TE;
+        if (WK > 1) {
+#pragma unroll
+            for (int r = 0; r < NE; ++r) mine[tid + 256 * r] = v[r];
+        } else {
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int j = 0; j < FN; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        mine[((wn * FN + j) * 16 + q + 4 * r) * TM + (wm * FM + i) * 16 + l16] = acc[i][j][r];
+        }
+        return;
+    }
+#pragma unroll
+    for (int r = 0; r < NE; ++r) {
+        const uint32_t e = tid + 256 * r;
+        const uint32_t m = m0 + e % TM, n = n0 + e / TM;
+        if (m < g.M && n < g.N) {
+            double* c = Cb + digit_offset(g.m, g.m.s1, m) + digit_offset(g.n, g.n.s1, n);
+            const double x = g.alpha * v[r];
+            *c = g.beta != 0.0 ? g.beta * *c + x : x;
+        }
+    }
 }
 
 // TILE: the tile goes to the partial buffer whatever the split (batched stages,
@@ -198,91 +301,166 @@ __device__ __forceinline__ void direct_tile(const DirectArgs& g, uint32_t bid, c
         }
     }
 
-    // lane holds tile element (m = l16 of block i, n = q + 4r of block j)
-    double* Cb = g.C + uint64_t(b) * g.bsC;
-    if (!TILE && WK == 1 && g.nsplit == 1) {
-        uint32_t cn[FN][4];
+    store_tile<FM, FN, WM, WN, WK, TILE>(g, acc, split, bt, m0, n0, lds);
+}
+
+// 64 x 64 and 128 x 128 tiles staged through LDS: 2 x 2 waves of F x F blocks
+// share the operands, each element is loaded once per tile, and an operand is
+// read along whichever of its rows (KA, KB false) or k (true) is contiguous.  That
+// is what the register path lacks on long contractions: its fragments need 20
+// L1 accesses for a 64-lane load when k and rows are both strided in memory, a
+// chunk then costs 2300 cycles of the CU instead of the 1024 of its MFMAs
+// (three 975^3 side by side: 174 us, 130 so; 2800^3: 950 us, 840 with 128 x
+// 128, which also needs half the LDS and L2 traffic of 64 x 64).  A chunk is
+// loaded into registers while the one before it is multiplied; LDS holds it as
+// [k][row] or [row][k], padded so that the 32 lanes of a half-wave read 32
+// different bank pairs.  What is left is the matrix cores' own rate: they are
+// busy 75% of the time and waits for data are 7%; neither a deeper prefetch (2
+// or 3 chunks) nor the stores to LDS between the products changes that, and
+// random values run 9% slower than constants (a power limit on short kernels:
+// the same loop reaches 72 TFLOP/s over 15 ms, 59 over 2 ms).
+template <int F>
+struct Staged {
+    static constexpr int T = 32 * F, PR = T + 16, PK = 18;             // tile side, pitches
+    static constexpr int kOperand = 16 * PR > T * PK ? 16 * PR : T * PK;   // elements of one chunk
+    static constexpr int kTab = 512;                                   // k offsets held at a time
+    static constexpr int kLds = 4 * kOperand * 8 + 2 * kTab * 4;
+};
+
+template <int F, bool KA, bool KB, bool TILE = false>
+__device__ __forceinline__ void staged_tile(const DirectArgs& g, uint32_t bid, char* lds) {
+    using S = Staged<F>;
+    constexpr int T = S::T, L = T / 16;   // tile side; elements a thread loads of an operand per chunk
+    double* const sa = reinterpret_cast<double*>(lds);                    // two chunks of A,
+    double* const sb = sa + 2 * S::kOperand;                              // two of B
+    uint32_t* ta = reinterpret_cast<uint32_t*>(sb + 2 * S::kOperand);
+    uint32_t* tb = ta + S::kTab;
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave & 1, wn = wave >> 1;
+    const int l16 = lane & 15, q = lane >> 4;
+    const uint32_t tiles = g.tilesM * g.tilesN;   // work id as in direct_tile
+    const uint32_t split = bid / (tiles * g.batch);
+    const uint32_t bt = bid % (tiles * g.batch);
+    const uint32_t b = bt / tiles, tile = bt % tiles;
+    // tiles in bands of 8 rows: those that run side by side on an XCD then share
+    // operand rows both ways
+    const uint32_t band = tile / (8 * g.tilesN) * 8, in = tile % (8 * g.tilesN);
+    const uint32_t rows = min(8u, g.tilesM - band);
+    const uint32_t tm = band + in % rows, tn = in / rows;
+    const uint32_t m0 = tm * T, n0 = tn * T;
+    const uint32_t kbeg = split * g.kchunk, kend = min(g.K, kbeg + g.kchunk);
+    const char* Ab = reinterpret_cast<const char*>(g.A + uint64_t(b) * g.bsA);
+    const char* Bb = reinterpret_cast<const char*>(g.B + uint64_t(b) * g.bsB);
+
+    // the elements (row, k) = (rX + i, kX) or (rX, kX + i) a thread carries, and
+    // the byte offsets of its rows (past the edge: the last one, never stored)
+    constexpr int NA = KA ? L : 1, NB = KB ? L : 1;
+    const int rA = KA ? tid / 16 : tid % T, kA = KA ? tid % 16 : tid / T;
+    const int rB = KB ? tid / 16 : tid % T, kB = KB ? tid % 16 : tid / T;
+    uint32_t ra[NA], rb[NB];
 #pragma unroll
-        for (int j = 0; j < FN; ++j)
+    for (int i = 0; i < NA; ++i) ra[i] = digit_offset(g.m, g.m.s0, min(m0 + rA + 16 * i, g.M - 1)) * 8u;
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                cn[j][r] = digit_offset(g.n, g.n.s1, min(n0 + (wn * FN + j) * 16 + q + 4 * r, g.N - 1));
+    for (int i = 0; i < NB; ++i) rb[i] = digit_offset(g.n, g.n.s0, min(n0 + rB + 16 * i, g.N - 1)) * 8u;
+
+    f64x4 acc[F][F];
 #pragma unroll
-        for (int i = 0; i < FM; ++i) {
-            const uint32_t m = m0 + (wm * FM + i) * 16 + l16;
-            const uint32_t cm = digit_offset(g.m, g.m.s1, min(m, g.M - 1));
-            // every C value of the row is read before any is written (one round trip)
-            double cv[FN][4];
-            if (g.beta != 0.0) {
+    for (int i = 0; i < F; ++i)
 #pragma unroll
-                for (int j = 0; j < FN; ++j)
+        for (int j = 0; j < F; ++j) acc[i][j] = f64x4{0, 0, 0, 0};
+
+    constexpr int KS = 256 / T;   // k step between a thread's elements along k
+    for (uint32_t kb = kbeg; kb < kend; kb += S::kTab) {
+        const uint32_t klen = min(uint32_t(S::kTab), kend - kb), nch = (klen + 15) / 16;
+        for (uint32_t k = tid; k < nch * 16; k += 256) {
+            const uint32_t kk = kb + min(k, klen - 1);   // past the end: the last k, zeroed before its use
+            ta[k] = digit_offset(g.k, g.k.s0, kk) * 8u;
+            tb[k] = digit_offset(g.k, g.k.s1, kk) * 8u;
+        }
+        __syncthreads();
+        double x[L], y[L];         // the next chunk's elements of A and B
+        uint32_t oa[L], ob[L];     // k offsets of the chunk to be loaded next
+        auto offsets = [&](uint32_t c) {
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) cv[j][r] = Cb[cm + cn[j][r]];
+            for (int i = 0; i < L; ++i) {
+                if (i == 0 || !KA) oa[i] = ta[c * 16 + kA + (KA ? 0 : KS * i)];
+                if (i == 0 || !KB) ob[i] = tb[c * 16 + kB + (KB ? 0 : KS * i)];
+            }
+        };
+        auto load = [&] {
+#pragma unroll
+            for (int i = 0; i < L; ++i)
+                x[i] = *reinterpret_cast<const double*>(Ab + (ra[KA ? i : 0] + oa[KA ? 0 : i]));
+#pragma unroll
+            for (int i = 0; i < L; ++i)
+                y[i] = *reinterpret_cast<const double*>(Bb + (rb[KB ? i : 0] + ob[KB ? 0 : i]));
+        };
+        auto put = [&](uint32_t c) {
+            double* pa = sa + (c & 1) * S::kOperand;
+            double* pb = sb + (c & 1) * S::kOperand;
+            if (c * 16 + 16 > klen) {   // the partial last chunk
+#pragma unroll
+                for (int i = 0; i < L; ++i) {
+                    x[i] = c * 16 + kA + (KA ? 0 : KS * i) < klen ? x[i] : 0.0;
+                    y[i] = c * 16 + kB + (KB ? 0 : KS * i) < klen ? y[i] : 0.0;
+                }
             }
 #pragma unroll
-            for (int j = 0; j < FN; ++j)
+            for (int i = 0; i < L; ++i) pa[KA ? (rA + 16 * i) * S::PK + kA : (kA + KS * i) * S::PR + rA] = x[i];
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const uint32_t n = n0 + (wn * FN + j) * 16 + q + 4 * r;
-                    if (m < g.M && n < g.N) {
-                        double v = g.alpha * acc[i][j][r];
-                        if (g.beta != 0.0) v += g.beta * cv[j][r];
-                        Cb[cm + cn[j][r]] = v;
-                    }
-                }
-        }
-        return;
-    }
-
-    constexpr int TE = TM * TN, NE = TE / 256;   // tile elements, and per thread
-    static_assert(TE % 256 == 0, "whole tile per thread count");
-    double v[NE];
-    if (WK > 1) {
-        double* red = reinterpret_cast<double*>(lds);
-        __syncthreads();   // the k tables are no longer read
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-            for (int j = 0; j < FN; ++j)
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    red[wk * TE + ((wn * FN + j) * 16 + q + 4 * r) * TM + (wm * FM + i) * 16 + l16] = acc[i][j][r];
+            for (int i = 0; i < L; ++i) pb[KB ? (rB + 16 * i) * S::PK + kB : (kB + KS * i) * S::PR + rB] = y[i];
+        };
+        offsets(0);
+        load();
+        offsets(min(1u, nch - 1));
+        put(0);
         __syncthreads();
+        for (uint32_t c = 0; c < nch; ++c) {
+            const double* pa = sa + (c & 1) * S::kOperand;
+            const double* pb = sb + (c & 1) * S::kOperand;
+            double fa0[F], fb0[F], fa1[F], fb1[F];
+            auto fragments = [&](double (&fa)[F], double (&fb)[F], int s) {
+                const int k = 4 * s + q;
 #pragma unroll
-        for (int r = 0; r < NE; ++r) {
-            double s = red[tid + 256 * r];
+                for (int i = 0; i < F; ++i) {
+                    const int r = (wm * F + i) * 16 + l16;
+                    fa[i] = pa[KA ? r * S::PK + k : k * S::PR + r];
+                }
 #pragma unroll
-            for (int w = 1; w < WK; ++w) s += red[w * TE + tid + 256 * r];
-            v[r] = s;
+                for (int j = 0; j < F; ++j) {
+                    const int r = (wn * F + j) * 16 + l16;
+                    fb[j] = pb[KB ? r * S::PK + k : k * S::PR + r];
+                }
+            };
+            auto mma = [&](const double (&fa)[F], const double (&fb)[F]) {
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = 0; i < F; ++i)
+#pragma unroll
+                    for (int j = 0; j < F; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fb[j], fa[i], acc[i][j], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            // nothing waits for what was just asked for: the next chunk is loaded
+            // with offsets read a chunk ago (past the end: the last chunk again),
+            // each step's fragments are read a step ahead
+            fragments(fa0, fb0, 0);
+            fragments(fa1, fb1, 1);
+            load();
+            offsets(min(c + 2, nch - 1));
+            mma(fa0, fb0);
+            fragments(fa0, fb0, 2);
+            mma(fa1, fb1);
+            fragments(fa1, fb1, 3);
+            mma(fa0, fb0);
+            mma(fa1, fb1);
+            put(c + 1);   // into the buffer whose readers passed the last barrier
+            __syncthreads();
         }
     }
-    if (TILE || g.nsplit > 1) {
-        double* P = g.P + uint64_t(bt) * g.nsplit * TE;
-        double* mine = P + uint64_t(split) * TE;
-        if (WK > 1) {
-#pragma unroll
-            for (int r = 0; r < NE; ++r) mine[tid + 256 * r] = v[r];
-        } else {
-#pragma unroll
-            for (int i = 0; i < FM; ++i)
-#pragma unroll
-                for (int j = 0; j < FN; ++j)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        mine[((wn * FN + j) * 16 + q + 4 * r) * TM + (wm * FM + i) * 16 + l16] = acc[i][j][r];
-        }
-        return;
-    }
-#pragma unroll
-    for (int r = 0; r < NE; ++r) {
-        const uint32_t e = tid + 256 * r;
-        const uint32_t m = m0 + e % TM, n = n0 + e / TM;
-        if (m < g.M && n < g.N) {
-            double* c = Cb + digit_offset(g.m, g.m.s1, m) + digit_offset(g.n, g.n.s1, n);
-            const double x = g.alpha * v[r];
-            *c = g.beta != 0.0 ? g.beta * *c + x : x;
-        }
-    }
+    store_tile<F, F, 2, 2, 1, TILE>(g, acc, split, b * tiles + tm + tn * g.tilesM, m0, n0, lds);
 }
 
 // C from the partial tiles of a split launch: one thread per tile element, the
@@ -316,6 +494,12 @@ __global__ __launch_bounds__(256) void k_direct(DirectArgs g) {
     direct_tile<FM, FN, WM, WN, WK, ST, VA, VB>(g, xcd_order(blockIdx.x, gridDim.x), lds);
 }
 
+template <int F, bool KA, bool KB>
+__global__ __launch_bounds__(256, F == 2 ? 3 : 2) void k_staged(DirectArgs g) {
+    __shared__ __attribute__((aligned(16))) char lds[Staged<F>::kLds];
+    staged_tile<F, KA, KB>(g, xcd_order(blockIdx.x, gridDim.x), lds);
+}
+
 // The tiles of up to kDirGroup problems of different contexts in one launch;
 // each tile is computed exactly as in a launch of its problem alone.
 struct DirectGroup {
@@ -332,24 +516,44 @@ __global__ __launch_bounds__(256) void k_direct_grouped(DirectGroup G) {
     direct_tile<FM, FN, WM, WN, WK, ST, VA, VB>(G.p[p], xcd_order(blockIdx.x - G.first[p], G.first[p + 1] - G.first[p]), lds);
 }
 
+template <int F, bool KA, bool KB>
+__global__ __launch_bounds__(256, F == 2 ? 3 : 2) void k_staged_grouped(DirectGroup G) {
+    __shared__ __attribute__((aligned(16))) char lds[Staged<F>::kLds];
+    int p = 0;
+    while (p + 1 < G.n && blockIdx.x >= G.first[p + 1]) ++p;
+    staged_tile<F, KA, KB>(G.p[p], xcd_order(blockIdx.x - G.first[p], G.first[p + 1] - G.first[p]), lds);
+}
+
+// constants of the time model (pick_shape), clock cycles
+constexpr double kL1 = 286.0, kLatency = 1033.0, kStart = 2337.0, kBlock = 258.0, kChip = 5534.0;
+constexpr double kLaunch = 1.5, kSplit = 2.6, kSplitBytes = 3509.0, kPerSplit = 0.06, kGHz = 2400.0;
+constexpr double kStagedBusy = 1.05, kStagedWait = 925.0;
+
 struct DirCfg {
-    int fm, fn, wm, wn, wk, stages;
+    int fm, fn, wm, wn, wk, stages;   // stages 0: staged through LDS
     int tm() const { return 16 * fm * wm; }
     int tn() const { return 16 * fn * wn; }
+    // cycles of a CU per chunk of a block (of each wave)
+    double busy() const {
+        if (!stages) return fm * fn * 256.0 * kStagedBusy;
+        return std::max(fm * fn * 256.0, (fm + fn) * kL1);
+    }
 };
 constexpr DirCfg kDirCfg[] = {
     {1, 1, 1, 1, 4, 4},   // 16 x 16: tiny outputs
     {2, 2, 1, 1, 4, 3},   // 32 x 32, waves share k
     {1, 1, 2, 2, 1, 4},   // 32 x 32, short k
-    {2, 2, 2, 2, 1, 3},   // 64 x 64
+    {2, 2, 2, 2, 1, 0},   // 64 x 64, staged through LDS
     {4, 1, 1, 1, 4, 3},   // 64 x 16
     {1, 4, 1, 1, 4, 3},   // 16 x 64
     {4, 1, 4, 1, 1, 2},   // 256 x 16, short k
     {1, 4, 1, 4, 1, 2},   // 16 x 256, short k
+    {4, 4, 2, 2, 1, 0},   // 128 x 128, staged
+    {2, 2, 2, 2, 1, 3},   // 64 x 64, from registers: a block alone on its CU
 };
 constexpr int kNDirCfg = int(sizeof(kDirCfg) / sizeof(kDirCfg[0]));
 
-template <int FM, int FN, int WM, int WN, int WK, int ST, class F>
+template <class F>
 static void with_layout(int va, int vb, F&& f) {
     if (va && vb) f(std::integral_constant<int, 3>{});
     else if (va) f(std::integral_constant<int, 1>{});
@@ -359,13 +563,23 @@ static void with_layout(int va, int vb, F&& f) {
 
 template <int FM, int FN, int WM, int WN, int WK, int ST>
 static void run_direct(int lay, dim3 grid, hipStream_t s, const DirectArgs* one, const DirectGroup* many) {
-    with_layout<FM, FN, WM, WN, WK, ST>(lay & 1, lay & 2, [&](auto L) {
+    with_layout(lay & 1, lay & 2, [&](auto L) {
         constexpr int l = decltype(L)::value;
         if (one)
             hipLaunchKernelGGL((k_direct<FM, FN, WM, WN, WK, ST, (l & 1) != 0, (l & 2) != 0>), grid, dim3(256), 0, s, *one);
         else
             hipLaunchKernelGGL((k_direct_grouped<FM, FN, WM, WN, WK, ST, (l & 1) != 0, (l & 2) != 0>), grid, dim3(256), 0,
                                s, *many);
+    });
+    AQ_HIP(hipGetLastError());
+}
+
+template <int F>
+static void run_staged(int lay, dim3 grid, hipStream_t s, const DirectArgs* one, const DirectGroup* many) {
+    with_layout(lay & 1, lay & 2, [&](auto L) {
+        constexpr bool ka = (decltype(L)::value & 1) != 0, kb = (decltype(L)::value & 2) != 0;
+        if (one) hipLaunchKernelGGL((k_staged<F, ka, kb>), grid, dim3(256), 0, s, *one);
+        else hipLaunchKernelGGL((k_staged_grouped<F, ka, kb>), grid, dim3(256), 0, s, *many);
     });
     AQ_HIP(hipGetLastError());
 }
@@ -377,11 +591,13 @@ static void dispatch_direct(int config, dim3 grid, hipStream_t s, const DirectAr
         case 0: run_direct<1, 1, 1, 1, 4, 4>(lay, grid, s, one, many); break;
         case 1: run_direct<2, 2, 1, 1, 4, 3>(lay, grid, s, one, many); break;
         case 2: run_direct<1, 1, 2, 2, 1, 4>(lay, grid, s, one, many); break;
-        case 3: run_direct<2, 2, 2, 2, 1, 3>(lay, grid, s, one, many); break;
+        case 3: run_staged<2>(lay, grid, s, one, many); break;
         case 4: run_direct<4, 1, 1, 1, 4, 3>(lay, grid, s, one, many); break;
         case 5: run_direct<1, 4, 1, 1, 4, 3>(lay, grid, s, one, many); break;
         case 6: run_direct<4, 1, 4, 1, 1, 2>(lay, grid, s, one, many); break;
-        default: run_direct<1, 4, 1, 4, 1, 2>(lay, grid, s, one, many); break;
+        case 7: run_direct<1, 4, 1, 4, 1, 2>(lay, grid, s, one, many); break;
+        case 8: run_staged<4>(lay, grid, s, one, many); break;
+        default: run_direct<2, 2, 2, 2, 1, 3>(lay, grid, s, one, many); break;
     }
 }
 
@@ -413,6 +629,12 @@ static bool k_runs(const DirDigits& k, const uint32_t* st) {
     return k.nd >= 1 && st[0] == 1 && (k.nd == 1 || k.len[0] % 4 == 0);
 }
 
+// The layout bits of an operand's kernel, whose k strides are `st`: a staged tile
+// reads it along k if that is contiguous; the register path loads pairs of k.
+static bool k_layout(const DirCfg& f, const DirDigits& k, const uint32_t* st) {
+    return f.stages == 0 ? k.nd >= 1 && st[0] == 1 : k_runs(k, st);
+}
+
 // Tile shape and split of one problem: the least modelled time over the
 // shapes and power-of-two splits.  Model (clock cycles; the constants are a
 // least-regret fit to 39 contractions of the CCSD iteration at five sizes, o =
@@ -422,8 +644,6 @@ static bool k_runs(const DirDigits& k, const uint32_t* st) {
 // least the load latency over the chunks in flight; blocks queue on 256 CUs;
 // operand tiles come in at a rate of the whole chip; a split pays a second
 // launch and the traffic of the partial tiles.
-constexpr double kL1 = 286.0, kLatency = 1033.0, kStart = 2337.0, kBlock = 258.0, kChip = 5534.0;
-constexpr double kLaunch = 1.5, kSplit = 2.6, kSplitBytes = 3509.0, kPerSplit = 0.06, kGHz = 2400.0;
 
 struct Pick {
     int cfg = -1;
@@ -441,8 +661,8 @@ static Pick pick_shape(const DirectArgs& a) {
             if (s > 1 && (chunks / s < f.wk || tiles * s > 16384)) break;
             const double blocks = tiles * s;
             const double per_wave = std::ceil(std::ceil(chunks / s) / f.wk);
-            const double busy = std::max(f.fm * f.fn * 256.0, (f.fm + f.fn) * kL1);
-            const double alone = per_wave * std::max(kLatency / (f.stages - 1), busy) + kStart;
+            const double busy = f.busy();
+            const double alone = per_wave * (f.stages ? std::max(kLatency / (f.stages - 1), busy) : busy + kStagedWait) + kStart;
             const double queued = std::ceil(blocks / 256.0) * (per_wave * busy + kBlock);
             const double fed = (f.tm() + f.tn()) * 128.0 * f.wk * per_wave * blocks / kChip;
             double t = kLaunch + std::max({alone, queued, fed}) / kGHz;
@@ -484,7 +704,7 @@ __device__ __forceinline__ void stage_tile(const DirectArgs& g, uint32_t bid, ch
 // blocks of a level are short and mostly wait (o = 8, v = 43: 37 us a launch
 // with 4/3/3 chunks and two waves, 29 us with 3/2/2 and three).
 __global__ __launch_bounds__(256, 3) void k_stage(StageGroup G) {
-    __shared__ __attribute__((aligned(16))) char lds[direct_lds(2, 2, 1, 1, 4)];   // the largest of the shapes
+    __shared__ __attribute__((aligned(16))) char lds[Staged<2>::kLds];   // the largest of the shapes
     int j = 0;
     while (j + 1 < G.n && blockIdx.x >= G.start[j + 1]) ++j;
     const uint32_t bid = blockIdx.x - G.start[j];
@@ -497,7 +717,13 @@ __global__ __launch_bounds__(256, 3) void k_stage(StageGroup G) {
     switch (g.config >> 2) {
         case 0: stage_tile<1, 1, 1, 1, 4, 3>(g, id, lds); break;
         case 1: stage_tile<2, 2, 1, 1, 4, 2>(g, id, lds); break;
-        default: stage_tile<2, 2, 2, 2, 1, 2>(g, id, lds); break;
+        default:
+            switch (g.config & 3) {
+                case 0: staged_tile<2, false, false, true>(g, id, lds); break;
+                case 1: staged_tile<2, true, false, true>(g, id, lds); break;
+                case 2: staged_tile<2, false, true, true>(g, id, lds); break;
+                default: staged_tile<2, true, true, true>(g, id, lds); break;
+            }
     }
 }
 
@@ -611,14 +837,19 @@ void launch_assemble(hipStream_t s, const AsmOut* outs, const AsmTerm* terms, in
 // Tiles and splits for the problems of one level, which share the chip: with a
 // bound T on what any block may take alone, each problem takes its cheapest
 // option in CU time within T, and the level takes the larger of T and the sum
-// of those; the T that gives the shortest level is kept.
+// of those; the T that gives the shortest level is kept.  A chunk of a block
+// alone takes about 2000 cycles in every tile; a model without that left K =
+// 5625 unsplit and its 264 us set the length of the level (o = 13, v = 75: 410 us
+// against 322).
 void plan_stage_level(DirectArgs* const* a, int n) {
     struct Option {
         int cfg;
         uint32_t nsplit;
         double alone, share;
     };
-    constexpr double kStageBlock = 1000.0;   // CU cycles of a block's start and end
+    constexpr double kStageBlock = 1000.0;     // CU cycles of a block's start and end
+    constexpr double kStageLatency = 2000.0;   // a chunk of a block alone, whatever its tile
+    constexpr double kStageSplit = 60.0;       // the assembly's cycles per partial tile
     std::vector<std::vector<Option>> opts(static_cast<size_t>(n));
     double lo = 1e300, hi = 0.0;
     for (int i = 0; i < n; ++i) {
@@ -629,11 +860,11 @@ void plan_stage_level(DirectArgs* const* a, int n) {
             for (uint32_t s = 1; s <= 128; s *= 2) {
                 if (s > 1 && (chunks / s < f.wk || tiles * s > 16384)) break;
                 const double per_wave = std::ceil(std::ceil(chunks / s) / f.wk);
-                const double busy = std::max(f.fm * f.fn * 256.0, (f.fm + f.fn) * kL1);
+                const double busy = f.busy();
                 const double cu = per_wave * busy + kStageBlock;
                 const double fed = (f.tm() + f.tn()) * 128.0 * f.wk * per_wave / kChip * 256.0;
                 const double sums = s > 1 ? f.tm() * f.tn() * 16.0 / kSplitBytes * 256.0 : 0.0;
-                const double alone = per_wave * std::max(kLatency, busy) + kStart + 60.0 * s;
+                const double alone = per_wave * std::max(kStageLatency, busy) + kStart + kStageSplit * s;
                 opts[size_t(i)].push_back({c, s, alone, tiles * s * (std::max(cu, fed) + sums) / 256.0});
                 lo = std::min(lo, alone);
                 hi = std::max(hi, alone);
@@ -670,7 +901,7 @@ void plan_stage_level(DirectArgs* const* a, int n) {
         p.nsplit = (p.K + p.kchunk - 1) / p.kchunk;
         for (DirDigits* d : {&p.m, &p.n, &p.k}) set_dividers(*d);
         const uint32_t shape = x->cfg == 3 ? 2 : uint32_t(x->cfg);   // k_stage's shapes: 16, 32, 64
-        p.config = shape * 4 + (k_runs(p.k, p.k.s0) ? 1 : 0) + (k_runs(p.k, p.k.s1) ? 2 : 0);
+        p.config = shape * 4 + (k_layout(f, p.k, p.k.s0) ? 1 : 0) + (k_layout(f, p.k, p.k.s1) ? 2 : 0);
         p.tm = uint32_t(f.tm());
         p.tn = uint32_t(f.tn());
     }
@@ -690,7 +921,7 @@ bool direct_contract(aq_ctx* ctx, DirectArgs a) {
     Scratch part(ctx, a.nsplit > 1 ? size_t(tiles) * a.nsplit * f.tm() * f.tn() * 8 : 0);
     for (DirDigits* d : {&a.m, &a.n, &a.k}) set_dividers(*d);
     a.P = part.as<double>();
-    const int config = p.cfg * 4 + (k_runs(a.k, a.k.s0) ? 1 : 0) + (k_runs(a.k, a.k.s1) ? 2 : 0);
+    const int config = p.cfg * 4 + (k_layout(f, a.k, a.k.s0) ? 1 : 0) + (k_layout(f, a.k, a.k.s1) ? 2 : 0);
     char name[64];
     snprintf(name, sizeof(name), "direct_f64_%dx%d", f.tm(), f.tn());
     const double mn = double(a.M) * a.N * a.batch;

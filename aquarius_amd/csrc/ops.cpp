@@ -400,10 +400,12 @@ static bool digits_of(const std::string& order, const Labeled& X, const Labeled&
 //    partials): 110 x 110 x 21560 50/32, 140 x 20 x 392000 244/160;
 //  - a short side and a short inner extent against a long side: 140 x 56000 x
 //    140 111/81;
-//  - large products whose operands are both contiguous along the rows: 975^3
-//    63/44, 1540^3 190/165, 2800^3 838/783 (the GEMM side 12-23% permutes);
-//    with k contiguous in one of them the GEMM side is the faster (1540^3
-//    193/265).
+//  - large products whose GEMM would have to permute: 975^3 72/64, 1600^3
+//    226/203, 2800^3 950/840 (both operands strided, amplitudes permuted anew);
+//    beyond, permuting costs less than the LDS tiles lose to the GEMM's (3080^3
+//    1240/1280).  Operands that are matrices as they lie stay with the GEMM
+//    (10000 x 256 x 256 39/57), and so do two that are both contiguous along k,
+//    which one cached copy or none serves (2800 x 400 x 19600 1030/1510).
 static bool direct_size(const DirectArgs& a, bool scattered, bool rows_x, bool rows_y, int64_t sizeX) {
     const double out = double(a.M) * a.N * a.batch, flops = 2.0 * out * a.K;
     if (scattered && out > 2e5) return false;
@@ -411,7 +413,9 @@ static bool direct_size(const DirectArgs& a, bool scattered, bool rows_x, bool r
     if (flops <= 6e8) return true;
     if (out <= 2.5e4) return flops <= 2e10;
     if (a.M <= 200 && a.K <= 200 && double(a.N) >= 50.0 * a.M) return flops <= 2e10;
-    return rows_x && rows_y && !scattered && a.M > 200 && a.N > 200 && a.K > 200 && flops <= 5e10;
+    const bool matrices = a.m.nd <= 1 && a.n.nd <= 1 && a.k.nd <= 1;   // nothing to permute
+    return !matrices && (rows_x || rows_y) && a.M > 200 && a.N > 200 && a.K > 200 &&
+           flops <= 5e10;
 }
 
 // The contraction through the direct kernels, if they take it.  C must be
