@@ -221,13 +221,20 @@ struct aq_rhfccsd {
     // intermediates, and so on; two products that several intermediates share
     // ("efam,fi" and "nmei,an") are formed once.  A stage is 10 launches instead
     // of 57.  Used while every product is FP64 arithmetic and the doubles have at
-    // most kBatchedDoubles elements, where launches and their latency dominate.
-    static constexpr double kBatchedDoubles = 1.2e6;
+    // most kBatchedDoubles elements: an FP64 iteration takes (general / batched, us)
+    // 1461/1130 at o = 14, v = 85, 2393/2110 at o = 16, v = 100, 4438/4255 at o =
+    // 10, v = 180, and 9161/9308 at o = 20, v = 140, where the general path has the
+    // larger tiles.  A mixed-precision solve whose first iterations run reduced, on
+    // the general path, has few FP64 ones left to gain by and would allocate for
+    // both: kBatchedMixed (a burst of eight jobs, o = 4 to 14: 105 ms so, 135 with
+    // the larger limit).
+    static constexpr double kBatchedDoubles = 3.5e6, kBatchedMixed = 1.2e6;
     std::unique_ptr<StageProgram> program;
     bool program_refused = false;
 
     bool batched(int prec) {
-        if (double(o) * o * v * v > kBatchedDoubles || program_refused) return false;
+        const double most = cfg.precision == AQ_PREC_FP64 ? kBatchedDoubles : kBatchedMixed;
+        if (double(o) * o * v * v > most || program_refused) return false;
         if (!program) {
             if (ctx->capture) return false;   // built on an eager iteration
             build_program();
@@ -344,10 +351,19 @@ struct aq_rhfccsd {
         P.add(0.5, z26);                          // :305
         P.add(-0.5, z27);                         // :306
         P.add(-1.0, z28);                         // :307
-        program_refused = !P.ok();
-        if (program_refused) return;
-        P.finish();
+        // its tiles stay allocated, unlike the operand copies that the general path
+        // keeps: they get half of what the budget leaves beside the DIIS history
+        const double n2 = double(o) * o * v * v, history = 16.0 * std::max(cfg.diis_order, 1) * (n2 + double(o) * v);
+        const double room = 0.5 * (double(ctx->budget) - double(ctx->tensor_bytes + ctx->pool_bytes) - history);
+        program_refused = true;
+        try {
+            if (room <= 0.0 || !P.finish(size_t(room))) return;
+        } catch (const Error& e) {
+            if (e.code != AQ_ERR_OOM) throw;
+            return;
+        }
         program = std::move(p);
+        program_refused = false;
     }
 
     void batched_contractions() {

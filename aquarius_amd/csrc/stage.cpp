@@ -33,14 +33,16 @@ void StageProgram::add_pairs(double coef, int product, bool antisymmetric) {
     outputs_.back().terms.push_back({coef, nullptr, "", product, antisymmetric ? 3 : 2});
 }
 
+constexpr size_t kDescBytes = size_t(1) << 16;   // more than the descriptors take
+
 static uint32_t log2_of(uint32_t x) {
     uint32_t l = 0;
     while ((1u << l) < x) ++l;
     return l;
 }
 
-void StageProgram::finish() {
-    AQ_CHECK(ok_, AQ_ERR_UNSUPPORTED, "contraction not of the batched stage's form");
+bool StageProgram::finish(size_t room) {
+    if (!ok_) return false;   // a contraction not of the batched stage's form
     int nlevels = 0;
     for (const auto& p : products_) nlevels = std::max(nlevels, p.level + 1);
     levels_.assign(size_t(nlevels), Level{});
@@ -58,6 +60,7 @@ void StageProgram::finish() {
         at.push_back(total);
         total += int64_t(p.a.tilesM) * p.a.tilesN * p.a.nsplit * p.a.tm * p.a.tn;
     }
+    if (size_t(total) * 8 + kDescBytes > room) return false;
     tiles_ = tensor::Tensor(ctx_, std::vector<int64_t>{std::max<int64_t>(total, 1)}, false);
     for (size_t k = 0; k < products_.size(); ++k) products_[k].a.P = tiles_.handle()->data + at[k];
 
@@ -154,6 +157,7 @@ void StageProgram::finish() {
         L.outs = reinterpret_cast<const AsmOut*>(dev + f.outs);
         L.terms = reinterpret_cast<const AsmTerm*>(dev + f.terms);
     }
+    return true;
 }
 
 void StageProgram::run() {

@@ -30,9 +30,10 @@ class StageProgram {
     void add(double coef, int product);
     void add_pairs(double coef, int product, bool antisymmetric);   // packed pairs (0,1) and (2,3)
 
-    bool ok() const { return ok_; }
     double largest_flops() const { return largest_; }
-    void finish();        // tiles, buffers, upload (allocates; synchronises)
+    // tiles, buffers, upload (allocates; synchronises); false if the products are
+    // not of the stage's form or its buffers take more than `room` bytes
+    bool finish(size_t room);
     void run();           // every launch on the context's stream
     const std::vector<const tensor::Tensor*>& outputs() const { return written_; }
 

@@ -22,7 +22,7 @@ NAMES = ("FAE", "FMI", "FME", "WMNIJ", "WMNEJ", "WAMIJ", "WAMEI", "WAMIE", "T1",
 @pytest.mark.parametrize("precision", ["fp64", "bf16x3"])   # bf16x3: every product is below min_reduced_flops
 @pytest.mark.parametrize("o,v,symmetric", [
     (1, 1, True), (1, 2, True), (2, 1, True), (1, 17, True), (3, 16, True), (4, 17, False), (5, 19, True),
-    (7, 33, True), (8, 32, False), (15, 31, True), (16, 16, True), (3, 65, True), (17, 64, True), (17, 65, True)])
+    (7, 33, True), (8, 32, False), (15, 31, True), (16, 16, True), (3, 65, True), (17, 64, True), (19, 98, True), (20, 94, True)])
 def test_stage_matches_oracle(o, v, symmetric, precision):
     seed, nQ = 100 * o + v, o + v + 3
     print(f"case: stage o={o} v={v} symmetric={symmetric} {precision}", flush=True)
@@ -45,3 +45,31 @@ def test_stage_matches_oracle(o, v, symmetric, precision):
                                            atol=tol * max(1.0, np.abs(want).max()), err_msg=f"{name} {it}")
         cc.close()
         ints.free()
+
+
+@pytest.mark.parametrize("spare", [16, 32, 256])
+def test_tight_budget(spare):
+    """`spare` doubles tensors beyond the solver and its DIIS history: too few
+    for the batched stage's buffers (the first two) the iteration runs with
+    evictable operand copies, to the same energy."""
+    o, v, order = 6, 30, 4
+    print(f"case: stage budget {spare}", flush=True)
+    eps, B = aq.synth_host(9, o, v, 40)
+    f, V = synth.fock(eps[:o], eps[o:]), synth.blocks_from_B(B, o)
+    cfg = rhfccsd.default_config()
+    cfg["diis"]["order"] = order
+    ref = rhfccsd.RHFCCSD(f, V, cfg)
+    held = 0
+    for bounded in (False, True):
+        with aq.Context(hbm_budget=held + (2 * order + spare) * 8 * (o * v) ** 2 if bounded else 0) as ctx:
+            ints = aq.Integrals.from_numpy(ctx, f, V)
+            cc = aq.RHFCCSD(ctx, ints, diis_order=order)
+            if not bounded:
+                held = ctx.memory()[0]
+            else:
+                for _ in range(6):
+                    e, _ = cc.iterate()
+                    ref.iterate()
+                assert abs(e - ref.energy) <= 1e-9 * abs(ref.energy)
+            cc.close()
+            ints.free()
