@@ -400,6 +400,10 @@ static bool digits_of(const std::string& order, const Labeled& X, const Labeled&
 //    partials): 110 x 110 x 21560 50/32, 140 x 20 x 392000 244/160;
 //  - a short side and a short inner extent against a long side: 140 x 56000 x
 //    140 111/81;
+//  - at most 32 columns and a short inner extent against a very long side, rows
+//    contiguous in A and C: the GEMM's narrowest wide tile, 128 x 64, multiplies
+//    up to twice the columns, 256 x 32 from registers does not (392000 x 20 x 140
+//    171/132, 607500 x 27 x 150 322/250, 1179648 x 32 x 192 699/556);
 //  - large products whose GEMM would have to permute: 975^3 72/64, 1600^3
 //    226/203, 2800^3 950/840 (both operands strided, amplitudes permuted anew);
 //    beyond, permuting costs less than the LDS tiles lose to the GEMM's (3080^3
@@ -412,6 +416,7 @@ static bool direct_size(const DirectArgs& a, bool scattered, bool rows_x, bool r
     if (a.N == 1 && !rows_x && sizeX > 8000000) return false;
     if (flops <= 6e8) return true;
     if (out <= 2.5e4) return flops <= 2e10;
+    if (a.N <= 32 && a.K <= 512 && rows_x && !scattered && double(a.M) >= 1000.0 * a.N) return flops <= 1e11;
     if (a.M <= 200 && a.K <= 200 && double(a.N) >= 50.0 * a.M) return flops <= 2e10;
     const bool matrices = a.m.nd <= 1 && a.n.nd <= 1 && a.k.nd <= 1;   // nothing to permute
     return !matrices && (rows_x || rows_y) && a.M > 200 && a.N > 200 && a.K > 200 &&

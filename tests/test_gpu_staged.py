@@ -1,5 +1,5 @@
 """FP64 contractions large enough for the tiles staged through LDS (64 x 64 and
-128 x 128), straight from labelled layouts: each operand contiguous along its
+128 x 128) and for the 256 x 32 tiles of a few columns, straight from labelled layouts: each operand contiguous along its
 rows or along k, digits that do not merge, partial tiles, partial chunks of 16
 k, several tables of 512 k, split inner extents, a batch label.  Reference:
 numpy.  Each element is within the bound of a sum of K rounded products in any
@@ -57,6 +57,14 @@ def test_rings(ctx, form, o, v, beta):
 def test_around_the_edges(ctx, form, M, N, K):
     print(f"case: staged edges {form} {M} {N} {K}", flush=True)
     check(ctx, form, {"m": M // 3 + 1, "x": 3, "n": N // 2 + 1, "y": 2, "k": K, "z": 2}, -1.0, 0.25)
+
+
+@pytest.mark.parametrize("beta", [0.0, 1.0])
+@pytest.mark.parametrize("o,v", [(17, 130), (20, 97), (27, 61), (31, 90), (32, 64), (33, 70)])
+@pytest.mark.parametrize("form", ["abej,ei,abij", "abej,ie,abij"])
+def test_few_columns(ctx, form, o, v, beta):
+    print(f"case: few columns {form} o={o} v={v} beta={beta}", flush=True)
+    check(ctx, form, {c: v if c < "i" else o for c in form if c != ","}, 1.0, beta)
 
 
 def test_batch_label(ctx):
