@@ -76,7 +76,7 @@ int aq_ctx_sync(aq_ctx* ctx);
 int aq_ctx_set_precision(aq_ctx* ctx, int precision, double min_reduced_flops);
 int aq_ctx_get_precision(const aq_ctx* ctx, int* precision);
 /* Kernel variant of the large-tile GEMM for one arithmetic (AQ_PREC_*):
- * -1 = library default (or the autotuner's choice), FP64/FP32: 0 = BK 16,
+ * -1 = library default (by the shape; or the autotuner's choice), FP64/FP32: 0 = BK 16,
  * 1 = BK 32, 2 = BK 16 with two waves per SIMD; BF16x3: 0 = 128x128 blocks,
  * 1 = 256x128, 2 = 128x256, 3 = 256x256 with eight waves (two per SIMD),
  * 4 = 256x256 with four waves.
@@ -559,7 +559,8 @@ int aq_server_drain(aq_server* s);
 int aq_server_stats_get(aq_server* s, aq_server_stats* out);
 /* Cross-job GEMM grouping (the serving loop's grouped launch; no reference
  * counterpart).  window_us > 0: the slots' eager GEMMs with 128x128 or 64x64
- * FP64/BF16x3 blocks are merged, across jobs, into one persistent grouped
+ * FP64/BF16x3 blocks (and, one launch each way, their direct FP64 contractions
+ * and the levels of their small iterations' batched stages) are merged, across jobs, into one persistent grouped
  * kernel launch per (format, operand layout, block) key: a fixed grid of
  * resident blocks walks the tiles of every member GEMM.  A GEMM joins
  * same-key GEMMs that other slots have pending; with none pending, and
