@@ -719,6 +719,7 @@ __global__ __launch_bounds__(256, 3) void k_stage(StageGroup G) {
     switch (g.config >> 2) {
         case 0: stage_tile<1, 1, 1, 1, 4, 3>(g, id, lds); break;
         case 1: stage_tile<2, 2, 1, 1, 4, 2>(g, id, lds); break;
+        case 3: stage_tile<4, 1, 1, 1, 4, 2>(g, id, lds); break;
         default:
             switch (g.config & 3) {
                 case 0: staged_tile<2, false, false, true>(g, id, lds); break;
@@ -842,7 +843,8 @@ void launch_assemble(hipStream_t s, const AsmOut* outs, const AsmTerm* terms, in
 // of those; the T that gives the shortest level is kept.  A chunk of a block
 // alone takes about 2000 cycles in every tile; a model without that left K =
 // 5625 unsplit and its 264 us set the length of the level (o = 13, v = 75: 410 us
-// against 322).
+// against 322).  The thin products take 64 x 16 tiles (304 us; with 64 x 64 for
+// 13 columns 322).
 void plan_stage_level(DirectArgs* const* a, int n) {
     struct Option {
         int cfg;
@@ -855,7 +857,7 @@ void plan_stage_level(DirectArgs* const* a, int n) {
     std::vector<std::vector<Option>> opts(static_cast<size_t>(n));
     double lo = 1e300, hi = 0.0;
     for (int i = 0; i < n; ++i) {
-        for (int c : {0, 1, 3}) {
+        for (int c : {0, 1, 3, 4}) {
             const DirCfg& f = kDirCfg[c];
             const double chunks = std::ceil(a[i]->K / 16.0);
             const double tiles = double((a[i]->M + f.tm() - 1) / f.tm()) * double((a[i]->N + f.tn() - 1) / f.tn());
@@ -902,7 +904,7 @@ void plan_stage_level(DirectArgs* const* a, int n) {
         p.kchunk = ((p.K + 15) / 16 + x->nsplit - 1) / x->nsplit * 16;
         p.nsplit = (p.K + p.kchunk - 1) / p.kchunk;
         for (DirDigits* d : {&p.m, &p.n, &p.k}) set_dividers(*d);
-        const uint32_t shape = x->cfg == 3 ? 2 : uint32_t(x->cfg);   // k_stage's shapes: 16, 32, 64
+        const uint32_t shape = x->cfg == 3 ? 2 : x->cfg == 4 ? 3 : uint32_t(x->cfg);   // k_stage's shapes: 16, 32, 64, 64 x 16
         p.config = shape * 4 + (k_layout(f, p.k, p.k.s0) ? 1 : 0) + (k_layout(f, p.k, p.k.s1) ? 2 : 0);
         p.tm = uint32_t(f.tm());
         p.tn = uint32_t(f.tn());
