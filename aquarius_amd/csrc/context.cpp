@@ -2,6 +2,7 @@
 // Replaces the role of Aquarius's Arena (src/util/distributed.hpp:28-74): the
 // place every tensor of one job lives.  One context = one HIP stream; nothing
 // here is global, so contexts on one device are independent.
+#include "blocks.hpp"
 #include "internal.hpp"
 
 #include <atomic>
@@ -26,93 +27,139 @@ size_t ctx_in_use(const aq_ctx* ctx) { return ctx->tensor_bytes + ctx->pool_byte
 // (36 to 46 ms per release here, twice in a burst of eight small jobs), and
 // every job's end frees nearly all it had.  Safe across the slots' streams: a
 // block carries an event recorded behind its last use, and a request from
-// another stream waits for it.  Bounded: beyond `limit` the oldest blocks go
-// back; a failed allocation and the server's end give everything back.
+// another stream waits for it.  Bounded by the server's budget (BlockLedger):
+// what does not fit beside the running jobs' reservations goes to the device
+// pool, oldest first.
 struct BlockCache {
-    struct Block {
-        void* p;
-        size_t bytes;
-        hipStream_t stream;
-        hipEvent_t freed;
-    };
+    int device = 0;
     std::mutex mu;
-    std::list<Block> kept;                           // oldest first
-    std::unordered_map<void*, size_t> given;         // blocks in use
+    BlockLedger led;
     std::vector<hipEvent_t> spare;
-    size_t bytes = 0, limit = 0;
 
     void* take(size_t n, hipStream_t stream) {
         std::lock_guard<std::mutex> lk(mu);
-        auto best = kept.end();
-        for (auto it = kept.begin(); it != kept.end(); ++it)   // at most an eighth wasted
-            if (it->bytes >= n && it->bytes - n <= n / 8 && (best == kept.end() || it->bytes < best->bytes)) best = it;
-        if (best == kept.end()) return nullptr;
-        if (best->stream != stream && hipStreamWaitEvent(stream, best->freed, 0) != hipSuccess) {
+        BlockLedger::Block b;
+        if (!led.take(n, b)) return nullptr;
+        const hipEvent_t freed = static_cast<hipEvent_t>(b.freed);
+        if (b.stream != stream && hipStreamWaitEvent(stream, freed, 0) != hipSuccess) {
             (void)hipGetLastError();
-            return nullptr;
+            (void)hipEventSynchronize(freed);   // a wait that cannot be queued is made on the host
         }
-        void* p = best->p;
-        given[p] = best->bytes;
-        bytes -= best->bytes;
-        spare.push_back(best->freed);
-        kept.erase(best);
-        return p;
+        recycle(freed);
+        return b.p;
     }
-    void note(void* p, size_t n) {
+    void note(void* p, size_t n) noexcept {
         std::lock_guard<std::mutex> lk(mu);
-        given[p] = n;
+        try {
+            led.lend(p, n, n);
+        } catch (...) {   // no host memory: not tracked, and freed as any other block
+        }
     }
-    // false: not one of ours (the caller frees it)
-    bool give(void* p, hipStream_t stream) {
+    // false: not kept (the caller frees it); pooled: the device pool got older blocks instead
+    bool give(void* p, hipStream_t stream, bool& pooled) noexcept {
         std::lock_guard<std::mutex> lk(mu);
-        auto it = given.find(p);
-        if (it == given.end()) return false;
-        Block b{p, it->second, stream, nullptr};
-        given.erase(it);
-        if (b.bytes > limit) return false;
-        if (!spare.empty()) {
-            b.freed = spare.back();
-            spare.pop_back();
-        } else if (hipEventCreateWithFlags(&b.freed, hipEventDisableTiming) != hipSuccess) {
-            (void)hipGetLastError();
+        hipEvent_t e = nullptr;
+        try {
+            const size_t bytes = led.back(p);
+            if (bytes == 0 || !led.fits(bytes)) return false;
+            if (!spare.empty()) {
+                e = spare.back();
+                spare.pop_back();
+            } else if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+                (void)hipGetLastError();
+                return false;
+            }
+            if (hipEventRecord(e, stream) != hipSuccess) {
+                (void)hipGetLastError();
+                (void)hipEventDestroy(e);
+                return false;
+            }
+            led.keep({p, bytes, stream, e});
+        } catch (...) {   // no host memory for the bookkeeping
+            if (e) (void)hipEventDestroy(e);
             return false;
         }
-        if (hipEventRecord(b.freed, stream) != hipSuccess) {
-            (void)hipGetLastError();
-            spare.push_back(b.freed);
-            return false;
-        }
-        kept.push_back(b);
-        bytes += b.bytes;
-        while (bytes > limit) release_oldest(stream);
+        pooled = pooled || led.over();
+        while (led.over()) release_oldest(stream);
         return true;
     }
-    void release_oldest(hipStream_t stream) {        // mu held
-        const Block b = kept.front();
-        kept.pop_front();
-        bytes -= b.bytes;
-        // a wait that cannot be queued is made on the host
-        if (b.stream != stream && hipStreamWaitEvent(stream, b.freed, 0) != hipSuccess) (void)hipEventSynchronize(b.freed);
-        (void)hipFreeAsync(b.p, stream);
-        spare.push_back(b.freed);
-    }
-    void flush(hipStream_t stream) {
+    void set_limit(size_t bytes) {
         std::lock_guard<std::mutex> lk(mu);
-        while (!kept.empty()) release_oldest(stream);
+        led.limit = bytes;
+    }
+    size_t slack() {
+        std::lock_guard<std::mutex> lk(mu);
+        return led.slack();
+    }
+    // Kept blocks beyond the limit (all: every kept block) to the device pool.
+    void release(hipStream_t stream, bool all, bool& pooled) {
+        std::lock_guard<std::mutex> lk(mu);
+        while (all ? !led.empty() : led.over()) {
+            release_oldest(stream);
+            pooled = true;
+        }
     }
     ~BlockCache() {
-        flush(nullptr);
+        bool pooled = false;
+        release(nullptr, true, pooled);
         (void)hipStreamSynchronize(nullptr);
         for (auto e : spare) (void)hipEventDestroy(e);
     }
+
+  private:
+    void recycle(hipEvent_t e) noexcept {            // mu held
+        try {
+            spare.push_back(e);
+        } catch (...) {
+            (void)hipEventDestroy(e);
+        }
+    }
+    void release_oldest(hipStream_t stream) noexcept {   // mu held
+        const BlockLedger::Block b = led.pop_oldest();
+        const hipEvent_t freed = static_cast<hipEvent_t>(b.freed);
+        // a wait that cannot be queued is made on the host
+        if (b.stream != stream && hipStreamWaitEvent(stream, freed, 0) != hipSuccess) {
+            (void)hipGetLastError();
+            (void)hipEventSynchronize(freed);
+        }
+        (void)hipFreeAsync(b.p, stream);
+        recycle(freed);
+    }
 };
 
-BlockCache* block_cache_create(size_t limit) {
+BlockCache* block_cache_create(int device) {
     auto* c = new BlockCache();
-    c->limit = limit;
+    c->device = device;
     return c;
 }
 void block_cache_destroy(BlockCache* c) { delete c; }
+void block_cache_limit(BlockCache* c, size_t bytes) { c->set_limit(bytes); }
+size_t block_cache_slack(BlockCache* c) { return c->slack(); }
+
+// A job starts: kept blocks that its reservation displaces go, and so do all of
+// them where the device runs short for what the runtime allocates by itself
+// (the scratch of a queue's first spilling kernel: up to 0.2 GB a queue, and
+// the queue aborts without it).
+void block_cache_settle(aq_ctx* ctx) {
+    constexpr size_t kDeviceReserve = size_t(4) << 30;
+    ctx->blocks->release(ctx->stream, false, ctx->pooled);
+    size_t free_b = 0, total_b = 0;
+    if (hipMemGetInfo(&free_b, &total_b) == hipSuccess && free_b < kDeviceReserve) {
+        ctx->blocks->release(ctx->stream, true, ctx->pooled);
+        (void)hipStreamSynchronize(ctx->stream);
+        trim_device_pool(ctx->device);   // also what other contexts left there
+    }
+    (void)hipGetLastError();
+    block_cache_trim(ctx);
+}
+
+// What the device pool got from this slot, back to the driver.
+void block_cache_trim(aq_ctx* ctx) {
+    if (!ctx->pooled) return;
+    ctx->pooled = false;
+    (void)hipStreamSynchronize(ctx->stream);   // the frees are complete
+    trim_device_pool(ctx->device);
+}
 
 // Stream-ordered device memory: allocations and frees are ordered on the
 // context's stream, so one context releasing memory never synchronises the
@@ -131,7 +178,12 @@ void* dmalloc(aq_ctx* ctx, size_t bytes) {
 
 void dfree(aq_ctx* ctx, void* p) {
     if (p) {
-        if (!ctx->blocks || !ctx->blocks->give(p, ctx->stream)) (void)hipFreeAsync(p, ctx->stream);
+        if (!ctx->blocks) {
+            (void)hipFreeAsync(p, ctx->stream);
+        } else if (!ctx->blocks->give(p, ctx->stream, ctx->pooled)) {
+            (void)hipFreeAsync(p, ctx->stream);
+            ctx->pooled = true;
+        }
         ctx->mem_gen += 1;
     }
 }
@@ -141,7 +193,9 @@ void dfree(aq_ctx* ctx, void* p) {
 // driver.  The pool keeps freed blocks between synchronisations (release
 // threshold at its maximum), which is what makes repeated allocation cheap
 // within a job; across jobs of different sizes those cached blocks can be
-// the wrong shapes for the next request, so they are trimmed before an
+// the wrong shapes for the next request, and memory that sits there is missing
+// to everything else on the device, the runtime's own allocations among it.
+// They are trimmed when a served job ends, when a server starts and before an
 // allocation is retried.
 void trim_device_pool(int device) {
     hipMemPool_t pool;
@@ -206,13 +260,13 @@ static void* raw_alloc(aq_ctx* ctx, size_t bytes) {
         // giving up any cached operand copy.
         const auto t0 = std::chrono::steady_clock::now();
         pool_release_all(ctx);
-        if (ctx->blocks) ctx->blocks->flush(ctx->stream);
+        if (ctx->blocks) ctx->blocks->release(ctx->stream, true, ctx->pooled);
         AQ_HIP(hipStreamSynchronize(ctx->stream));
         trim_device_pool(ctx->device);
         p = dmalloc(ctx, bytes);
         if (!p) {
             evict_cache(ctx, ctx->budget);   // drop every cached copy
-            if (ctx->blocks) ctx->blocks->flush(ctx->stream);
+            if (ctx->blocks) ctx->blocks->release(ctx->stream, true, ctx->pooled);
             AQ_HIP(hipStreamSynchronize(ctx->stream));
             trim_device_pool(ctx->device);
             p = dmalloc(ctx, bytes);
@@ -273,7 +327,6 @@ void drop_caches(aq_ctx* ctx) {
     ctx->cache_lru.clear();
     ctx->cache_bytes = 0;
 }
-
 
 // ---------------------------------------------------------------- timing
 
@@ -460,7 +513,6 @@ int aq_ctx_trim(aq_ctx* ctx) {
         AQ_CHECK(ctx, AQ_ERR_INVALID, "null context");
         AQ_HIP(hipStreamSynchronize(ctx->stream));
         drop_caches(ctx);
-        if (ctx->blocks) return;   // a server's slot: for its next jobs
         AQ_HIP(hipStreamSynchronize(ctx->stream));
         trim_device_pool(ctx->device);
     });

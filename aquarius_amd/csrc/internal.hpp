@@ -143,6 +143,7 @@ struct aq_ctx {
 
     // freed blocks shared with a server's other slots (null: the device pool's)
     aqamd::BlockCache* blocks = nullptr;
+    bool pooled = false;            // some went to the device pool since it was trimmed
 
     // reductions
     double* d_partials = nullptr;   // device: kRedSlots slots x kRedPartials partials
@@ -184,10 +185,14 @@ size_t ctx_in_use(const aq_ctx* ctx);
 void evict_cache(aq_ctx* ctx, size_t need);
 void drop_caches(aq_ctx* ctx);                       // operand copies and pooled scratch back to the allocator
 void trim_device_pool(int device);                   // the device pool's unused memory back to the driver
-// a server's freed blocks, kept for its next jobs (at most `limit` bytes); its
-// contexts are destroyed before it
-BlockCache* block_cache_create(size_t limit);
+// a server's freed blocks, kept for its next jobs (at most `bytes` of them, with
+// what reused blocks are larger than asked for); its contexts are destroyed before it
+BlockCache* block_cache_create(int device);
 void block_cache_destroy(BlockCache* c);
+void block_cache_limit(BlockCache* c, size_t bytes);
+size_t block_cache_slack(BlockCache* c);
+void block_cache_settle(aq_ctx* ctx);                // a job starts on this slot: back within the limit
+void block_cache_trim(aq_ctx* ctx);                  // its memory is freed: what was not kept goes to the driver
 void invalidate_cache(aq_ctx* ctx);                  // every cached copy must be rebuilt before use
 void noalloc_scratch_init(int device);               // noalloc.cpp: resolve the fixed device array once per device
 

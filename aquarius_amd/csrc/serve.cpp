@@ -6,7 +6,9 @@
 // budget when admitted and releases them when it finishes; admission scans
 // the queue in arrival order and starts the first job that fits (backfill),
 // except that once the oldest queued job has waited longer than
-// max_bypass_s no later job may overtake it.  Jobs run to convergence with
+// max_bypass_s no later job may overtake it.  Finished jobs leave their memory to
+// the next ones as far as the budget has room beside the reservations, and the
+// rest to the driver.  Jobs run to convergence with
 // their integrals, amplitudes and DIIS history resident on the device; their
 // kernels overlap on the GPU through the per-slot streams (and, with grouping
 // on, same-key GEMMs of different jobs run as one grouped launch on the
@@ -77,9 +79,11 @@ struct aq_server {
         const int64_t head = queue.front();
         const Job& hj = jobs[head];
         const bool head_blocked = now() - hj.t_queued > max_bypass_s;
+        // blocks in use that are larger than what was asked for count as well
+        const size_t held = reserved ? reserved + block_cache_slack(blocks) : 0;
         for (int64_t id : queue) {
             const Job& j = jobs[id];
-            if (reserved + j.res.bytes_reserved <= budget) return id;
+            if (held + j.res.bytes_reserved <= budget) return id;
             if (head_blocked) return -1;   // the oldest job must go first
         }
         return -1;
@@ -102,10 +106,13 @@ struct aq_server {
             if (mo) aq_tensor_destroy(mo);
             for (auto* t : ints)
                 if (t) aq_tensor_destroy(t);
-            // the job's memory goes to the server's block cache, for the next job
+            // the job's memory goes to the server's block cache, for the next job;
+            // what the budget does not leave room for goes back to the driver
             (void)hipStreamSynchronize(ctx->stream);
             drop_caches(ctx);
+            block_cache_trim(ctx);
         };
+        block_cache_settle(ctx);
         try {
             if (!job.inputs.empty()) {
                 use = job.inputs.data();
@@ -130,6 +137,7 @@ struct aq_server {
                 tensor::check(aq_synth_host(s.seed, s.o, s.v, nQ, s.sigma, eps.data(), B.data()));
                 tensor::check(aq_synth_build(ctx, s.o, s.v, nQ, eps.data(), B.data(), ints));
             }
+            block_cache_trim(ctx);   // what building the integrals freed: up to v^4 doubles
             tensor::check(aq_rhfccsd_create(ctx, use, use + 3, &s.cfg, &cc));
             job.res.mp2 = 0.0;
             tensor::check(aq_rhfccsd_mp2(cc, &job.res.mp2));
@@ -162,6 +170,7 @@ struct aq_server {
                 Job& j = jobs[id];
                 queue.erase(std::find(queue.begin(), queue.end(), id));
                 reserved += j.res.bytes_reserved;
+                block_cache_limit(blocks, budget - reserved);
                 j.res.status = AQ_JOB_RUNNING;
                 j.res.slot = slot;
                 j.res.t_start = now();
@@ -192,6 +201,7 @@ struct aq_server {
                 j.res = local.res;
                 j.res.t_end = now();
                 reserved -= j.res.bytes_reserved;
+                block_cache_limit(blocks, budget - reserved);
                 running -= 1;
                 if (code == AQ_OK) {
                     j.res.status = AQ_JOB_DONE;
@@ -254,11 +264,13 @@ int aq_server_create(int device, size_t hbm_budget, int slots, double max_bypass
                 s->ctxs.push_back(c);
                 tensor::check(aq_ctx_set_autotune(c, 1));
             }
+            trim_device_pool(device);   // what earlier contexts freed
             size_t free_b = 0, total_b = 0;
             AQ_HIP(hipMemGetInfo(&free_b, &total_b));
-            s->blocks = block_cache_create(total_b / 8);
+            s->blocks = block_cache_create(device);
             for (auto* c : s->ctxs) c->blocks = s->blocks;
             s->budget = hbm_budget ? std::min(hbm_budget, size_t(0.95 * double(free_b))) : size_t(0.9 * double(free_b));
+            block_cache_limit(s->blocks, s->budget);
             for (int i = 0; i < slots; ++i) s->workers.emplace_back([s, i] { s->worker(i); });
         } catch (...) {
             for (auto* c : s->ctxs) aq_ctx_destroy(c);
