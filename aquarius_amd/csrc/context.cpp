@@ -12,6 +12,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
 #include <mutex>
 
 namespace aqamd {
@@ -91,6 +92,10 @@ struct BlockCache {
         std::lock_guard<std::mutex> lk(mu);
         return led.slack();
     }
+    size_t kept() {
+        std::lock_guard<std::mutex> lk(mu);
+        return led.kept();
+    }
     // Kept blocks beyond the limit (all: every kept block) to the device pool.
     void release(hipStream_t stream, bool all, bool& pooled) {
         std::lock_guard<std::mutex> lk(mu);
@@ -127,17 +132,44 @@ struct BlockCache {
     }
 };
 
-BlockCache* block_cache_create(int device) {
-    auto* c = new BlockCache();
-    c->device = device;
-    return c;
+// Every server's cache: a context that runs short of memory, or is trimmed,
+// takes back what servers on its device keep.  Locked before a cache's own mutex.
+static std::mutex g_caches_mu;
+static std::vector<BlockCache*> g_caches;
+
+size_t kept_bytes(int device) {
+    std::lock_guard<std::mutex> lk(g_caches_mu);
+    size_t n = 0;
+    for (auto* c : g_caches)
+        if (c->device == device) n += c->kept();
+    return n;
 }
-void block_cache_destroy(BlockCache* c) { delete c; }
+
+static void release_kept_blocks(aq_ctx* ctx) {
+    std::lock_guard<std::mutex> lk(g_caches_mu);
+    for (auto* c : g_caches)
+        if (c->device == ctx->device) c->release(ctx->stream, true, ctx->pooled);
+}
+
+BlockCache* block_cache_create(int device) {
+    std::unique_ptr<BlockCache> c(new BlockCache());
+    c->device = device;
+    std::lock_guard<std::mutex> lk(g_caches_mu);
+    g_caches.push_back(c.get());
+    return c.release();
+}
+void block_cache_destroy(BlockCache* c) {
+    {
+        std::lock_guard<std::mutex> lk(g_caches_mu);
+        g_caches.erase(std::remove(g_caches.begin(), g_caches.end(), c), g_caches.end());
+    }
+    delete c;
+}
 void block_cache_limit(BlockCache* c, size_t bytes) { c->set_limit(bytes); }
 size_t block_cache_slack(BlockCache* c) { return c->slack(); }
 
-// A job starts: kept blocks that its reservation displaces go, and so do all of
-// them where the device runs short for what the runtime allocates by itself
+// A job starts: kept blocks that its reservation displaces go, and so do all
+// servers' where the device runs short for what the runtime allocates by itself
 // (the scratch of a queue's first spilling kernel: up to 0.2 GB a queue, and
 // the queue aborts without it).
 void block_cache_settle(aq_ctx* ctx) {
@@ -145,7 +177,7 @@ void block_cache_settle(aq_ctx* ctx) {
     ctx->blocks->release(ctx->stream, false, ctx->pooled);
     size_t free_b = 0, total_b = 0;
     if (hipMemGetInfo(&free_b, &total_b) == hipSuccess && free_b < kDeviceReserve) {
-        ctx->blocks->release(ctx->stream, true, ctx->pooled);
+        release_kept_blocks(ctx);
         (void)hipStreamSynchronize(ctx->stream);
         trim_device_pool(ctx->device);   // also what other contexts left there
     }
@@ -256,17 +288,18 @@ static void* raw_alloc(aq_ctx* ctx, size_t bytes) {
     void* p = dmalloc(ctx, bytes);
     if (!p) {
         // The device pool holds freed blocks of other sizes (and other contexts'
-        // memory): hand the unused blocks back to the driver and retry before
-        // giving up any cached operand copy.
+        // memory), and servers keep finished jobs' blocks: hand the unused
+        // memory back to the driver and retry before giving up any cached
+        // operand copy.
         const auto t0 = std::chrono::steady_clock::now();
         pool_release_all(ctx);
-        if (ctx->blocks) ctx->blocks->release(ctx->stream, true, ctx->pooled);
+        release_kept_blocks(ctx);
         AQ_HIP(hipStreamSynchronize(ctx->stream));
         trim_device_pool(ctx->device);
         p = dmalloc(ctx, bytes);
         if (!p) {
             evict_cache(ctx, ctx->budget);   // drop every cached copy
-            if (ctx->blocks) ctx->blocks->release(ctx->stream, true, ctx->pooled);
+            release_kept_blocks(ctx);
             AQ_HIP(hipStreamSynchronize(ctx->stream));
             trim_device_pool(ctx->device);
             p = dmalloc(ctx, bytes);
@@ -410,6 +443,7 @@ int aq_ctx_create(int device, size_t hbm_budget, aq_ctx** out) {
             AQ_HIP(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
             size_t free_b = 0, total_b = 0;
             AQ_HIP(hipMemGetInfo(&free_b, &total_b));
+            free_b += kept_bytes(device);   // given up on request
             ctx->budget = hbm_budget ? hbm_budget : static_cast<size_t>(0.9 * double(free_b));
             ctx->d_partials = static_cast<double*>(dmalloc(ctx, sizeof(double) * kRedSlots * kRedPartials));
             AQ_CHECK(ctx->d_partials, AQ_ERR_OOM, "device allocation of reduction slots failed");
@@ -513,6 +547,7 @@ int aq_ctx_trim(aq_ctx* ctx) {
         AQ_CHECK(ctx, AQ_ERR_INVALID, "null context");
         AQ_HIP(hipStreamSynchronize(ctx->stream));
         drop_caches(ctx);
+        release_kept_blocks(ctx);
         AQ_HIP(hipStreamSynchronize(ctx->stream));
         trim_device_pool(ctx->device);
     });

@@ -191,6 +191,7 @@ BlockCache* block_cache_create(int device);
 void block_cache_destroy(BlockCache* c);
 void block_cache_limit(BlockCache* c, size_t bytes);
 size_t block_cache_slack(BlockCache* c);
+size_t kept_bytes(int device);                       // what all servers on the device keep
 void block_cache_settle(aq_ctx* ctx);                // a job starts on this slot: back within the limit
 void block_cache_trim(aq_ctx* ctx);                  // its memory is freed: what was not kept goes to the driver
 void invalidate_cache(aq_ctx* ctx);                  // every cached copy must be rebuilt before use

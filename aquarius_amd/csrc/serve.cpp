@@ -61,7 +61,8 @@ struct aq_server {
     std::vector<aq_ctx*> ctxs;
     GemmBatcher* batcher = nullptr;   // cross-job GEMM grouping (null: off)
     std::vector<std::thread> workers;
-    BlockCache* blocks = nullptr;     // memory kept between jobs
+    BlockCache* blocks = nullptr;     // memory kept between jobs,
+    size_t keep = 0;                  // at most so much of it
     std::mutex mu;
     std::condition_variable cv_work, cv_done;
     std::deque<int64_t> queue;
@@ -72,6 +73,9 @@ struct aq_server {
     std::chrono::steady_clock::time_point t0 = std::chrono::steady_clock::now();
 
     double now() const { return std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count(); }
+
+    // What may be kept beside the running jobs (mu held).
+    void limit_kept() { block_cache_limit(blocks, std::min(keep, budget - reserved)); }
 
     // Pick the next admissible job (mu held); -1 if none.
     int64_t pick() {
@@ -170,7 +174,7 @@ struct aq_server {
                 Job& j = jobs[id];
                 queue.erase(std::find(queue.begin(), queue.end(), id));
                 reserved += j.res.bytes_reserved;
-                block_cache_limit(blocks, budget - reserved);
+                limit_kept();
                 j.res.status = AQ_JOB_RUNNING;
                 j.res.slot = slot;
                 j.res.t_start = now();
@@ -201,7 +205,7 @@ struct aq_server {
                 j.res = local.res;
                 j.res.t_end = now();
                 reserved -= j.res.bytes_reserved;
-                block_cache_limit(blocks, budget - reserved);
+                limit_kept();
                 running -= 1;
                 if (code == AQ_OK) {
                     j.res.status = AQ_JOB_DONE;
@@ -267,10 +271,12 @@ int aq_server_create(int device, size_t hbm_budget, int slots, double max_bypass
             trim_device_pool(device);   // what earlier contexts freed
             size_t free_b = 0, total_b = 0;
             AQ_HIP(hipMemGetInfo(&free_b, &total_b));
+            free_b += kept_bytes(device);
+            s->keep = total_b / 8;
             s->blocks = block_cache_create(device);
             for (auto* c : s->ctxs) c->blocks = s->blocks;
             s->budget = hbm_budget ? std::min(hbm_budget, size_t(0.95 * double(free_b))) : size_t(0.9 * double(free_b));
-            block_cache_limit(s->blocks, s->budget);
+            s->limit_kept();
             for (int i = 0; i < slots; ++i) s->workers.emplace_back([s, i] { s->worker(i); });
         } catch (...) {
             for (auto* c : s->ctxs) aq_ctx_destroy(c);

@@ -63,3 +63,16 @@ def test_server_returns_what_earlier_contexts_freed(before):
             assert before - free() <= (3 << 30) + OVERHEAD
             s.drain()
         kept.free()
+
+
+def test_trim_of_another_context_takes_back_what_a_server_keeps(before):
+    print("case: trim beside an idle server", flush=True)
+    with aq.Context() as ctx, aq.Server(slots=2, hbm_budget=24 << 30) as s:
+        serve(s, SIZES)
+        s.drain()
+        assert before - free() > 2 * OVERHEAD    # kept for the next jobs
+        with aq.Context() as other:              # its default budget: nine tenths of what it can get
+            assert other.memory()[1] >= 0.9 * (before - OVERHEAD)
+        ctx.trim()
+        assert before - free() <= OVERHEAD
+        serve(s, SIZES[:3])                      # and the server goes on
