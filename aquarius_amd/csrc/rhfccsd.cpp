@@ -133,6 +133,7 @@ struct aq_rhfccsd {
     // <ab|ef> = <ba|fe> and <ab|ij> = <ba|ji> (so Tau(ef,ij) = Tau(fe,ji)).
     void derive_packed() {
         program.reset();   // holds addresses of the packed operators
+        program_flops = -1.0;
         packed = false;
         if (cfg.packed_ladder && o >= 2 && v >= 2) {
             launch_pair_asymmetry(ctx, dptr(VABCD), v, v, 0);
@@ -231,21 +232,26 @@ struct aq_rhfccsd {
     static constexpr double kBatchedDoubles = 3.5e6, kBatchedMixed = 1.2e6;
     std::unique_ptr<StageProgram> program;
     bool program_refused = false;
+    double program_flops = -1.0;   // of its largest product (-1: not known yet)
 
     bool batched(int prec) {
         const double most = cfg.precision == AQ_PREC_FP64 ? kBatchedDoubles : kBatchedMixed;
         if (double(o) * o * v * v > most || program_refused) return false;
+        // a phase of reduced arithmetic that cannot use it allocates nothing for it
+        if (prec != AQ_PREC_FP64 && program_flops >= cfg.min_reduced_flops) return false;
         if (!program) {
             if (ctx->capture) return false;   // built on an eager iteration
-            build_program();
-            if (!program) return false;
+            std::unique_ptr<StageProgram> p(new StageProgram(ctx));
+            describe(*p);
+            program_flops = p->largest_flops();
+            if (prec != AQ_PREC_FP64 && program_flops >= cfg.min_reduced_flops) return false;
+            finish_program(std::move(p));
         }
-        return prec == AQ_PREC_FP64 || program->largest_flops() < cfg.min_reduced_flops;
+        return program != nullptr;
     }
 
-    void build_program() {
-        std::unique_ptr<StageProgram> p(new StageProgram(ctx));
-        StageProgram& P = *p;
+    // The stage's products and outputs.
+    void describe(StageProgram& P) const {
         enum { kFirst, kSecond, kThird };
         // from amplitudes and integrals
         const int fme = P.product(kFirst, VABIJSA, "efmn", T1, "fn", "me");
@@ -351,13 +357,16 @@ struct aq_rhfccsd {
         P.add(0.5, z26);                          // :305
         P.add(-0.5, z27);                         // :306
         P.add(-1.0, z28);                         // :307
+    }
+
+    void finish_program(std::unique_ptr<StageProgram> p) {
         // its tiles stay allocated, unlike the operand copies that the general path
         // keeps: they get half of what the budget leaves beside the DIIS history
         const double n2 = double(o) * o * v * v, history = 16.0 * std::max(cfg.diis_order, 1) * (n2 + double(o) * v);
         const double room = 0.5 * (double(ctx->budget) - double(ctx->tensor_bytes + ctx->pool_bytes) - history);
         program_refused = true;
         try {
-            if (room <= 0.0 || !P.finish(size_t(room))) return;
+            if (room <= 0.0 || !p->finish(size_t(room))) return;
         } catch (const Error& e) {
             if (e.code != AQ_ERR_OOM) throw;
             return;
