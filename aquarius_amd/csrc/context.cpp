@@ -2,7 +2,6 @@
 // Replaces the role of Aquarius's Arena (src/util/distributed.hpp:28-74): the
 // place every tensor of one job lives.  One context = one HIP stream; nothing
 // here is global, so contexts on one device are independent.
-#include "blocks.hpp"
 #include "internal.hpp"
 
 #include <atomic>
@@ -27,66 +26,55 @@ size_t ctx_in_use(const aq_ctx* ctx) { return ctx->tensor_bytes + ctx->pool_byte
 // pool releases its free memory to the driver once that exceeds what is in use
 // (36 to 46 ms per release here, twice in a burst of eight small jobs), and
 // every job's end frees nearly all it had.  Safe across the slots' streams: a
-// block carries an event recorded behind its last use, and a request from
-// another stream waits for it.  Bounded by the server's budget (BlockLedger):
+// block goes to other slots only when its job has ended and its stream is
+// synchronised (before that to the same stream, in order), so no slot ever waits
+// for another's events.  Such waits do not go together with graphs: an event of
+// a stream that another thread captures by now cannot be waited for, and a host
+// wait for it ends that capture.  Bounded by the server's budget (BlockLedger):
 // what does not fit beside the running jobs' reservations goes to the device
 // pool, oldest first.
 struct BlockCache {
     int device = 0;
     std::mutex mu;
     BlockLedger led;
-    std::vector<hipEvent_t> spare;
 
-    void* take(size_t n, hipStream_t stream) {
+    void* take(size_t n) {
         std::lock_guard<std::mutex> lk(mu);
-        BlockLedger::Block b;
-        if (!led.take(n, b)) return nullptr;
-        const hipEvent_t freed = static_cast<hipEvent_t>(b.freed);
-        if (b.stream != stream && hipStreamWaitEvent(stream, freed, 0) != hipSuccess) {
-            (void)hipGetLastError();
-            (void)hipEventSynchronize(freed);   // a wait that cannot be queued is made on the host
-        }
-        recycle(freed);
-        return b.p;
+        KeptBlock b;
+        return led.take(n, b) ? b.p : nullptr;
     }
-    void note(void* p, size_t n) noexcept {
+    void lend(void* p, size_t bytes, size_t asked) noexcept {
         std::lock_guard<std::mutex> lk(mu);
         try {
-            led.lend(p, n, n);
+            led.lend(p, bytes, asked);
         } catch (...) {   // no host memory: not tracked, and freed as any other block
         }
     }
-    // false: not kept (the caller frees it); pooled: the device pool got older blocks instead
-    bool give(void* p, hipStream_t stream, bool& pooled) noexcept {
+    BlockLedger::Lent back(void* p) {
         std::lock_guard<std::mutex> lk(mu);
-        hipEvent_t e = nullptr;
+        return led.back(p);
+    }
+    // An idle block; false: no room (the caller frees it).  pooled: the device
+    // pool got older blocks instead.
+    bool keep(const KeptBlock& b, hipStream_t stream, bool& pooled) noexcept {
+        std::lock_guard<std::mutex> lk(mu);
+        if (!led.fits(b.bytes)) return false;
         try {
-            const size_t bytes = led.back(p);
-            if (bytes == 0 || !led.fits(bytes)) return false;
-            if (!spare.empty()) {
-                e = spare.back();
-                spare.pop_back();
-            } else if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
-                (void)hipGetLastError();
-                return false;
-            }
-            if (hipEventRecord(e, stream) != hipSuccess) {
-                (void)hipGetLastError();
-                (void)hipEventDestroy(e);
-                return false;
-            }
-            led.keep({p, bytes, stream, e});
+            led.keep(b);
         } catch (...) {   // no host memory for the bookkeeping
-            if (e) (void)hipEventDestroy(e);
             return false;
         }
-        pooled = pooled || led.over();
-        while (led.over()) release_oldest(stream);
+        release_over(stream, pooled);
         return true;
     }
     void set_limit(size_t bytes) {
         std::lock_guard<std::mutex> lk(mu);
         led.limit = bytes;
+    }
+    // what may be lent beyond the requests' sizes
+    size_t spare() {
+        std::lock_guard<std::mutex> lk(mu);
+        return led.limit > led.slack() ? led.limit - led.slack() : 0;
     }
     size_t slack() {
         std::lock_guard<std::mutex> lk(mu);
@@ -99,36 +87,22 @@ struct BlockCache {
     // Kept blocks beyond the limit (all: every kept block) to the device pool.
     void release(hipStream_t stream, bool all, bool& pooled) {
         std::lock_guard<std::mutex> lk(mu);
-        while (all ? !led.empty() : led.over()) {
-            release_oldest(stream);
-            pooled = true;
-        }
+        release_over(stream, pooled);
+        while (all && !led.empty()) release_oldest(stream, pooled);
     }
     ~BlockCache() {
         bool pooled = false;
         release(nullptr, true, pooled);
         (void)hipStreamSynchronize(nullptr);
-        for (auto e : spare) (void)hipEventDestroy(e);
     }
 
   private:
-    void recycle(hipEvent_t e) noexcept {            // mu held
-        try {
-            spare.push_back(e);
-        } catch (...) {
-            (void)hipEventDestroy(e);
-        }
+    void release_oldest(hipStream_t stream, bool& pooled) noexcept {   // mu held
+        (void)hipFreeAsync(led.pop_oldest().p, stream);
+        pooled = true;
     }
-    void release_oldest(hipStream_t stream) noexcept {   // mu held
-        const BlockLedger::Block b = led.pop_oldest();
-        const hipEvent_t freed = static_cast<hipEvent_t>(b.freed);
-        // a wait that cannot be queued is made on the host
-        if (b.stream != stream && hipStreamWaitEvent(stream, freed, 0) != hipSuccess) {
-            (void)hipGetLastError();
-            (void)hipEventSynchronize(freed);
-        }
-        (void)hipFreeAsync(b.p, stream);
-        recycle(freed);
+    void release_over(hipStream_t stream, bool& pooled) noexcept {
+        while (led.over()) release_oldest(stream, pooled);
     }
 };
 
@@ -174,6 +148,7 @@ size_t block_cache_slack(BlockCache* c) { return c->slack(); }
 // the queue aborts without it).
 void block_cache_settle(aq_ctx* ctx) {
     constexpr size_t kDeviceReserve = size_t(4) << 30;
+    ctx->drained = false;
     ctx->blocks->release(ctx->stream, false, ctx->pooled);
     size_t free_b = 0, total_b = 0;
     if (hipMemGetInfo(&free_b, &total_b) == hipSuccess && free_b < kDeviceReserve) {
@@ -196,27 +171,60 @@ void block_cache_trim(aq_ctx* ctx) {
 // Stream-ordered device memory: allocations and frees are ordered on the
 // context's stream, so one context releasing memory never synchronises the
 // device under other contexts (concurrent serving).
+static void pool_free(aq_ctx* ctx, void* p) {
+    (void)hipFreeAsync(p, ctx->stream);
+    ctx->pooled = true;
+}
+
 void* dmalloc(aq_ctx* ctx, size_t bytes) {
-    if (ctx->blocks)
-        if (void* p = ctx->blocks->take(bytes, ctx->stream)) return p;
+    if (ctx->blocks) {
+        KeptBlock b;
+        if (ctx->own.take(bytes, ctx->blocks->spare(), b)) {
+            ctx->blocks->lend(b.p, b.bytes, bytes);
+            ctx->blocks->release(ctx->stream, false, ctx->pooled);
+            return b.p;
+        }
+        if (void* p = ctx->blocks->take(bytes)) return p;
+        // within the reservation also with what the job has freed
+        while (!ctx->own.blocks.empty() && ctx_in_use(ctx) + bytes + ctx->own.bytes > ctx->budget)
+            pool_free(ctx, ctx->own.pop_oldest().p);
+    }
     void* p = nullptr;
     if (hipMallocAsync(&p, bytes, ctx->stream) != hipSuccess) {
         (void)hipGetLastError();
         return nullptr;
     }
-    if (ctx->blocks) ctx->blocks->note(p, bytes);
+    if (ctx->blocks) ctx->blocks->lend(p, bytes, bytes);
     return p;
 }
 
 void dfree(aq_ctx* ctx, void* p) {
-    if (p) {
-        if (!ctx->blocks) {
-            (void)hipFreeAsync(p, ctx->stream);
-        } else if (!ctx->blocks->give(p, ctx->stream, ctx->pooled)) {
-            (void)hipFreeAsync(p, ctx->stream);
-            ctx->pooled = true;
+    if (!p) return;
+    ctx->mem_gen += 1;
+    if (!ctx->blocks) {
+        (void)hipFreeAsync(p, ctx->stream);
+        return;
+    }
+    const BlockLedger::Lent l = ctx->blocks->back(p);
+    if (l.bytes && ctx->drained) {
+        if (ctx->blocks->keep({p, l.bytes}, ctx->stream, ctx->pooled)) return;
+    } else if (l.bytes && ctx_in_use(ctx) - l.asked + ctx->own.bytes + l.bytes <= ctx->budget) {
+        try {
+            ctx->own.keep({p, l.bytes});
+            return;
+        } catch (const std::bad_alloc&) {
         }
-        ctx->mem_gen += 1;
+    }
+    pool_free(ctx, p);
+}
+
+// A job has ended and its stream is synchronised: what it frees from here on, and
+// has freed, is idle.
+void block_cache_drained(aq_ctx* ctx) {
+    ctx->drained = true;
+    while (!ctx->own.blocks.empty()) {
+        const KeptBlock b = ctx->own.pop_oldest();
+        if (!ctx->blocks->keep(b, ctx->stream, ctx->pooled)) pool_free(ctx, b.p);
     }
 }
 
@@ -293,12 +301,14 @@ static void* raw_alloc(aq_ctx* ctx, size_t bytes) {
         // operand copy.
         const auto t0 = std::chrono::steady_clock::now();
         pool_release_all(ctx);
+        while (!ctx->own.blocks.empty()) pool_free(ctx, ctx->own.pop_oldest().p);
         release_kept_blocks(ctx);
         AQ_HIP(hipStreamSynchronize(ctx->stream));
         trim_device_pool(ctx->device);
         p = dmalloc(ctx, bytes);
         if (!p) {
             evict_cache(ctx, ctx->budget);   // drop every cached copy
+            while (!ctx->own.blocks.empty()) pool_free(ctx, ctx->own.pop_oldest().p);
             release_kept_blocks(ctx);
             AQ_HIP(hipStreamSynchronize(ctx->stream));
             trim_device_pool(ctx->device);

@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "../../include/aqamd.h"
+#include "blocks.hpp"
 
 namespace aqamd {
 
@@ -143,7 +144,9 @@ struct aq_ctx {
 
     // freed blocks shared with a server's other slots (null: the device pool's)
     aqamd::BlockCache* blocks = nullptr;
-    bool pooled = false;            // some went to the device pool since it was trimmed
+    aqamd::SlotBlocks own;          // freed by the running job
+    bool drained = true;            // no job runs here, the stream is synchronised
+    bool pooled = false;            // some blocks went to the device pool since it was trimmed
 
     // reductions
     double* d_partials = nullptr;   // device: kRedSlots slots x kRedPartials partials
@@ -193,6 +196,7 @@ void block_cache_limit(BlockCache* c, size_t bytes);
 size_t block_cache_slack(BlockCache* c);
 size_t kept_bytes(int device);                       // what all servers on the device keep
 void block_cache_settle(aq_ctx* ctx);                // a job starts on this slot: back within the limit
+void block_cache_drained(aq_ctx* ctx);               // it has ended, its stream is synchronised
 void block_cache_trim(aq_ctx* ctx);                  // its memory is freed: what was not kept goes to the driver
 void invalidate_cache(aq_ctx* ctx);                  // every cached copy must be rebuilt before use
 void noalloc_scratch_init(int device);               // noalloc.cpp: resolve the fixed device array once per device

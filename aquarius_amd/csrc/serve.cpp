@@ -106,13 +106,14 @@ struct aq_server {
         aq_rhfccsd* cc = nullptr;
         aq_tensor* mo = nullptr;
         auto cleanup = [&]() {
+            // the job's memory goes to the server's block cache, for the next job;
+            // what the budget does not leave room for goes back to the driver
+            (void)hipStreamSynchronize(ctx->stream);
+            block_cache_drained(ctx);
             if (cc) aq_rhfccsd_destroy(cc);
             if (mo) aq_tensor_destroy(mo);
             for (auto* t : ints)
                 if (t) aq_tensor_destroy(t);
-            // the job's memory goes to the server's block cache, for the next job;
-            // what the budget does not leave room for goes back to the driver
-            (void)hipStreamSynchronize(ctx->stream);
             drop_caches(ctx);
             block_cache_trim(ctx);
         };
