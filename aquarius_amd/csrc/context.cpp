@@ -346,8 +346,10 @@ void dev_free(aq_ctx* ctx, void* p, size_t bytes) {
     ctx->pool_free[round_up(bytes)].push_back(p);
 }
 
+size_t alloc_bytes(size_t bytes) { return std::max<size_t>(round_up(bytes), 256); }
+
 double* tensor_alloc(aq_ctx* ctx, size_t bytes) {
-    bytes = std::max<size_t>(round_up(bytes), 256);
+    bytes = alloc_bytes(bytes);
     void* p = raw_alloc(ctx, bytes);
     ctx->tensor_bytes += bytes;
     note_peak(ctx);
@@ -355,7 +357,7 @@ double* tensor_alloc(aq_ctx* ctx, size_t bytes) {
 }
 
 void tensor_free(aq_ctx* ctx, double* p, size_t bytes) {
-    bytes = std::max<size_t>(round_up(bytes), 256);
+    bytes = alloc_bytes(bytes);
     dfree(ctx, p);
     ctx->tensor_bytes -= bytes;
 }

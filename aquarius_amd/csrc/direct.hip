@@ -869,7 +869,11 @@ void plan_stage_level(DirectArgs* const* a, int n) {
                 const double fed = (f.tm() + f.tn()) * 128.0 * f.wk * per_wave / kChip * 256.0;
                 const double sums = s > 1 ? f.tm() * f.tn() * 16.0 / kSplitBytes * 256.0 : 0.0;
                 const double alone = per_wave * std::max(kStageLatency, busy) + kStart + kStageSplit * s;
-                opts[size_t(i)].push_back({c, s, alone, tiles * s * (std::max(cu, fed) + sums) / 256.0});
+                const double share = tiles * s * (std::max(cu, fed) + sums) / 256.0;
+                // not an option that is never the better one
+                bool worse = false;
+                for (const auto& x : opts[size_t(i)]) worse = worse || (x.alone <= alone && x.share <= share);
+                if (!worse) opts[size_t(i)].push_back({c, s, alone, share});
                 lo = std::min(lo, alone);
                 hi = std::max(hi, alone);
             }

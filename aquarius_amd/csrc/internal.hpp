@@ -184,10 +184,13 @@ void* dev_alloc(aq_ctx* ctx, size_t bytes);        // pooled scratch
 void dev_free(aq_ctx* ctx, void* p, size_t bytes);   // back to the pool
 double* tensor_alloc(aq_ctx* ctx, size_t bytes);     // persistent (counted against budget)
 void tensor_free(aq_ctx* ctx, double* p, size_t bytes);
+size_t alloc_bytes(size_t bytes);                    // what a tensor of `bytes` is charged
 size_t ctx_in_use(const aq_ctx* ctx);
 void evict_cache(aq_ctx* ctx, size_t need);
 void drop_caches(aq_ctx* ctx);                       // operand copies and pooled scratch back to the allocator
 void trim_device_pool(int device);                   // the device pool's unused memory back to the driver
+// bytes of a closed-shell solver's batched stage (rhfccsd.cpp); 0 where it has none
+size_t batched_stage_bytes(int o, int v, int precision, bool packed_ladder);
 // a server's freed blocks, kept for its next jobs (at most `bytes` of them, with
 // what reused blocks are larger than asked for); its contexts are destroyed before it
 BlockCache* block_cache_create(int device);

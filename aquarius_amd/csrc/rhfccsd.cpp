@@ -133,6 +133,7 @@ struct aq_rhfccsd {
     // <ab|ef> = <ba|fe> and <ab|ij> = <ba|ji> (so Tau(ef,ij) = Tau(fe,ji)).
     void derive_packed() {
         program.reset();   // holds addresses of the packed operators
+        program_refused = false;
         program_flops = -1.0;
         packed = false;
         if (cfg.packed_ladder && o >= 2 && v >= 2) {
@@ -213,6 +214,7 @@ struct aq_rhfccsd {
 
         derive_packed();
         note_input_versions();
+        set_program_room();
         diis.reset(new DIIS(ctx, cfg.diis_order, cfg.diis_start, cfg.diis_damping, 2, 2));   // :98
     }
 
@@ -230,13 +232,28 @@ struct aq_rhfccsd {
     // both: kBatchedMixed (a burst of eight jobs, o = 4 to 14: 105 ms so, 135 with
     // the larger limit).
     static constexpr double kBatchedDoubles = 3.5e6, kBatchedMixed = 1.2e6;
+    static bool batched_size(int o, int v, int precision) {
+        return double(o) * o * v * v <= (precision == AQ_PREC_FP64 ? kBatchedDoubles : kBatchedMixed);
+    }
     std::unique_ptr<StageProgram> program;
     bool program_refused = false;
+    size_t program_room = 0;   // bytes that its buffers may take
     double program_flops = -1.0;   // of its largest product (-1: not known yet)
 
+    // Its buffers stay allocated, unlike the operand copies that the general path
+    // keeps.  They may take what the budget leaves beside the tensors that exist
+    // when the solver does and its whole DIIS history, so that the choice of path
+    // (which decides the order of sums) depends on sizes and the budget alone, not
+    // on scratch that happens to be pooled or on the iteration.
+    void set_program_room() {
+        const size_t n1 = size_t(o) * v;
+        const size_t history = 2 * size_t(std::max(cfg.diis_order, 1)) * (alloc_bytes(8 * n1 * n1) + alloc_bytes(8 * n1));
+        const size_t taken = ctx->tensor_bytes + history;
+        program_room = ctx->budget > taken ? ctx->budget - taken : 0;
+    }
+
     bool batched(int prec) {
-        const double most = cfg.precision == AQ_PREC_FP64 ? kBatchedDoubles : kBatchedMixed;
-        if (double(o) * o * v * v > most || program_refused) return false;
+        if (!batched_size(o, v, cfg.precision) || program_refused) return false;
         // a phase of reduced arithmetic that cannot use it allocates nothing for it
         if (prec != AQ_PREC_FP64 && program_flops >= cfg.min_reduced_flops) return false;
         if (!program) {
@@ -245,13 +262,25 @@ struct aq_rhfccsd {
             describe(*p);
             program_flops = p->largest_flops();
             if (prec != AQ_PREC_FP64 && program_flops >= cfg.min_reduced_flops) return false;
-            finish_program(std::move(p));
+            program_refused = true;
+            try {
+                if (!p->finish(program_room)) return false;
+            } catch (const Error& e) {
+                if (e.code != AQ_ERR_OOM) throw;
+                return false;
+            } catch (const tensor::TensorError& e) {
+                if (e.code != AQ_ERR_OOM) throw;
+                return false;
+            }
+            program = std::move(p);
+            program_refused = false;
         }
-        return program != nullptr;
+        return true;
     }
 
-    // The stage's products and outputs.
-    void describe(StageProgram& P) const {
+    // The stage's products and outputs, for a StageProgram or for the sizes alone.
+    template <class Program>
+    void describe(Program& P) const {
         enum { kFirst, kSecond, kThird };
         // from amplitudes and integrals
         const int fme = P.product(kFirst, VABIJSA, "efmn", T1, "fn", "me");
@@ -275,8 +304,9 @@ struct aq_rhfccsd {
         const int z12 = P.product(kFirst, VAIJBSA, "amie", T1, "em", "ai");
         const int z13 = P.product(kFirst, VABCI, "efam", TauSA, "efim", "ai");
         const int z21 = P.product(kFirst, VABCI, "abej", T1, "ei", "abij");
-        const int sp = packed ? P.product(kFirst, Vp, "pq", Tp, "iq", "pi") : -1;
-        const int sm = packed ? P.product(kFirst, Vm, "pq", Tm, "iq", "pi") : -1;
+        // pairs: p, q (virtual) and x (occupied) symmetric, r, s and y antisymmetric
+        const int sp = packed ? P.product(kFirst, Vp, "pq", Tp, "xq", "px") : -1;
+        const int sm = packed ? P.product(kFirst, Vm, "rs", Tm, "ys", "ry") : -1;
         const int lad = packed ? -1 : P.product(kFirst, VABCD, "abef", Tau, "efij", "abij");
         P.output(kFirst, FME, "me");
         P.add(1.0, fAI, "em");                    // :244
@@ -357,22 +387,6 @@ struct aq_rhfccsd {
         P.add(0.5, z26);                          // :305
         P.add(-0.5, z27);                         // :306
         P.add(-1.0, z28);                         // :307
-    }
-
-    void finish_program(std::unique_ptr<StageProgram> p) {
-        // its tiles stay allocated, unlike the operand copies that the general path
-        // keeps: they get half of what the budget leaves beside the DIIS history
-        const double n2 = double(o) * o * v * v, history = 16.0 * std::max(cfg.diis_order, 1) * (n2 + double(o) * v);
-        const double room = 0.5 * (double(ctx->budget) - double(ctx->tensor_bytes + ctx->pool_bytes) - history);
-        program_refused = true;
-        try {
-            if (room <= 0.0 || !p->finish(size_t(room))) return;
-        } catch (const Error& e) {
-            if (e.code != AQ_ERR_OOM) throw;
-            return;
-        }
-        program = std::move(p);
-        program_refused = false;
     }
 
     void batched_contractions() {
@@ -676,6 +690,23 @@ struct aq_rhfccsd {
         WAMEI["amei"] -= WMNEJ["nmei"] * T1["an"];                 // :186
     }
 };
+
+size_t aqamd::batched_stage_bytes(int o, int v, int precision, bool packed_ladder) {
+    if (!aq_rhfccsd::batched_size(o, v, precision)) return 0;
+    aq_rhfccsd shape;   // sizes only
+    shape.o = o;
+    shape.v = v;
+    shape.packed = packed_ladder && o >= 2 && v >= 2;
+    StageSizes sizes(o, v);
+    shape.describe(sizes);
+    const size_t bytes = sizes.bytes();
+    if (!shape.packed) return bytes;
+    // integrals without the pair symmetry take the unpacked ladder
+    shape.packed = false;
+    StageSizes unpacked(o, v);
+    shape.describe(unpacked);
+    return std::max(bytes, unpacked.bytes());
+}
 
 extern "C" {
 

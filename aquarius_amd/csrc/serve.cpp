@@ -53,6 +53,7 @@ inline std::vector<std::vector<int64_t>> input_shapes(int64_t o, int64_t v) {
 using namespace aqamd;
 
 size_t job_bytes(int o, int v, int nQ, int diis_order, int precision, bool integrals);
+size_t job_reservation(int o, int v, int nQ, const aq_rhfccsd_config& cfg, bool integrals, size_t budget);
 
 struct aq_server {
     int device = 0;
@@ -254,6 +255,43 @@ size_t job_bytes(int o, int v, int nQ, int diis_order, int precision, bool integ
     return size_t(8.0 * std::max(solve, build) * 1.10) + (size_t(64) << 20);
 }
 
+// What a job reserves: its bytes and, where that is more, its tensors beside the
+// buffers of the batched stage (more occupied than virtual orbitals; otherwise the
+// room for operand copies, which that path does not use, is larger), so that a
+// served solve takes the path that it takes alone.  A server too small for
+// that still runs the job, without the batched stage.
+size_t job_reservation(int o, int v, int nQ, const aq_rhfccsd_config& cfg, bool integrals, size_t budget) {
+    const size_t need = job_bytes(o, v, nQ, cfg.diis_order, cfg.precision, integrals);
+    const size_t stage = batched_stage_bytes(o, v, cfg.precision, cfg.packed_ladder != 0);
+    if (stage == 0) return need;
+    const int64_t O = o, V = v, k = std::max(cfg.diis_order, 1);
+    const int64_t N2 = O * O * V * V, P = V * (V + 1) / 2, Q = V * (V - 1) / 2, Op = O * (O + 1) / 2, Om = O * (O - 1) / 2;
+    size_t with = stage;
+    auto tensors = [&](int64_t count, int64_t doubles) { with += size_t(count) * alloc_bytes(size_t(doubles) * 8); };
+    if (integrals) {
+        tensors(1, V * V * V * V);
+        tensors(1, V * V * V * O);
+        tensors(3, N2);
+        tensors(1, O * O * O * V);
+        tensors(1, O * O * O * O);
+        tensors(1, V * O);
+        tensors(1, V * V);
+        tensors(1, O * O);
+    }
+    tensors(9, N2);             // T2, Z2, Tau, T2SA, TauSA, VABIJSA, VAIJBSA, WAMEI, WAMIE
+    tensors(2, O * O * O * V);
+    tensors(1, O * O * O * O);
+    tensors(3, V * O);
+    tensors(1, V * V);
+    tensors(1, O * O);
+    tensors(1, V);
+    tensors(1, O);
+    for (int64_t pairs : {P * P, Q * Q, P * Op, P * Op, Q * Om, Q * Om}) tensors(1, pairs);
+    tensors(2 * k, N2);         // DIIS
+    tensors(2 * k, V * O);
+    return with <= budget ? std::max(need, with) : need;
+}
+
 extern "C" {
 
 int aq_server_create(int device, size_t hbm_budget, int slots, double max_bypass_s, aq_server** out) {
@@ -313,7 +351,7 @@ int aq_server_submit(aq_server* s, const aq_job_spec* spec, int64_t* job_id) {
                          "job input tensor " + std::to_string(k) + " has the wrong shape");
             AQ_CHECK(js.o > 0 && js.v > 0, AQ_ERR_INVALID, "job needs o > 0 and v > 0");
             // the integrals are borrowed: reserve the solver's own memory only
-            need = job_bytes(js.o, js.v, 0, js.cfg.diis_order, js.cfg.precision, /*integrals=*/false);
+            need = job_reservation(js.o, js.v, 0, js.cfg, /*integrals=*/false, s->budget);
             // their writes must be complete before another stream reads them
             for (auto* t : inputs) AQ_HIP(hipStreamSynchronize(t->ctx->stream));
         } else if (spec->fcidump) {
@@ -324,10 +362,10 @@ int aq_server_submit(aq_server* s, const aq_job_spec* spec, int64_t* job_id) {
                      "FCIDUMP job needs a closed shell (MS2 = 0, even NELEC < 2 NORB)");
             js.o = nelec / 2;
             js.v = norb - js.o;
-            need = job_bytes(js.o, js.v, -norb, js.cfg.diis_order, js.cfg.precision, true);
+            need = job_reservation(js.o, js.v, -norb, js.cfg, true, s->budget);
         } else {
             AQ_CHECK(spec->o > 0 && spec->v > 0, AQ_ERR_INVALID, "job needs o > 0 and v > 0");
-            need = aq_job_bytes_estimate(spec->o, spec->v, spec->nQ, spec->cfg.diis_order, spec->cfg.precision);
+            need = job_reservation(spec->o, spec->v, spec->nQ, spec->cfg, true, s->budget);
         }
         std::lock_guard<std::mutex> lk(s->mu);
         AQ_CHECK(!s->stopping, AQ_ERR_INVALID, "server is stopping");

@@ -41,6 +41,53 @@ static uint32_t log2_of(uint32_t x) {
     return l;
 }
 
+// doubles of the tiles of a planned product
+static int64_t tile_doubles(const DirectArgs& a) { return int64_t(a.tilesM) * a.tilesN * a.nsplit * a.tm * a.tn; }
+
+double StageSizes::len(char c) const {
+    switch (c) {
+        case 'p': case 'q': return v_ * (v_ + 1) / 2;
+        case 'r': case 's': return v_ * (v_ - 1) / 2;
+        case 'x': return o_ * (o_ + 1) / 2;
+        case 'y': return o_ * (o_ - 1) / 2;
+        default: return c < 'i' ? v_ : o_;
+    }
+}
+
+int StageSizes::product(int level, const tensor::Tensor&, const char* ia, const tensor::Tensor&, const char* ib,
+                        const char* ic) {
+    // as plan_product: the rows hold the first output label
+    const std::string a(ia), b(ib);
+    const std::string &X = b.find(ic[0]) != std::string::npos ? b : a, &Y = &X == &a ? b : a;
+    double M = 1.0, N = 1.0, K = 1.0;
+    for (char c : X) (Y.find(c) != std::string::npos ? K : M) *= len(c);
+    for (char c : Y)
+        if (X.find(c) == std::string::npos) N *= len(c);
+    ok_ = ok_ && std::max({M * K, N * K, M * N}) < double(1 << 28);
+    if (int(levels_.size()) <= level) levels_.resize(size_t(level) + 1);
+    DirectArgs p{};
+    p.batch = 1;
+    if (ok_) {
+        p.M = uint32_t(M);
+        p.N = uint32_t(N);
+        p.K = uint32_t(K);
+    }
+    levels_[size_t(level)].push_back(p);
+    return count_++;
+}
+
+size_t StageSizes::bytes() {
+    if (!ok_) return 0;
+    int64_t total = 0;
+    for (auto& l : levels_) {
+        std::vector<DirectArgs*> a;
+        for (auto& p : l) a.push_back(&p);
+        plan_stage_level(a.data(), int(a.size()));
+        for (const auto& p : l) total += tile_doubles(p);
+    }
+    return alloc_bytes(size_t(total) * 8) + kDescBytes;
+}
+
 bool StageProgram::finish(size_t room) {
     if (!ok_) return false;   // a contraction not of the batched stage's form
     int nlevels = 0;
@@ -58,9 +105,9 @@ bool StageProgram::finish(size_t room) {
     }
     for (auto& p : products_) {
         at.push_back(total);
-        total += int64_t(p.a.tilesM) * p.a.tilesN * p.a.nsplit * p.a.tm * p.a.tn;
+        total += tile_doubles(p.a);
     }
-    if (size_t(total) * 8 + kDescBytes > room) return false;
+    if (alloc_bytes(size_t(total) * 8) + kDescBytes > room) return false;
     tiles_ = tensor::Tensor(ctx_, std::vector<int64_t>{std::max<int64_t>(total, 1)}, false);
     for (size_t k = 0; k < products_.size(); ++k) products_[k].a.P = tiles_.handle()->data + at[k];
 

@@ -35,7 +35,6 @@ class StageProgram {
     // not of the stage's form or its buffers take more than `room` bytes
     bool finish(size_t room);
     void run();           // every launch on the context's stream
-    const std::vector<const tensor::Tensor*>& outputs() const { return written_; }
 
   private:
     struct Product {
@@ -73,6 +72,26 @@ class StageProgram {
     std::vector<Level> levels_;
     std::vector<const tensor::Tensor*> written_;
     tensor::Tensor tiles_, desc_;
+};
+
+// What a program's buffers take, from the labels alone: a-h virtual, i-o occupied,
+// p, q / r, s symmetric / antisymmetric virtual pairs, x / y occupied ones.
+class StageSizes {
+  public:
+    StageSizes(int o, int v) : o_(o), v_(v) {}
+    int product(int level, const tensor::Tensor&, const char* ia, const tensor::Tensor&, const char* ib, const char* ic);
+    void output(int, const tensor::Tensor&, const char*, bool = false) {}
+    void add(double, const tensor::Tensor&, const char*) {}
+    void add(double, int) {}
+    void add_pairs(double, int, bool) {}
+    size_t bytes();       // 0: not of the stage's form
+
+  private:
+    double len(char c) const;
+    double o_, v_;
+    bool ok_ = true;
+    std::vector<std::vector<DirectArgs>> levels_;
+    int count_ = 0;
 };
 
 }  // namespace aqamd

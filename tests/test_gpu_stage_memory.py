@@ -1,5 +1,9 @@
-"""Memory of the batched contraction stage: a reduced phase that cannot use its
-buffers holds none."""
+"""Memory of the batched contraction stage: a solve takes the same path (and so
+gives the same bits) whether it is served, under a budget that holds its buffers,
+or alone, whatever scratch is pooled; and a reduced phase that cannot use its
+buffers holds none.
+
+Which path ran is read from the timing classes of the kernels."""
 
 import pytest
 
@@ -29,6 +33,54 @@ def footprint(o, v, order, **over):
         cc.close()
         ints.free()
     return held, stage - min(stage, slot), energies
+
+
+def classes(ctx):
+    return {k.split("_")[0] + "_" + k.split("_")[1] for k in ctx.timing()}
+
+
+@pytest.mark.parametrize("o,v", [(13, 75), (18, 90), (30, 30)])
+def test_served_takes_the_path_it_takes_alone(o, v):
+    print(f"case: served o={o} v={v}", flush=True)
+    cfg = lambda: aq.default_config(diis_order=8, max_iterations=6, convergence=0.0)
+    with aq.Context() as ctx:
+        ints = aq.Integrals.synthetic(ctx, 3, o, v)
+        ctx.sync()
+        cc = aq.RHFCCSD(ctx, ints, config=cfg())
+        alone = cc.run()
+        cc.close()
+        with aq.Server(slots=2, hbm_budget=24 << 30) as s:
+            for jobs in ({"inputs": ints}, {}):     # the caller's integrals, and the job's own
+                r = s.wait(s.submit(3, o, v, config=cfg(), **jobs))
+                assert r["status"] == aq.JOB_DONE, r["error"]
+                # conv is one element of a residual: a sum in another order shows
+                assert (r["energy"], r["conv"]) == (alone["energy"], alone["conv"])
+        ints.free()
+
+
+@pytest.mark.parametrize("pooled", [False, True])
+def test_pooled_scratch_does_not_change_the_path(pooled):
+    o, v, order = 8, 40, 4
+    print(f"case: pooled scratch {pooled}", flush=True)
+    held, stage, want = footprint(o, v, order)
+    assert stage > 0
+    with aq.Context(hbm_budget=held + history(o, v, order) + 3 * stage // 2) as ctx:
+        ints = aq.Integrals.synthetic(ctx, 3, o, v)
+        cc = aq.RHFCCSD(ctx, ints, diis_order=order)
+        ctx.trim()
+        if pooled:   # an aliased sum's snapshot stays in the pool
+            x = ctx.tensor((stage // 4 // 24, 3))
+            ctx.sum(1.0, x, "ab", 1.0, x, "ab")
+            y = ctx.tensor((max(int((stage // 4 // 8) ** 0.5), 2),) * 2)
+            ctx.sum(1.0, y, "aa", 0.5, y, "ab")
+            x.free()
+            y.free()
+        ctx.enable_timing(True)
+        got = [cc.iterate()[0] for _ in range(3)]
+        assert "stage_contract" in classes(ctx)
+        assert got == want
+        cc.close()
+        ints.free()
 
 
 def test_reduced_phase_holds_no_buffers():
