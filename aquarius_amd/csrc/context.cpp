@@ -289,6 +289,7 @@ static void* raw_alloc(aq_ctx* ctx, size_t bytes) {
     if (ctx_in_use(ctx) + bytes > ctx->budget) {
         pool_release_all(ctx);
         evict_cache(ctx, bytes);
+        while (ctx_in_use(ctx) + bytes > ctx->budget && !ctx->reclaimable.empty()) ctx->reclaimable.front()->reclaim();
     }
     AQ_CHECK(ctx_in_use(ctx) + bytes <= ctx->budget, AQ_ERR_OOM,
              "HBM budget exceeded: need " + std::to_string(bytes) + " B, in use " +
@@ -308,6 +309,7 @@ static void* raw_alloc(aq_ctx* ctx, size_t bytes) {
         p = dmalloc(ctx, bytes);
         if (!p) {
             evict_cache(ctx, ctx->budget);   // drop every cached copy
+            while (!ctx->reclaimable.empty()) ctx->reclaimable.front()->reclaim();
             while (!ctx->own.blocks.empty()) pool_free(ctx, ctx->own.pop_oldest().p);
             release_kept_blocks(ctx);
             AQ_HIP(hipStreamSynchronize(ctx->stream));

@@ -120,6 +120,16 @@ struct aq_tensor {
 namespace aqamd {
 struct GemmBatcher;
 struct BlockCache;
+
+// Holds memory of its context that it can do without: given up when an
+// allocation does not fit the budget otherwise.  May be called inside any
+// allocation of the context, so nothing it frees is in use by the caller.
+struct Reclaimable {
+    virtual void reclaim() = 0;   // also leaves the context's list
+
+  protected:
+    ~Reclaimable() = default;
+};
 }
 
 struct aq_ctx {
@@ -147,6 +157,8 @@ struct aq_ctx {
     aqamd::SlotBlocks own;          // freed by the running job
     bool drained = true;            // no job runs here, the stream is synchronised
     bool pooled = false;            // some blocks went to the device pool since it was trimmed
+
+    std::vector<aqamd::Reclaimable*> reclaimable;   // oldest first
 
     // reductions
     double* d_partials = nullptr;   // device: kRedSlots slots x kRedPartials partials

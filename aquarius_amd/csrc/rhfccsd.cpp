@@ -32,7 +32,7 @@ using aqamd::tensor::scalar;
 
 using namespace aqamd;
 
-struct aq_rhfccsd {
+struct aq_rhfccsd final : aqamd::Reclaimable {
     aq_ctx* ctx = nullptr;
     aq_rhfccsd_config cfg{};
     int o = 0, v = 0;
@@ -132,7 +132,7 @@ struct aq_rhfccsd {
     // The ladder can run on the (anti)symmetric packed forms when
     // <ab|ef> = <ba|fe> and <ab|ij> = <ba|ji> (so Tau(ef,ij) = Tau(fe,ji)).
     void derive_packed() {
-        program.reset();   // holds addresses of the packed operators
+        reclaim();         // the program holds addresses of the packed operators
         program_refused = false;
         program_flops = -1.0;
         packed = false;
@@ -244,12 +244,20 @@ struct aq_rhfccsd {
     // keeps.  They may take what the budget leaves beside the tensors that exist
     // when the solver does and its whole DIIS history, so that the choice of path
     // (which decides the order of sums) depends on sizes and the budget alone, not
-    // on scratch that happens to be pooled or on the iteration.
+    // on scratch that happens to be pooled or on the iteration.  They are given up
+    // when something else in the context needs the memory (reclaim).
     void set_program_room() {
         const size_t n1 = size_t(o) * v;
         const size_t history = 2 * size_t(std::max(cfg.diis_order, 1)) * (alloc_bytes(8 * n1 * n1) + alloc_bytes(8 * n1));
         const size_t taken = ctx->tensor_bytes + history;
         program_room = ctx->budget > taken ? ctx->budget - taken : 0;
+    }
+
+    void reclaim() override {
+        program.reset();
+        if (!ctx) return;
+        auto& r = ctx->reclaimable;
+        r.erase(std::remove(r.begin(), r.end(), this), r.end());
     }
 
     bool batched(int prec) {
@@ -272,6 +280,7 @@ struct aq_rhfccsd {
                 if (e.code != AQ_ERR_OOM) throw;
                 return false;
             }
+            ctx->reclaimable.push_back(this);
             program = std::move(p);
             program_refused = false;
         }
@@ -579,7 +588,10 @@ struct aq_rhfccsd {
         graph.warm_prec = prec;
     }
 
-    ~aq_rhfccsd() { drop_graph(); }
+    ~aq_rhfccsd() {
+        drop_graph();
+        reclaim();
+    }
 
     // rhfccsd.cxx:194-327
     void iterate() {

@@ -1,10 +1,11 @@
 """Memory of the batched contraction stage: a solve takes the same path (and so
 gives the same bits) whether it is served, under a budget that holds its buffers,
-or alone, whatever scratch is pooled; and a reduced phase that cannot use its
-buffers holds none.
+or alone, whatever scratch is pooled; its buffers give way to what else the
+context has to hold; and a reduced phase that cannot use them holds none.
 
 Which path ran is read from the timing classes of the kernels."""
 
+import numpy as np
 import pytest
 
 import aquarius_amd as aq
@@ -79,6 +80,36 @@ def test_pooled_scratch_does_not_change_the_path(pooled):
         got = [cc.iterate()[0] for _ in range(3)]
         assert "stage_contract" in classes(ctx)
         assert got == want
+        cc.close()
+        ints.free()
+
+
+def test_buffers_give_way():
+    """A tensor that fits beside the solver, but not beside the stage's buffers too: it is
+    allocated, and the solve goes on along the general path."""
+    o, v, order = 30, 30, 4
+    print("case: buffers give way", flush=True)
+    held, stage, _ = footprint(o, v, order)
+    with aq.Context() as ctx:
+        ints = aq.Integrals.synthetic(ctx, 3, o, v)
+        cc = aq.RHFCCSD(ctx, ints, diis_order=order)
+        want = [cc.iterate()[0] for _ in range(6)]
+        cc.close()
+        ints.free()
+    with aq.Context(hbm_budget=held + history(o, v, order) + 4 * stage) as ctx:
+        ints = aq.Integrals.synthetic(ctx, 3, o, v)
+        cc = aq.RHFCCSD(ctx, ints, diis_order=order)
+        ctx.enable_timing(True)
+        got = [cc.iterate()[0] for _ in range(2)]
+        assert "stage_contract" in classes(ctx)
+        extra = ctx.tensor((int(3.6 * stage) // 8,), zero=False)
+        ctx.timing_reset()
+        got += [cc.iterate()[0] for _ in range(2)]
+        assert "stage_contract" not in classes(ctx)
+        cc.hbar(with_wabej=True)
+        extra.free()
+        got += [cc.iterate()[0] for _ in range(2)]
+        np.testing.assert_allclose(got, want, rtol=1e-9, atol=0)
         cc.close()
         ints.free()
 
