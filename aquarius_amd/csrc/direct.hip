@@ -925,7 +925,7 @@ bool direct_contract(aq_ctx* ctx, DirectArgs a) {
     a.kchunk = (chunks + p.nsplit - 1) / p.nsplit * 16;
     a.nsplit = (a.K + a.kchunk - 1) / a.kchunk;
     const uint64_t tiles = uint64_t(a.tilesM) * a.tilesN * a.batch;
-    if (tiles * a.nsplit >= (uint64_t(1) << 31)) return false;
+    if (tiles * a.nsplit >= kDirBlocks) return false;
     Scratch part(ctx, a.nsplit > 1 ? size_t(tiles) * a.nsplit * f.tm() * f.tn() * 8 : 0);
     for (DirDigits* d : {&a.m, &a.n, &a.k}) set_dividers(*d);
     a.P = part.as<double>();
@@ -936,6 +936,7 @@ bool direct_contract(aq_ctx* ctx, DirectArgs a) {
     // a server's slots merge same-kernel problems of different jobs; the thin
     // ones launch alone, as thin GEMMs do
     const bool grouped = ctx->batcher && !ctx->capture && a.M > 16 && a.N > 16 &&
+                         tiles * a.nsplit < kDirBlocks / kDirGroup &&
                          batcher_offer_direct(ctx, config, a, int64_t(tiles) * a.nsplit);
     if (!grouped) {
         TimedLaunch tl(ctx, name, 2.0 * mn * a.K,

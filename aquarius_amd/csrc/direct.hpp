@@ -34,10 +34,14 @@ struct DirectArgs {
     uint32_t config, tm, tn;  // batched stages: kernel (tile shape * 4 + layout bits) and tile
 };
 
+// Blocks of a launch: fewer than 2^32 threads, 256 a block.
+constexpr uint64_t kDirBlocks = uint64_t(1) << 24;
+constexpr int kDirGroup = 8;   // problems per grouped launch
+
 // Runs the problem if the direct kernels take its sizes; false: not taken.
 bool direct_contract(aq_ctx* ctx, DirectArgs a);
-// a group of same-kernel problems in one launch (grouping across contexts)
-constexpr int kDirGroup = 8;   // problems per launch
+// a group of same-kernel problems in one launch (grouping across contexts), each
+// of fewer than kDirBlocks / kDirGroup blocks
 void launch_direct_group(int config, const DirectArgs* const* p, int n, hipStream_t s);
 
 // ---- batched stages: the contractions of a solver's small iteration, level by

@@ -185,6 +185,7 @@ bool StageProgram::finish(size_t room) {
             }
         }
         AQ_CHECK(args.size() <= 64 && outs.size() <= 64, AQ_ERR_INVALID, "stage level size");
+        if (L.s.blocks >= kDirBlocks / kDirGroup || L.blocks >= kDirBlocks) return false;
         L.nout = int(outs.size());
         Offsets& f = offs[size_t(l)];
         f.prob = place(args.data(), args.size() * sizeof(DirectArgs));
