@@ -524,33 +524,24 @@ __global__ __launch_bounds__(256, F == 2 ? 3 : 2) void k_staged_grouped(DirectGr
     staged_tile<F, KA, KB>(G.p[p], xcd_order(blockIdx.x - G.first[p], G.first[p + 1] - G.first[p]), lds);
 }
 
-// constants of the time model (pick_shape), clock cycles
-constexpr double kL1 = 286.0, kLatency = 1033.0, kStart = 2337.0, kBlock = 258.0, kChip = 5534.0;
-constexpr double kLaunch = 1.5, kSplit = 2.6, kSplitBytes = 3509.0, kPerSplit = 0.06, kGHz = 2400.0;
-constexpr double kStagedBusy = 1.05, kStagedWait = 925.0;
-
 struct DirCfg {
     int fm, fn, wm, wn, wk, stages;   // stages 0: staged through LDS
+    int resident;                     // blocks of 256 threads a CU holds (registers)
     int tm() const { return 16 * fm * wm; }
     int tn() const { return 16 * fn * wn; }
-    // cycles of a CU per chunk of a block (of each wave)
-    double busy() const {
-        if (!stages) return fm * fn * 256.0 * kStagedBusy;
-        return std::max(fm * fn * 256.0, (fm + fn) * kL1);
-    }
 };
 constexpr DirCfg kDirCfg[] = {
-    {1, 1, 1, 1, 4, 4},   // 16 x 16: tiny outputs
-    {2, 2, 1, 1, 4, 3},   // 32 x 32, waves share k
-    {1, 1, 2, 2, 1, 4},   // 32 x 32, short k
-    {2, 2, 2, 2, 1, 0},   // 64 x 64, staged through LDS
-    {4, 1, 1, 1, 4, 3},   // 64 x 16
-    {1, 4, 1, 1, 4, 3},   // 16 x 64
-    {4, 1, 4, 1, 1, 2},   // 256 x 16, short k
-    {1, 4, 1, 4, 1, 2},   // 16 x 256, short k
-    {4, 4, 2, 2, 1, 0},   // 128 x 128, staged
-    {2, 2, 2, 2, 1, 3},   // 64 x 64, from registers: a block alone on its CU
-    {4, 2, 4, 1, 1, 2},   // 256 x 32, short k: 607500 x 27 x 150 streams 991 MB in 204 us, 4.9 TB/s
+    {1, 1, 1, 1, 4, 4, 4},   // 16 x 16: tiny outputs
+    {2, 2, 1, 1, 4, 3, 2},   // 32 x 32, waves share k
+    {1, 1, 2, 2, 1, 4, 4},   // 32 x 32, short k
+    {2, 2, 2, 2, 1, 0, 3},   // 64 x 64, staged through LDS
+    {4, 1, 1, 1, 4, 3, 2},   // 64 x 16
+    {1, 4, 1, 1, 4, 3, 2},   // 16 x 64
+    {4, 1, 4, 1, 1, 2, 2},   // 256 x 16, short k
+    {1, 4, 1, 4, 1, 2, 2},   // 16 x 256, short k
+    {4, 4, 2, 2, 1, 0, 2},   // 128 x 128, staged
+    {2, 2, 2, 2, 1, 3, 2},   // 64 x 64, from registers: a block alone on its CU
+    {4, 2, 4, 1, 1, 2, 2},   // 256 x 32, short k: 607500 x 27 x 150 streams 991 MB in 204 us, 4.9 TB/s
 };
 constexpr int kNDirCfg = int(sizeof(kDirCfg) / sizeof(kDirCfg[0]));
 
@@ -638,14 +629,23 @@ static bool k_layout(const DirCfg& f, const DirDigits& k, const uint32_t* st) {
 }
 
 // Tile shape and split of one problem: the least modelled time over the
-// shapes and power-of-two splits.  Model (clock cycles; the constants are a
-// least-regret fit to 39 contractions of the CCSD iteration at five sizes, o =
-// 5 to 20, v = 19 to 140, timed in every shape and split; its choices are
-// within 2% of the best choice on average): a chunk of 16 k costs a wave its
-// MFMAs (64 each) or the L1 accesses of its fragments, and a single wave at
-// least the load latency over the chunks in flight; blocks queue on 256 CUs;
-// operand tiles come in at a rate of the whole chip; a split pays a second
-// launch and the traffic of the partial tiles.
+// shapes and power-of-two splits.  Model (clock cycles): a chunk of 16 k costs a
+// wave its MFMAs (64 each) or the L1 accesses of its fragments (more where k is
+// the contiguous index), and a single wave at least the load latency over the
+// chunks in flight; blocks queue on 256 CUs, as many at a time as registers let
+// a CU hold; waves that share k are added at the end; operand tiles come in at a
+// rate of the whole chip; a split pays a second launch and the traffic of the
+// partial tiles.  The constants are a least-regret fit to 515 contractions (the
+// forms of the CCSD iteration at o = 4 to 28, v = 17 to 165, and plain products up
+// to 1e9 FLOP), each timed in every shape and split; over these and 190 more (long
+// inner extents, batches, short products with long sides) the chosen one is 2.2%
+// slower than the best on average, 9% at the 90th percentile.  (A model without
+// residency and the waves' sum, fitted to 39 contractions, was 3.7% and 15% off:
+// 1110^3 in 32 x 32 tiles 102 us, now 64 x 64 in two splits 78; 201600 x 14 x 120 in
+// 64 x 16 tiles 52 us, now 256 x 16 43.)
+constexpr double kL1Rows = 320.0, kL1K = 369.0, kLatency = 934.0, kStart = 3460.0, kReduce = 905.0, kChip = 4508.0;
+constexpr double kLaunch = 1.5, kSplit = 2.955, kSplitBytes = 5148.0, kPerSplit = 0.06, kCyclesPerUs = 2400.0;
+constexpr double kStagedWait = 676.0;
 
 struct Pick {
     int cfg = -1;
@@ -656,19 +656,29 @@ struct Pick {
 static Pick pick_shape(const DirectArgs& a) {
     Pick best;
     const double chunks = std::ceil(a.K / 16.0);
+    auto contiguous = [](const DirDigits& d, const uint32_t* st) { return d.nd > 0 && st[0] == 1; };
+    const double l1A = !contiguous(a.m, a.m.s0) && contiguous(a.k, a.k.s0) ? kL1K : kL1Rows;
+    const double l1B = !contiguous(a.n, a.n.s0) && contiguous(a.k, a.k.s1) ? kL1K : kL1Rows;
     for (int c = 0; c < kNDirCfg; ++c) {
         const DirCfg& f = kDirCfg[c];
+        // at most a quarter of such a tile is the product (batches of tiny ones)
+        if (uint32_t(f.tm()) >= 2 * ((a.M + 15) / 16 * 16) && uint32_t(f.tn()) >= 2 * ((a.N + 15) / 16 * 16)) continue;
         const double tiles = double((a.M + f.tm() - 1) / f.tm()) * double((a.N + f.tn() - 1) / f.tn()) * a.batch;
+        // cycles of a CU per chunk of a block (of each wave); 128 x 128 spills 5 to
+        // 9 registers in three of its four layouts
+        const double mfma = f.fm * f.fn * 256.0;
+        const double busy = f.stages ? std::max(mfma, f.fm * l1A + f.fn * l1B) : mfma * (f.fm == 4 ? 1.27 : 1.064);
+        const double wait = f.stages ? std::max(kLatency / (f.stages - 1), busy) : busy + kStagedWait;
+        const double ends = f.wk > 1 ? kReduce : 0.0;
         for (uint32_t s = 1; s <= 128; s *= 2) {
             if (s > 1 && (chunks / s < f.wk || tiles * s > 16384)) break;
-            const double blocks = tiles * s;
+            const double blocks = tiles * s, cu = std::ceil(blocks / 256.0);
             const double per_wave = std::ceil(std::ceil(chunks / s) / f.wk);
-            const double busy = f.busy();
-            const double alone = per_wave * (f.stages ? std::max(kLatency / (f.stages - 1), busy) : busy + kStagedWait) + kStart;
-            const double queued = std::ceil(blocks / 256.0) * (per_wave * busy + kBlock);
+            const double alone = per_wave * wait + kStart + ends;
+            const double queued = std::max(cu * (per_wave * busy + ends), std::ceil(cu / f.resident) * alone);
             const double fed = (f.tm() + f.tn()) * 128.0 * f.wk * per_wave * blocks / kChip;
-            double t = kLaunch + std::max({alone, queued, fed}) / kGHz;
-            if (s > 1) t += kSplit + tiles * f.tm() * f.tn() * 8.0 * (2 * s + 1) / kSplitBytes / kGHz + s * kPerSplit;
+            double t = kLaunch + std::max({alone, queued, fed}) / kCyclesPerUs;
+            if (s > 1) t += kSplit + tiles * f.tm() * f.tn() * 8.0 * (2 * s + 1) / kSplitBytes / kCyclesPerUs + s * kPerSplit;
             if (t < best.us) best = {c, s, t};
         }
     }
@@ -852,6 +862,7 @@ void plan_stage_level(DirectArgs* const* a, int n) {
         double alone, share;
     };
     constexpr double kStageBlock = 1000.0;     // CU cycles of a block's start and end
+    constexpr double kStageStart = 2337.0, kStageL1 = 286.0, kStageChip = 5534.0, kStageSplitBytes = 3509.0;
     constexpr double kStageLatency = 2000.0;   // a chunk of a block alone, whatever its tile
     constexpr double kStageSplit = 60.0;       // the assembly's cycles per partial tile
     std::vector<std::vector<Option>> opts(static_cast<size_t>(n));
@@ -864,11 +875,12 @@ void plan_stage_level(DirectArgs* const* a, int n) {
             for (uint32_t s = 1; s <= 128; s *= 2) {
                 if (s > 1 && (chunks / s < f.wk || tiles * s > 16384)) break;
                 const double per_wave = std::ceil(std::ceil(chunks / s) / f.wk);
-                const double busy = f.busy();
+                const double mfma = f.fm * f.fn * 256.0;
+                const double busy = f.stages ? std::max(mfma, (f.fm + f.fn) * kStageL1) : mfma * 1.05;
                 const double cu = per_wave * busy + kStageBlock;
-                const double fed = (f.tm() + f.tn()) * 128.0 * f.wk * per_wave / kChip * 256.0;
-                const double sums = s > 1 ? f.tm() * f.tn() * 16.0 / kSplitBytes * 256.0 : 0.0;
-                const double alone = per_wave * std::max(kStageLatency, busy) + kStart + kStageSplit * s;
+                const double fed = (f.tm() + f.tn()) * 128.0 * f.wk * per_wave / kStageChip * 256.0;
+                const double sums = s > 1 ? f.tm() * f.tn() * 16.0 / kStageSplitBytes * 256.0 : 0.0;
+                const double alone = per_wave * std::max(kStageLatency, busy) + kStageStart + kStageSplit * s;
                 const double share = tiles * s * (std::max(cu, fed) + sums) / 256.0;
                 // not an option that is never the better one
                 bool worse = false;

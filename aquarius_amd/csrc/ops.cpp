@@ -388,37 +388,57 @@ static bool digits_of(const std::string& order, const Labeled& X, const Labeled&
 }
 
 // Whether the direct kernels (direct.hip) serve a contraction better than the
-// GEMM kernels on permuted operands.  Measured per contraction of the CCSD
-// iteration, amplitude operands permuted anew and integrals cached on the GEMM
-// side (time GEMM side / direct, us):
+// GEMM kernels on permuted operands.  Measured per contraction (time GEMM side /
+// direct, us), the second operand permuted anew and the first one's copy cached
+// on the GEMM side:
 //  - up to 6e8 FLOP nearly everything gains: o=5, v=19 490/203, o=8, v=43
-//    699/274, o=11, v=60 860/440 over the 39 contractions.  Exceptions: rows
+//    699/274, o=11, v=60 860/440 over the 39 contractions of the CCSD iteration;
+//    plain products 200^3 16/5, 400^3 25/10, 666^3 29/21.  Exceptions: rows
 //    contiguous in one operand but not in C (scattered stores), e.g. 39600 x
-//    11 x 60 11.0/14.7, from 2e5 outputs on; and a matrix-vector product along
-//    a large operand's contiguous index (12100 x 1 x 1540 31/48);
+//    11 x 60 11.0/14.7, from 2e5 outputs on; a matrix-vector product along
+//    a large operand's contiguous index (12100 x 1 x 1540 31/48); a batch index that
+//    is the contiguous one of an operand (300 x 3 x 300, 200 times 41/154; 64^3, 500
+//    times 35/55; gone below 64 outputs each: 4^3, 60000 times 226/122) and batches
+//    of short sums (107 x 4 x 3, 9500 times 42/128);
+//  - operands that are matrices as they lie, which the GEMM need not permute: at
+//    most 16 columns from 2e5 outputs on (79507 x 6 x 43 9.3/11.2, 328509 x 14 x 69
+//    39/47), and above 5.5e5 outputs short sums (16000 x 64 x 64 9.9/13.2, 29587 x 66
+//    x 39 16/20; both sides long 3000 x 3000 x 33 45/35, 12000 x 12000 x 2 286/323) and
+//    operands both contiguous along k (4096 x 256 x 256 18.7/21.7).  Otherwise they
+//    gain too (2000 x 300 x 300 22/19, 16000 x 40 x 160 14.7/12.3);
 //  - small outputs with a long inner extent (a split GEMM with a serial sum of
 //    partials): 110 x 110 x 21560 50/32, 140 x 20 x 392000 244/160;
 //  - a short side and a short inner extent against a long side: 140 x 56000 x
-//    140 111/81;
+//    140 111/81 (matrices below 2e9 FLOP the other way: 117 x 26325 x 117 27/32);
 //  - at most 32 columns and a short inner extent against a very long side, rows
 //    contiguous in A and C: the GEMM's narrowest wide tile, 128 x 64, multiplies
 //    up to twice the columns, 256 x 32 from registers does not (392000 x 20 x 140
-//    171/132, 607500 x 27 x 150 322/250, 1179648 x 32 x 192 699/556);
-//  - large products whose GEMM would have to permute: 975^3 72/64, 1600^3
-//    226/203, 2800^3 950/840 (both operands strided, amplitudes permuted anew);
-//    beyond, permuting costs less than the LDS tiles lose to the GEMM's (3080^3
-//    1240/1280).  Operands that are matrices as they lie stay with the GEMM
-//    (10000 x 256 x 256 39/57), and so do two that are both contiguous along k,
-//    which one cached copy or none serves (2800 x 400 x 19600 1030/1510).
-static bool direct_size(const DirectArgs& a, bool scattered, bool rows_x, bool rows_y, int64_t sizeX) {
+//    171/132, 607500 x 27 x 150 322/250, 1179648 x 32 x 192 699/556).  Up to 16
+//    columns the GEMM wastes none: 201600 x 14 x 120 39/43 with the cached copy
+//    (121/43 where the long operand is new);
+//  - large products whose GEMM would have to permute: 1110^3 77/78 (84/78 with
+//    both operands new), 1600^3 189/171, 2800^3 831/729; beyond, permuting costs
+//    less than the LDS tiles lose to the GEMM's (3080^3 1240/1280).
+//    Two operands that are both contiguous along k stay with the GEMM, which one
+//    cached copy or none serves (2800 x 400 x 19600 1030/1510).
+static bool direct_size(const DirectArgs& a, bool scattered, bool rows_x, bool rows_y, int64_t sizeX, bool batch_first) {
     const double out = double(a.M) * a.N * a.batch, flops = 2.0 * out * a.K;
     if (scattered && out > 2e5) return false;
     if (a.N == 1 && !rows_x && sizeX > 8000000) return false;
+    const bool matrices = a.m.nd <= 1 && a.n.nd <= 1 && a.k.nd <= 1;   // nothing to permute
+    if (a.batch < 65536) {   // as many as the GEMM takes
+        if (batch_first && double(a.M) * a.N > 64) return false;
+        if (a.batch > 1 && a.K <= 16 && double(a.M) * a.N > 256) return false;
+        if (matrices && a.batch == 1 && a.N <= 16 && out > 2e5) return false;
+        const double side = std::min(a.M, a.N);
+        if (matrices && a.batch == 1 && side > 32 && out > 5.5e5 && (side < 1500 || out > 2e7) &&
+            (a.K <= 64 || (!rows_x && !rows_y)))
+            return false;
+    }
     if (flops <= 6e8) return true;
     if (out <= 2.5e4) return flops <= 2e10;
     if (a.N <= 32 && a.K <= 512 && rows_x && !scattered && double(a.M) >= 1000.0 * a.N) return flops <= 1e11;
-    if (a.M <= 200 && a.K <= 200 && double(a.N) >= 50.0 * a.M) return flops <= 2e10;
-    const bool matrices = a.m.nd <= 1 && a.n.nd <= 1 && a.k.nd <= 1;   // nothing to permute
+    if (a.M <= 200 && a.K <= 200 && double(a.N) >= 50.0 * a.M) return flops <= 2e10 && (!matrices || flops >= 2e9);
     return !matrices && (rows_x || rows_y) && a.M > 200 && a.N > 200 && a.K > 200 &&
            flops <= 5e10;
 }
@@ -455,7 +475,8 @@ static bool run_direct(aq_ctx* ctx, double alpha, const Labeled& A, const Labele
     a.N = uint32_t(swap ? M : N);
     a.K = uint32_t(K);
     a.batch = uint32_t(NB);
-    if (!direct_size(a, rows_x && has(Rl, uc) && ux != uc, rows_x, rows_y, X.size())) return false;
+    const bool batch_first = !bl.empty() && (bl[0] == ux || bl[0] == uy);
+    if (!direct_size(a, rows_x && has(Rl, uc) && ux != uc, rows_x, rows_y, X.size(), batch_first)) return false;
     a.A = X.data;
     a.B = Y.data;
     a.C = Cdata;
