@@ -84,7 +84,7 @@ int aq_ctx_get_precision(const aq_ctx* ctx, int* precision);
 int aq_ctx_set_gemm_variant(aq_ctx* ctx, int precision, int variant);
 /* GEMM autotuning (no reference counterpart).  With enable != 0 the first
  * GEMM of every shape bucket (arithmetic, operand layouts, and M, N, K and
- * batch in half-octaves) times each kernel variant once on this context's
+ * batch in half-octaves) times each kernel variant once (BF16x3: 0 to 3) on this context's
  * stream, into a scratch output, and the fastest serves that bucket from then
  * on for every context on the device.  Variants compute identical results
  * (the split-K partition does not depend on them), so tuning changes speed
