@@ -87,8 +87,13 @@ class DIIS {
         }
         // the newest slots (:92-120): the residuals are stored by the launch
         // that forms their products, x by the extrapolation (or `keep`)
-        reserve(old_x_[0], x);
-        reserve(old_dx_[0], dx);
+        try {
+            reserve(old_x_[0], x);
+            reserve(old_dx_[0], dx);
+        } catch (...) {   // the caller's results are there all the same
+            if (hipStreamSynchronize(ctx_->stream) == hipSuccess) synced();
+            throw;
+        }
 
         // e[i][0] = <dx, old_dx[i]> for every stored slot (:122-135)
         int nreal = 1;
@@ -204,7 +209,9 @@ class DIIS {
 
     void reserve(std::vector<Tensor>& slot, const std::vector<Tensor*>& src) {
         if (!slot.empty()) return;
-        for (auto* t : src) slot.emplace_back(ctx_, t->lengths(), false);
+        std::vector<Tensor> s;   // all of them or, when one does not fit, none
+        for (auto* t : src) s.emplace_back(ctx_, t->lengths(), false);
+        slot = std::move(s);
     }
     // x into its newest history slot
     void keep(const std::vector<Tensor*>& x) {
