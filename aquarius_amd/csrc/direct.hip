@@ -310,15 +310,19 @@ __device__ __forceinline__ void direct_tile(const DirectArgs& g, uint32_t bid, c
 // is what the register path lacks on long contractions: its fragments need 20
 // L1 accesses for a 64-lane load when k and rows are both strided in memory, a
 // chunk then costs 2300 cycles of the CU instead of the 1024 of its MFMAs
-// (three 975^3 side by side: 174 us, 130 so; 2800^3: 950 us, 840 with 128 x
-// 128, which also needs half the LDS and L2 traffic of 64 x 64).  A chunk is
-// loaded into registers while the one before it is multiplied; LDS holds it as
-// [k][row] or [row][k], padded so that the 32 lanes of a half-wave read 32
-// different bank pairs.  What is left is the matrix cores' own rate: they are
-// busy 75% of the time and waits for data are 7%; neither a deeper prefetch (2
-// or 3 chunks) nor the stores to LDS between the products changes that, and
-// random values run 9% slower than constants (a power limit on short kernels:
-// the same loop reaches 72 TFLOP/s over 15 ms, 59 over 2 ms).
+// (64 x 64 from registers and so: 1110^3 in two splits 110 and 80 us, 1600^3 191 and
+// 178; 2800^3 943, 837, and 744
+// with 128 x 128, which also needs half the LDS and L2 traffic of 64 x 64).  A
+// chunk is loaded into registers while the one before it is multiplied; LDS holds
+// it as [k][row] or [row][k], padded so that the 32 lanes of a half-wave read 32
+// different bank pairs.  What bounds it: the matrix cores are busy 73% of a CU's
+// busy cycles at 64 x 64 and 82% at 128 x 128 (2800^3), waves wait for data 17% and
+// 11% of their time and for the matrix cores to take an instruction most of the
+// rest.  A deeper prefetch (2 or 3 chunks) and stores to LDS between the products
+// change nothing.  128 x 128 has no registers left: 256, and 5 to 9 spilled in
+// three of its four layouts; what that costs is not known.  Random values run up to
+// 9% slower than constants (a power limit on short kernels: the same loop reaches
+// 72 TFLOP/s over 15 ms, 59 over 2 ms).
 template <int F>
 struct Staged {
     static constexpr int T = 32 * F, PR = T + 16, PK = 18;             // tile side, pitches
@@ -655,30 +659,33 @@ struct Pick {
 
 static Pick pick_shape(const DirectArgs& a) {
     Pick best;
-    const double chunks = std::ceil(a.K / 16.0);
+    const uint32_t chunks = (a.K + 15) / 16;
+    const uint32_t padM = (a.M + 15) / 16 * 16, padN = (a.N + 15) / 16 * 16;
     auto contiguous = [](const DirDigits& d, const uint32_t* st) { return d.nd > 0 && st[0] == 1; };
     const double l1A = !contiguous(a.m, a.m.s0) && contiguous(a.k, a.k.s0) ? kL1K : kL1Rows;
     const double l1B = !contiguous(a.n, a.n.s0) && contiguous(a.k, a.k.s1) ? kL1K : kL1Rows;
     for (int c = 0; c < kNDirCfg; ++c) {
         const DirCfg& f = kDirCfg[c];
+        const uint32_t tm = uint32_t(f.tm()), tn = uint32_t(f.tn()), wk = uint32_t(f.wk);
         // at most a quarter of such a tile is the product (batches of tiny ones)
-        if (uint32_t(f.tm()) >= 2 * ((a.M + 15) / 16 * 16) && uint32_t(f.tn()) >= 2 * ((a.N + 15) / 16 * 16)) continue;
-        const double tiles = double((a.M + f.tm() - 1) / f.tm()) * double((a.N + f.tn() - 1) / f.tn()) * a.batch;
+        if (tm >= 2 * padM && tn >= 2 * padN) continue;
+        const uint64_t tiles = uint64_t((a.M + tm - 1) / tm) * ((a.N + tn - 1) / tn) * a.batch;
         // cycles of a CU per chunk of a block (of each wave); 128 x 128 spills 5 to
         // 9 registers in three of its four layouts
         const double mfma = f.fm * f.fn * 256.0;
         const double busy = f.stages ? std::max(mfma, f.fm * l1A + f.fn * l1B) : mfma * (f.fm == 4 ? 1.27 : 1.064);
         const double wait = f.stages ? std::max(kLatency / (f.stages - 1), busy) : busy + kStagedWait;
-        const double ends = f.wk > 1 ? kReduce : 0.0;
-        for (uint32_t s = 1; s <= 128; s *= 2) {
-            if (s > 1 && (chunks / s < f.wk || tiles * s > 16384)) break;
-            const double blocks = tiles * s, cu = std::ceil(blocks / 256.0);
-            const double per_wave = std::ceil(std::ceil(chunks / s) / f.wk);
+        const double ends = f.wk > 1 ? kReduce : 0.0, feed = (tm + tn) * 128.0 * f.wk / kChip;
+        const double partials = double(tiles) * tm * tn * 8.0 / kSplitBytes / kCyclesPerUs;
+        for (uint32_t l = 0, s = 1; l < 8; ++l, s *= 2) {
+            const uint64_t blocks = tiles << l;
+            if (s > 1 && (chunks < wk * s || blocks > 16384)) break;
+            const uint64_t cu = (blocks + 255) / 256, rounds = (cu + uint32_t(f.resident) - 1) / uint32_t(f.resident);
+            const double per_wave = ((chunks + s - 1) / s + wk - 1) / wk;
             const double alone = per_wave * wait + kStart + ends;
-            const double queued = std::max(cu * (per_wave * busy + ends), std::ceil(cu / f.resident) * alone);
-            const double fed = (f.tm() + f.tn()) * 128.0 * f.wk * per_wave * blocks / kChip;
-            double t = kLaunch + std::max({alone, queued, fed}) / kCyclesPerUs;
-            if (s > 1) t += kSplit + tiles * f.tm() * f.tn() * 8.0 * (2 * s + 1) / kSplitBytes / kCyclesPerUs + s * kPerSplit;
+            const double queued = std::max(double(cu) * (per_wave * busy + ends), double(rounds) * alone);
+            double t = kLaunch + std::max({alone, queued, feed * per_wave * double(blocks)}) / kCyclesPerUs;
+            if (s > 1) t += kSplit + partials * (2 * s + 1) + s * kPerSplit;
             if (t < best.us) best = {c, s, t};
         }
     }
@@ -714,7 +721,9 @@ __device__ __forceinline__ void stage_tile(const DirectArgs& g, uint32_t bid, ch
 
 // Fewer chunks in flight than the single kernels, for three waves per SIMD: the
 // blocks of a level are short and mostly wait (o = 8, v = 43: 37 us a launch
-// with 4/3/3 chunks and two waves, 29 us with 3/2/2 and three).
+// with 4/3/3 chunks and two waves, 29 us with 3/2/2 and three).  The 64 x 64 tile
+// takes all of the 168 registers that three waves leave, and 8 are spilled; the
+// other shapes need fewer (o = 13, v = 75: 171 us a level, matrix cores busy 60%).
 __global__ __launch_bounds__(256, 3) void k_stage(StageGroup G) {
     __shared__ __attribute__((aligned(16))) char lds[Staged<2>::kLds];   // the largest of the shapes
     int j = 0;

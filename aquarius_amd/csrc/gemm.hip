@@ -1358,7 +1358,8 @@ void gemm(aq_ctx* ctx, const GemmDesc& d) {
         // same ragged-round rule over the grid of 256 x 256 tiles and W2 = 256
         // (the packed ladder: 815 and 810 tiles = 3.2 rounds, split 5 ways
         // fill 16 rounds instead of 4 rounds of whole tiles), with the partials
-        // capped at 2 GiB so that the operand cache keeps its copies.
+        // (floats; the test counts 8 bytes) capped at 1 GiB so that the operand
+        // cache keeps its copies.
         const int64_t W2 = 256, T2 = ((d.M + 255) / 256) * ((d.N + 255) / 256) * d.batch;
         if (T2 > W2 && T2 <= 8 * W2) {
             const double r1 = double((T2 + W2 - 1) / W2);

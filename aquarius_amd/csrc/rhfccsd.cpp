@@ -222,8 +222,8 @@ struct aq_rhfccsd final : aqamd::Reclaimable {
     // the same products as contractions(), those that depend on nothing but
     // amplitudes and integrals side by side, then those that need the first
     // intermediates, and so on; two products that several intermediates share
-    // ("efam,fi" and "nmei,an") are formed once.  A stage is 10 launches instead
-    // of 57.  Used while every product is FP64 arithmetic and the doubles have at
+    // ("efam,fi" and "nmei,an") are formed once.  A stage is 8 launches (7 where
+    // the ladder is not packed) instead of 57.  Used while every product is FP64 arithmetic and the doubles have at
     // most kBatchedDoubles elements: an FP64 iteration takes (general / batched, us)
     // 1461/1130 at o = 14, v = 85, 2393/2110 at o = 16, v = 100, 4438/4255 at o =
     // 10, v = 180, and 9161/9308 at o = 20, v = 140, where the general path has the
