@@ -66,13 +66,19 @@ def test_server_returns_what_earlier_contexts_freed(before):
 
 
 def test_trim_of_another_context_takes_back_what_a_server_keeps(before):
+    """At least the largest four-virtual block is kept after the jobs; a context created
+    then counts it as free in its default budget (nine tenths), and trim gives it back."""
     print("case: trim beside an idle server", flush=True)
+    largest = 8 * max(v for _, v in SIZES) ** 4
     with aq.Context() as ctx, aq.Server(slots=2, hbm_budget=24 << 30) as s:
         serve(s, SIZES)
         s.drain()
-        assert before - free() > 2 * OVERHEAD    # kept for the next jobs
-        with aq.Context() as other:              # its default budget: nine tenths of what it can get
-            assert other.memory()[1] >= 0.9 * (before - OVERHEAD)
+        kept = free()
+        with aq.Context() as other:
+            budget = other.memory()[1]
         ctx.trim()
-        assert before - free() <= OVERHEAD
+        trimmed = free()
+        assert trimmed - kept >= largest
+        assert budget >= 0.9 * (trimmed - OVERHEAD)
+        assert before - trimmed <= OVERHEAD
         serve(s, SIZES[:3])                      # and the server goes on
