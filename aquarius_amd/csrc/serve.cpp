@@ -256,9 +256,9 @@ size_t job_bytes(int o, int v, int nQ, int diis_order, int precision, bool integ
 }
 
 // What a job reserves: its bytes and, where that is more, its tensors beside the
-// buffers of the batched stage (more occupied than virtual orbitals; otherwise the
-// room for operand copies, which that path does not use, is larger), so that a
-// served solve takes the path that it takes alone.  A server too small for
+// buffers of the batched stage, so that a served solve takes the path that it takes
+// alone.  That is where o comes near v (18 / 29, 30 / 30); otherwise the room for
+// operand copies, which that path does not use, is larger.  A server too small for
 // that still runs the job, without the batched stage.
 size_t job_reservation(int o, int v, int nQ, const aq_rhfccsd_config& cfg, bool integrals, size_t budget) {
     const size_t need = job_bytes(o, v, nQ, cfg.diis_order, cfg.precision, integrals);
